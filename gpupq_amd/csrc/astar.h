@@ -24,6 +24,32 @@ __device__ __forceinline__ int nbr_dx(uint32_t k) { return k < 4 ? (k == 0 ? 1 :
 __device__ __forceinline__ int nbr_dy(uint32_t k) { return k < 4 ? (k == 2 ? 1 : (k == 3 ? -1 : 0)) : ((k & 2) ? -1 : 1); }
 __device__ __forceinline__ uint32_t nbr_cost(uint32_t conn, uint32_t k) { return conn == 4 ? 1u : (k < 4 ? 10u : 14u); }
 
+// Bit k of the result: neighbour k of (x, y) lies in the w x h grid and is free.  Three rows of
+// three cells span at most two bitmap words each, so six loads with clamped addresses, none of
+// them dependent on another, fetch every bit an expansion needs.
+__device__ __forceinline__ uint32_t free_neighbours(const uint32_t* bits, uint32_t conn, int x, int y, int w, int h) {
+  const int x0 = x > 0 ? x - 1 : 0, x2 = x + 1 < w ? x + 1 : w - 1;
+  uint32_t lo[3], hi[3];
+  uint64_t row[3];
+#pragma unroll
+  for (int r = 0; r < 3; ++r) {
+    const int yy = y + r - 1 < 0 ? 0 : (y + r - 1 < h ? y + r - 1 : h - 1);
+    row[r] = (uint64_t)yy * (uint64_t)w;
+    lo[r] = bits[(row[r] + (uint64_t)x0) >> 5];
+    hi[r] = bits[(row[r] + (uint64_t)x2) >> 5];
+  }
+  uint32_t m = 0;
+#pragma unroll
+  for (uint32_t k = 0; k < 8; ++k) {
+    const int nx = x + nbr_dx(k), ny = y + nbr_dy(k), r = nbr_dy(k) + 1;
+    const uint64_t i = row[r] + (uint64_t)nx;
+    const uint32_t word = (i >> 5) == ((row[r] + (uint64_t)x0) >> 5) ? lo[r] : hi[r];
+    const bool in = nx >= 0 && ny >= 0 && nx < w && ny < h && k < conn;
+    if (in && !((word >> (i & 31)) & 1u)) m |= 1u << k;
+  }
+  return m;
+}
+
 struct AstarState {
   uint32_t best;                 // best goal cost found so far (0xFFFFFFFF: none)
   uint32_t done;

@@ -82,6 +82,10 @@ __device__ __forceinline__ uint32_t list_of(uint32_t cell, uint32_t lists) {
   return (uint32_t)(((uint64_t)(cell * 0x9E3779B1u) * lists) >> 32);
 }
 
+// One pop and expansion per list.  A step is bound by the latency of one list's dependent
+// accesses, not by bytes: the popped cell's g and its neighbours' obstacle bits are loaded
+// together, then all relaxations are in flight at once.  One neighbour after the other (bit,
+// then atomic) took 11.2 us per launch, this 7.4 us (4096 lists, 1001 x 703, 8-connected).
 template <class Q>
 __global__ __launch_bounds__(256) void astar_step_kernel(Q q, AstarDev a) {
   uint32_t expanded = 0, newly_closed = 0;
@@ -97,7 +101,10 @@ __global__ __launch_bounds__(256) void astar_step_kernel(Q q, AstarDev a) {
     q.set_done(idx);
     const uint32_t cell = e.seq, f = e.ts, hv = e.src;
     const uint32_t g = f - hv;
-    if (g != __hip_atomic_load(&a.g[cell], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) continue;   // stale
+    const int x = (int)(cell % a.width), y = (int)(cell / a.width);
+    const uint32_t g_now = __hip_atomic_load(&a.g[cell], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const uint32_t nbr = free_neighbours(a.blocked, a.conn, x, y, (int)a.width, (int)a.height);
+    if (g != g_now) continue;                       // stale
     if (cell == a.target) {
       atomicMin(&a.st->best, g);
       continue;
@@ -105,15 +112,21 @@ __global__ __launch_bounds__(256) void astar_step_kernel(Q q, AstarDev a) {
     if (best != 0xFFFFFFFFu && f >= best) continue;   // cannot improve on the goal found
     ++expanded;
     const uint32_t bit = 1u << (cell & 31);
-    if (!(atomicOr(&a.closed[cell >> 5], bit) & bit)) ++newly_closed;
-    const int x = (int)(cell % a.width), y = (int)(cell / a.width);
-    for (uint32_t k = 0; k < a.conn; ++k) {
-      const int nx = x + nbr_dx(k), ny = y + nbr_dy(k);
-      if (nx < 0 || ny < 0 || nx >= (int)a.width || ny >= (int)a.height) continue;
-      const uint32_t v = (uint32_t)ny * a.width + (uint32_t)nx;
-      if (bit_get(a.blocked, v)) continue;
+    const uint32_t was = atomicOr(&a.closed[cell >> 5], bit);
+    // all relaxations in flight at once, and with them the closed bit
+    uint32_t old[8];
+#pragma unroll
+    for (uint32_t k = 0; k < 8; ++k) {
+      const uint32_t v = (uint32_t)(y + nbr_dy(k)) * a.width + (uint32_t)(x + nbr_dx(k));
+      old[k] = (nbr >> k) & 1u ? atomicMin(&a.g[v], g + nbr_cost(a.conn, k)) : 0u;
+    }
+    if (!(was & bit)) ++newly_closed;
+#pragma unroll
+    for (uint32_t k = 0; k < 8; ++k) {
       const uint32_t g2 = g + nbr_cost(a.conn, k);
-      if (atomicMin(&a.g[v], g2) <= g2) continue;
+      if (!((nbr >> k) & 1u) || old[k] <= g2) continue;
+      const int nx = x + nbr_dx(k), ny = y + nbr_dy(k);
+      const uint32_t v = (uint32_t)ny * a.width + (uint32_t)nx;
       const uint32_t h2 = grid_heur(a.conn, nx, ny, (int)a.tx, (int)a.ty);
       const uint32_t list = list_of(v, a.lists);
       q.insert_or_update(Event{g2 + h2, list, h2, v}, (int)list);   // decrease-key on a LAQ in that mode

@@ -211,23 +211,33 @@ __device__ bool search_query(const BatchDev& d, Shared& sh, uint32_t* cnt, uint6
     const uint32_t best_now = *(volatile uint32_t*)&sh.best;
     if (hn && key_f(top) < best_now) {
       const uint64_t key = top;
-      top = heap_pop(hp, hn);
       const uint32_t cell = key_cell(key), f = key_f(key);
       const int x = (int)(cell % W), y = (int)(cell / W);
       const uint32_t g0 = f - grid_heur(Q.conn, x, y, (int)Q.tx, (int)Q.ty);
-      if ((tag_bits | g0) == __hip_atomic_load(&g[cell], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
+      // the cell's g and its neighbours' obstacle bits are fetched while the heap is sifted
+      const uint32_t g_now = __hip_atomic_load(&g[cell], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      const uint32_t nbr = free_neighbours(bits, Q.conn, x, y, (int)W, (int)W);
+      top = heap_pop(hp, hn);
+      if ((tag_bits | g0) == g_now) {
         ++expanded;
-        for (uint32_t k = 0; k < Q.conn; ++k) {
+        // all relaxations in flight at once: a neighbour's improvement does not depend on another's
+        uint32_t old[8];
+#pragma unroll
+        for (uint32_t k = 0; k < 8; ++k) {
+          const uint32_t v = (uint32_t)(y + nbr_dy(k)) * W + (uint32_t)(x + nbr_dx(k));
+          old[k] = ((nbr >> k) & 1u) && v != target ? atomicMin(&g[v], tag_bits | (g0 + nbr_cost(Q.conn, k))) : 0u;
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < 8; ++k) {
+          if (!((nbr >> k) & 1u)) continue;
           const int nx = x + nbr_dx(k), ny = y + nbr_dy(k);
-          if (nx < 0 || ny < 0 || nx >= (int)W || ny >= (int)W) continue;
           const uint32_t v = (uint32_t)ny * W + (uint32_t)nx;
-          if (bit_get(bits, v)) continue;
           const uint32_t g2 = g0 + nbr_cost(Q.conn, k);
           if (v == target) {
             atomicMin(&sh.best, g2);
             continue;
           }
-          if (atomicMin(&g[v], tag_bits | g2) <= (tag_bits | g2)) continue;
+          if (old[k] <= (tag_bits | g2)) continue;
           const uint32_t h2 = grid_heur(Q.conn, nx, ny, (int)Q.tx, (int)Q.ty);
           if (g2 + h2 >= *(volatile uint32_t*)&sh.best) continue;   // cannot beat the goal found
           const uint64_t k2 = make_key(g2 + h2, h2, v);
