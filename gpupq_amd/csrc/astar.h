@@ -143,6 +143,7 @@ class AstarBatch {
   gpq_status plain_one(const uint32_t* d_id, uint32_t spec_index, uint32_t slot, uint32_t* d_done, uint32_t* h_done,
                        hipStream_t s);
   uint32_t resident_slots() const { return resident; }
+  uint64_t open_list_bytes() const;     // of one slot
   const uint32_t* device_ids() const { return d_ids_all; }
 
   std::vector<gpq_query_spec> specs;

@@ -3,16 +3,25 @@
 // The reference runs one block per agent and pulls agents from an atomic counter
 // (get_new_agent, src/a_star.cu:149-164); thread 0 pops up to 8 vertices, the block expands
 // them, deduplicates, and thread 0 inserts or updates (src/a_star.cu:325-374,441-569).  Here
-// every thread of the workgroup owns one open list (a binary heap of 64-bit keys in HBM,
-// stored slot-major: entry i of list t at heap[i * K + t]) and pops its own best entry each
-// iteration, so K expansions run in parallel.  Improved neighbours are routed to the list
-// hash(cell) mod K through an LDS staging area (own list when the stage is full); g is
-// relaxed with atomicMin, so entries made stale by a cheaper path are recognised on pop.
-// The search of a query ends when the best goal cost found is <= the smallest f of all
-// lists, which makes the result the optimal cost (admissible, consistent heuristic).
+// the open list of a query is a row of buckets by f: bucket i holds the pending entries with
+// f in [i * 2^s, (i + 1) * 2^s), appended and read in order, for the kBuckets buckets from the
+// lowest pending one on; entries beyond them (or for a full bucket) wait in an unsorted far
+// store, which is scanned when its smallest f comes up.  Each iteration the workgroup's K
+// threads take the first K entries of the lowest buckets and expand them in parallel; g is
+// relaxed with atomicMin, so entries made stale by a cheaper path are recognised when taken.
+// An entry's successors have f at least its own (consistent heuristic), so no entry is ever
+// appended below the lowest bucket.  The search of a query ends when the best goal cost found is
+// <= the smallest f that may be pending, which makes the result the optimal cost.
 //
-// Key = f << 38 | h << 22 | cell: order by f, ties to the smaller h (closer to the goal).
-// Limits that follow: side <= 2048 (cell < 2^22), f < 2^26.
+// What bounds it: the latency of an iteration (two barriers and four dependent accesses: bucket
+// entry, g and obstacle bits, relaxations, append), times the longest query's iterations, which its
+// path's steps bound from below.  Expanding an entry's best successor in the same iteration (2
+// to 16 of a chain) made iterations longer by more than it saved (15 to 29 ms).  The
+// list this replaced, a binary heap per thread, moved some 3 KB per expansion in sifts over
+// scattered lines and took 19 us per iteration against 7 us here: 512 queries of side 256 to
+// 2048 in 512-thread workgroups, 42.6 -> 12.0 ms.
+//
+// Entry = f << 22 | cell.  Limits that follow: side <= 2048 (cell < 2^22), f < 2^26.
 //
 // g entries carry a generation tag so that a slot is not cleared per query: entry =
 // tag << 26 | g, where the tag of the slot's current query is smaller than every tag written
@@ -31,9 +40,17 @@ namespace gpq {
 namespace {
 
 constexpr uint32_t kMaxSide = 2048;
-constexpr uint64_t kNoKey = ~0ull;
 constexpr uint32_t kNoCost = 0xFFFFFFFFu;
 constexpr int kMaxWaves = 16;
+
+// Buckets of a query's open list: one per lane of the wave that plans an iteration.
+constexpr uint32_t kBuckets = 64;
+// f values per bucket, as a power of two: f - h(source) is even on both kinds of grid, so a bucket
+// is one f value.  Wider buckets expand more cells out of order: 512 queries of side 256 to 2048
+// took 12.0 ms at width 2, 13.2 at 4, 15.6 at 8 and 23 at 16.  Taking entries of the lowest 32,
+// 16 or 8 buckets only (fewer expansions, idler iterations) took 12.1, 16.6 and 18.7 ms.
+constexpr uint32_t kShift = 1;
+constexpr uint32_t kNoBucket = 0xFFFFFFFFu;
 
 struct BatchQuery {
   uint32_t side, conn, sx, sy, tx, ty;
@@ -53,12 +70,19 @@ struct SlotState {
   unsigned long long expanded;
 };
 
+// A query's open list between the launches of the plain drive.
+struct SlotList {
+  uint32_t cnt[kBuckets], rd[kBuckets];
+  uint32_t base, far_n, far_min, pad;
+};
+
 struct BatchDev {
   const BatchQuery* q;
   const uint32_t* bits;                 // pooled obstacle bitmaps
   uint32_t* g;                          // [slot][g_stride]
-  uint64_t* heap;                       // [slot][H][K]
-  uint32_t* hn;                         // [slot][K] list lengths (plain drive)
+  uint64_t* far;                        // [slot][far_cap]
+  uint64_t* bucket;                     // [slot][kBuckets][bucket_cap]
+  SlotList* list;                       // [slot] (plain drive)
   SlotState* slot;
   long long* cost;                      // [query]
   unsigned long long* expanded;         // [query]
@@ -69,105 +93,189 @@ struct BatchDev {
   uint32_t* counter;                    // work counter of the persistent launch
   uint32_t slot_base;                   // workgroup b of the launch uses slot slot_base + b
   uint64_t g_stride;
-  uint32_t heap_cap, stage_cap, log2k;
-  uint32_t lds_rows;                    // heap levels held in LDS: entries [0, lds_rows)
+  uint64_t far_cap;
+  uint32_t bucket_cap;
 };
 
-__device__ __forceinline__ uint64_t make_key(uint32_t f, uint32_t h, uint32_t cell) {
-  return ((uint64_t)f << 38) | ((uint64_t)h << 22) | cell;
-}
-__device__ __forceinline__ uint32_t key_f(uint64_t k) { return (uint32_t)(k >> 38); }
-__device__ __forceinline__ uint32_t key_cell(uint64_t k) { return (uint32_t)(k & 0x3FFFFFu); }
-
-__device__ __forceinline__ uint32_t owner_of(uint32_t cell, uint32_t log2k) {
-  return log2k ? (cell * 0x9E3779B1u) >> (32 - log2k) : 0u;
-}
-
-__device__ __forceinline__ uint64_t wave_min_u64(uint64_t v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    const uint64_t o = __shfl_xor(v, off, kWave);
-    v = o < v ? o : v;
-  }
-  return v;
-}
-
-// Binary heap of one thread.  Entry i lives in LDS (row i of a slot-major [T][K] array)
-// for i < T -- the levels every push and pop touches -- and in HBM (row i of the slot's
-// [H][K] array) below; HBM rows < T only hold the LDS rows between plain-drive launches.
-struct ThreadHeap {
-  uint64_t* lds;      // lds_rows + tid
-  uint64_t* hbm;      // slot heap + tid
-  uint32_t K, T;
-  __device__ __forceinline__ uint64_t get(uint32_t i) const { return i < T ? lds[i * K] : hbm[(uint64_t)i * K]; }
-  __device__ __forceinline__ void set(uint32_t i, uint64_t v) const {
-    if (i < T) lds[i * K] = v;
-    else hbm[(uint64_t)i * K] = v;
-  }
-};
-
-// Returns the new top.
-__device__ __forceinline__ uint64_t heap_push(const ThreadHeap& hp, uint32_t& hn, uint64_t key, uint64_t top) {
-  uint32_t i = hn++;
-  while (i > 0) {
-    const uint32_t p = (i - 1) >> 1;
-    const uint64_t pv = hp.get(p);
-    if (pv <= key) break;
-    hp.set(i, pv);
-    i = p;
-  }
-  hp.set(i, key);
-  return key < top ? key : top;
-}
-
-__device__ __forceinline__ uint64_t heap_pop(const ThreadHeap& hp, uint32_t& hn) {
-  --hn;
-  if (hn == 0) return kNoKey;
-  const uint64_t last = hp.get(hn);
-  uint32_t i = 0;
-  uint64_t top = last;
-  for (;;) {
-    uint32_t c = 2 * i + 1;
-    if (c >= hn) break;
-    uint64_t cv = hp.get(c);
-    if (c + 1 < hn) {
-      const uint64_t c2 = hp.get(c + 1);
-      if (c2 < cv) { cv = c2; ++c; }
-    }
-    if (last <= cv) break;
-    hp.set(i, cv);
-    if (i == 0) top = cv;
-    i = c;
-  }
-  hp.set(i, last);
-  return top;
-}
+__device__ __forceinline__ uint64_t make_entry(uint32_t f, uint32_t cell) { return ((uint64_t)f << 22) | cell; }
+__device__ __forceinline__ uint32_t entry_f(uint64_t e) { return (uint32_t)(e >> 22); }
+__device__ __forceinline__ uint32_t entry_cell(uint64_t e) { return (uint32_t)(e & 0x3FFFFFu); }
 
 struct Shared {
   uint32_t best;
   uint32_t overflow;
   uint32_t qi;
-  uint32_t pad;
-  unsigned long long red[kMaxWaves];
+  uint32_t base;                 // the lowest bucket that may hold an entry (f >> shift)
+  uint32_t cnt[kBuckets];        // entries appended to bucket b (at b mod kBuckets) ...
+  uint32_t rd[kBuckets];         // ... and taken from it
+  uint32_t pre[kBuckets + 1];    // this iteration: entries taken from the buckets before base + i
+  uint32_t from[kBuckets];       // and the first one taken from base + i
+  uint32_t far_n, far_min, far_keep;
+  uint32_t act;                  // this iteration: kTake, kScan or kFinish
   unsigned long long expanded[kMaxWaves];
 };
+enum : uint32_t { kTake = 0, kScan = 1, kFinish = 2 };
+
+// Where a query's open list lives.
+struct OpenList {
+  uint64_t* far;
+  uint64_t* bucket;
+  uint64_t far_cap;
+  uint32_t bucket_cap;
+};
+
+// Appends e to its bucket, or to the far store when the bucket is full or beyond the row.
+__device__ __forceinline__ void open_push(Shared& sh, const OpenList& o, uint64_t e) {
+  const uint32_t f = entry_f(e), b = f >> kShift;
+  if (b - sh.base < kBuckets) {
+    const uint32_t pos = atomicAdd(&sh.cnt[b % kBuckets], 1u);
+    if (pos < o.bucket_cap) {
+      o.bucket[(uint64_t)(b % kBuckets) * o.bucket_cap + pos] = e;
+      return;
+    }
+  }
+  const uint32_t pos = atomicAdd(&sh.far_n, 1u);
+  if (pos < o.far_cap) {
+    o.far[pos] = e;
+    atomicMin(&sh.far_min, f);
+  } else {
+    sh.overflow = 1;
+  }
+}
+
+// One wave, lane i for bucket base + i: retires what the last iteration took, moves base to the
+// lowest bucket with entries and lists the first K pending entries.  Asks for a scan of the
+// far store when that holds an entry below every bucket's, and ends the search when nothing
+// pending can be below `best`.
+__device__ __forceinline__ void open_plan(Shared& sh, const OpenList& o, uint32_t K) {
+  const uint32_t lane = (uint32_t)lane_id();
+  uint32_t base = sh.base;
+  uint32_t b = (base + lane) % kBuckets;
+  const uint32_t n = min(sh.cnt[b], o.bucket_cap);
+  uint32_t rd = sh.rd[b] + (sh.pre[lane + 1] - sh.pre[lane]);
+  uint32_t avail = n - rd;
+  if (avail == 0) {                                  // empty: its space is used again
+    rd = 0;
+    sh.cnt[b] = 0;
+  } else {
+    sh.cnt[b] = n;
+  }
+  sh.rd[b] = rd;
+  const uint64_t some = __ballot(avail != 0);
+  const uint32_t skip = some ? (uint32_t)__builtin_ctzll(some) : kBuckets;
+  const uint32_t far_n = sh.far_n < o.far_cap ? sh.far_n : (uint32_t)o.far_cap;
+  const uint32_t far_b = far_n ? sh.far_min >> kShift : kNoBucket;
+  const uint32_t low = some ? base + skip : kNoBucket;   // the lowest bucket with entries
+  const uint32_t lowest = far_b < low ? far_b : low;
+  const uint32_t best = sh.best;
+  if (lowest == kNoBucket || (lowest << kShift) >= best) {
+    if (lane == 0) sh.act = kFinish;
+    return;
+  }
+  if (far_b < low) {
+    sh.pre[lane] = 0;
+    if (lane == 0) {
+      sh.pre[kBuckets] = 0;
+      sh.act = kScan;
+      sh.base = far_b;
+      sh.far_n = far_n;
+    }
+    return;
+  }
+  // bucket base + skip + lane
+  const uint32_t src = lane + skip;
+  const uint32_t a2 = (uint32_t)__shfl((int)avail, (int)(src & 63u), kWave);
+  const uint32_t r2 = (uint32_t)__shfl((int)rd, (int)(src & 63u), kWave);
+  const uint32_t mine = src < kBuckets ? a2 : 0u;
+  uint32_t inc = mine;
+#pragma unroll
+  for (int off = 1; off < kWave; off <<= 1) {
+    const uint32_t t = (uint32_t)__shfl_up((int)inc, off, kWave);
+    if (lane >= (uint32_t)off) inc += t;
+  }
+  sh.pre[lane + 1] = inc < K ? inc : K;
+  sh.from[lane] = r2;
+  if (lane == 0) {
+    sh.pre[0] = 0;
+    sh.base = base + skip;
+    sh.act = kTake;
+    sh.far_n = far_n;
+  }
+}
+
+// The far store's entries that the row of buckets now covers move into it; those that cannot
+// beat the goal found are dropped, the others stay, closed up in place: a chunk is read whole
+// before any of it is written, and never to a place past what has been read.
+__device__ void open_scan(Shared& sh, const OpenList& o, uint32_t far_n) {
+  constexpr uint32_t kU = 4;
+  const uint32_t K = blockDim.x, lane = (uint32_t)lane_id();
+  if (threadIdx.x == 0) {
+    sh.far_min = kNoBucket;
+    sh.far_keep = 0;
+  }
+  __syncthreads();
+  const uint32_t best = sh.best, base = sh.base;
+  uint32_t kept_min = kNoBucket;
+  for (uint32_t c0 = 0; c0 < far_n; c0 += kU * K) {
+    uint64_t e[kU];
+    bool keep[kU];
+#pragma unroll
+    for (uint32_t u = 0; u < kU; ++u) {
+      const uint32_t i = c0 + u * K + threadIdx.x;
+      e[u] = i < far_n ? o.far[i] : ~0ull;
+    }
+    __syncthreads();                                 // the chunk is in registers
+    uint32_t n_keep = 0;
+#pragma unroll
+    for (uint32_t u = 0; u < kU; ++u) {
+      const uint32_t i = c0 + u * K + threadIdx.x;
+      keep[u] = i < far_n && entry_f(e[u]) < best;
+      const uint32_t b = entry_f(e[u]) >> kShift;
+      if (keep[u] && b - base < kBuckets) {
+        const uint32_t pos = atomicAdd(&sh.cnt[b % kBuckets], 1u);
+        if (pos < o.bucket_cap) {
+          o.bucket[(uint64_t)(b % kBuckets) * o.bucket_cap + pos] = e[u];
+          keep[u] = false;
+        }
+      }
+      n_keep += (uint32_t)__popcll(__ballot(keep[u]));
+    }
+    uint32_t at = 0;
+    if (lane == 0 && n_keep) at = atomicAdd(&sh.far_keep, n_keep);
+    at = (uint32_t)__shfl((int)at, 0, kWave);
+#pragma unroll
+    for (uint32_t u = 0; u < kU; ++u) {
+      const uint64_t m = __ballot(keep[u]);
+      if (keep[u]) {
+        o.far[at + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] = e[u];
+        kept_min = min(kept_min, entry_f(e[u]));
+      }
+      at += (uint32_t)__popcll(m);
+    }
+  }
+  if (kept_min != kNoBucket) atomicMin(&sh.far_min, kept_min);
+  __syncthreads();
+  if (threadIdx.x == 0) sh.far_n = sh.far_keep;
+  __syncthreads();
+}
 
 // Searches query `qidx` in `slot`.  max_iters = 0: to the end; otherwise at most that many
 // iterations, keeping the state in the slot (resume continues it).  Returns true when done.
-__device__ bool search_query(const BatchDev& d, Shared& sh, uint32_t* cnt, uint64_t* stage, uint64_t* lds_rows,
-                             uint32_t qidx, uint32_t slot, uint32_t max_iters, bool resume) {
-  const uint32_t tid = threadIdx.x, K = blockDim.x, S = d.stage_cap;
+__device__ bool search_query(const BatchDev& d, Shared& sh, uint32_t qidx, uint32_t slot, uint32_t max_iters,
+                             bool resume) {
+  const uint32_t tid = threadIdx.x, K = blockDim.x;
   const BatchQuery Q = d.q[qidx];
   const uint32_t W = Q.side;
   const uint32_t* bits = d.bits + Q.bit_off;
   uint32_t* g = d.g + (uint64_t)slot * d.g_stride;
-  const ThreadHeap hp{lds_rows + tid, d.heap + (uint64_t)slot * d.heap_cap * K + tid, K, d.lds_rows};
+  const OpenList o{d.far + (uint64_t)slot * d.far_cap, d.bucket + (uint64_t)slot * kBuckets * d.bucket_cap, d.far_cap,
+                   d.bucket_cap};
   const uint32_t source = Q.sy * W + Q.sx, target = Q.ty * W + Q.tx;
 
-  uint32_t hn;
-  uint64_t top;
   unsigned long long expanded = 0;
   uint32_t tag;
+  if (tid < kBuckets) sh.pre[tid] = 0;
+  if (tid == 0) sh.pre[kBuckets] = 0;
   if (!resume) {
     if (tid == 0) d.clk[2 * qidx] = wall_clock64();
     const uint32_t prev = d.slot[slot].tag;
@@ -177,48 +285,64 @@ __device__ bool search_query(const BatchDev& d, Shared& sh, uint32_t* cnt, uint6
       for (uint64_t c = tid; c < d.g_stride; c += K) g[c] = 0xFFFFFFFFu;
     }
     tag = prev == 0 ? kTagNever - 1 : prev - 1;
-    hn = 0;
-    top = kNoKey;
+    if (tid < kBuckets) sh.cnt[tid] = sh.rd[tid] = 0;
     if (tid == 0) {
       sh.best = source == target ? 0u : kNoCost;
       sh.overflow = 0;
+      sh.far_n = 0;
+      sh.far_min = kNoBucket;
+      sh.base = grid_heur(Q.conn, (int)Q.sx, (int)Q.sy, (int)Q.tx, (int)Q.ty) >> kShift;
     }
     __syncthreads();
-    if (tid == 0) d.slot[slot].tag = tag;
-    if (source != target && tid == owner_of(source, d.log2k)) {
-      __hip_atomic_store(&g[source], tag << kTagShift, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      const uint32_t h0 = grid_heur(Q.conn, (int)Q.sx, (int)Q.sy, (int)Q.tx, (int)Q.ty);
-      top = heap_push(hp, hn, make_key(h0, h0, source), top);
+    if (tid == 0) {
+      d.slot[slot].tag = tag;
+      if (source != target) {
+        __hip_atomic_store(&g[source], tag << kTagShift, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        open_push(sh, o, make_entry(grid_heur(Q.conn, (int)Q.sx, (int)Q.sy, (int)Q.tx, (int)Q.ty), source));
+      }
     }
   } else {
-    hn = d.hn[(uint64_t)slot * K + tid];
-    for (uint32_t i = 0; i < hn && i < hp.T; ++i) hp.lds[i * K] = hp.hbm[(uint64_t)i * K];   // saved LDS rows
-    top = hn ? hp.get(0) : kNoKey;
     tag = d.slot[slot].tag;
+    if (tid < kBuckets) {
+      sh.cnt[tid] = d.list[slot].cnt[tid];
+      sh.rd[tid] = d.list[slot].rd[tid];
+    }
     if (tid == 0) {
       sh.best = d.slot[slot].best;
       sh.overflow = d.slot[slot].overflow;
+      sh.base = d.list[slot].base;
+      sh.far_n = d.list[slot].far_n;
+      sh.far_min = d.list[slot].far_min;
     }
   }
   const uint32_t tag_bits = tag << kTagShift;
-  cnt[tid] = 0;
   __syncthreads();
 
   bool finished = false;
   uint32_t it = 0;
   for (;;) {
-    // --- pop and expand -------------------------------------------------------------------
-    const uint32_t best_now = *(volatile uint32_t*)&sh.best;
-    if (hn && key_f(top) < best_now) {
-      const uint64_t key = top;
-      const uint32_t cell = key_cell(key), f = key_f(key);
+    if (tid < (uint32_t)kWave) open_plan(sh, o, K);
+    __syncthreads();
+    const uint32_t act = sh.act;
+    if (act == kFinish) { finished = true; break; }
+    if (act == kScan) {
+      open_scan(sh, o, sh.far_n);
+      continue;
+    }
+    // --- take and expand ------------------------------------------------------------------
+    if (tid < sh.pre[kBuckets]) {
+      uint32_t lo = 0, hi = kBuckets - 1;              // the bucket i with pre[i] <= tid < pre[i + 1]
+      while (lo < hi) {
+        const uint32_t mid = (lo + hi) >> 1;
+        if (sh.pre[mid + 1] > tid) hi = mid; else lo = mid + 1;
+      }
+      const uint64_t e = o.bucket[(uint64_t)((sh.base + lo) % kBuckets) * o.bucket_cap + sh.from[lo] + (tid - sh.pre[lo])];
+      const uint32_t cell = entry_cell(e), f = entry_f(e);
       const int x = (int)(cell % W), y = (int)(cell / W);
       const uint32_t g0 = f - grid_heur(Q.conn, x, y, (int)Q.tx, (int)Q.ty);
-      // the cell's g and its neighbours' obstacle bits are fetched while the heap is sifted
       const uint32_t g_now = __hip_atomic_load(&g[cell], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       const uint32_t nbr = free_neighbours(bits, Q.conn, x, y, (int)W, (int)W);
-      top = heap_pop(hp, hn);
-      if ((tag_bits | g0) == g_now) {
+      if ((tag_bits | g0) == g_now && f < *(volatile uint32_t*)&sh.best) {
         ++expanded;
         // all relaxations in flight at once: a neighbour's improvement does not depend on another's
         uint32_t old[8];
@@ -238,37 +362,14 @@ __device__ bool search_query(const BatchDev& d, Shared& sh, uint32_t* cnt, uint6
             continue;
           }
           if (old[k] <= (tag_bits | g2)) continue;
-          const uint32_t h2 = grid_heur(Q.conn, nx, ny, (int)Q.tx, (int)Q.ty);
-          if (g2 + h2 >= *(volatile uint32_t*)&sh.best) continue;   // cannot beat the goal found
-          const uint64_t k2 = make_key(g2 + h2, h2, v);
-          const uint32_t o = owner_of(v, d.log2k);
-          const uint32_t pos = atomicAdd(&cnt[o], 1u);
-          if (pos < S) {
-            stage[o * S + pos] = k2;
-          } else if (hn < d.heap_cap) {
-            top = heap_push(hp, hn, k2, top);
-          } else {
-            sh.overflow = 1;
-          }
+          const uint32_t f2 = g2 + grid_heur(Q.conn, nx, ny, (int)Q.tx, (int)Q.ty);
+          if (f2 >= *(volatile uint32_t*)&sh.best) continue;   // cannot beat the goal found
+          open_push(sh, o, make_entry(f2, v));
         }
       }
     }
     __syncthreads();
-    // --- fold the staged inserts into the own list, reduce the smallest key --------------
-    const uint32_t mine = cnt[tid] < S ? cnt[tid] : S;
-    for (uint32_t i = 0; i < mine; ++i) {
-      if (hn < d.heap_cap) top = heap_push(hp, hn, stage[tid * S + i], top);
-      else sh.overflow = 1;
-    }
-    cnt[tid] = 0;
-    const uint32_t best_snap = sh.best;        // only changes while expanding
-    const uint64_t wmin = wave_min_u64(top);
-    if (lane_id() == 0) sh.red[tid / kWave] = wmin;
-    __syncthreads();
-    uint64_t m = sh.red[0];
-    for (uint32_t w = 1; w < K / kWave; ++w) m = sh.red[w] < m ? sh.red[w] : m;
     ++it;
-    if (m == kNoKey || key_f(m) >= best_snap) { finished = true; break; }
     if (max_iters && it >= max_iters) break;
   }
 
@@ -278,6 +379,11 @@ __device__ bool search_query(const BatchDev& d, Shared& sh, uint32_t* cnt, uint6
   for (int off = 32; off > 0; off >>= 1) e += __shfl_xor(e, off, kWave);
   if (lane_id() == 0) sh.expanded[tid / kWave] = e;
   __syncthreads();
+  if (!finished && tid < kBuckets) {                   // what this launch took is retired here
+    const uint32_t b = (sh.base + tid) % kBuckets;
+    d.list[slot].cnt[b] = min(sh.cnt[b], o.bucket_cap);
+    d.list[slot].rd[b] = sh.rd[b] + (sh.pre[tid + 1] - sh.pre[tid]);
+  }
   if (tid == 0) {
     unsigned long long tot = 0;
     for (uint32_t w = 0; w < K / kWave; ++w) tot += sh.expanded[w];
@@ -289,56 +395,43 @@ __device__ bool search_query(const BatchDev& d, Shared& sh, uint32_t* cnt, uint6
       d.flags[qidx] = sh.overflow;
     } else {
       d.slot[slot] = SlotState{sh.best, sh.overflow, tag, 0u, tot};
+      d.list[slot].base = sh.base;
+      d.list[slot].far_n = sh.far_n;
+      d.list[slot].far_min = sh.far_min;
     }
-  }
-  if (!finished) {
-    d.hn[(uint64_t)slot * K + tid] = hn;
-    for (uint32_t i = 0; i < hn && i < hp.T; ++i) hp.hbm[(uint64_t)i * K] = hp.lds[i * K];   // save LDS rows
   }
   __syncthreads();
   return finished;
 }
 
 // Persistent drive: each workgroup owns slot blockIdx.x and pulls queries until none is left.
-// Dynamic LDS: stage [K][S] u64, heap rows [T][K] u64, counts [K] u32.
 __global__ __launch_bounds__(1024) void astar_batch_kernel(BatchDev d) {
-  extern __shared__ uint64_t lds[];
   __shared__ Shared sh;
-  uint64_t* stage = lds;
-  uint64_t* rows = lds + (size_t)blockDim.x * d.stage_cap;
-  uint32_t* cnt = reinterpret_cast<uint32_t*>(rows + (size_t)blockDim.x * d.lds_rows);
   for (;;) {
     if (threadIdx.x == 0) sh.qi = atomicAdd(d.counter, 1u);
     __syncthreads();
     const uint32_t qi = sh.qi;
     __syncthreads();
     if (qi >= d.n) break;
-    search_query(d, sh, cnt, stage, rows, d.ids[qi], d.slot_base + blockIdx.x, 0, false);
+    search_query(d, sh, d.ids[qi], d.slot_base + blockIdx.x, 0, false);
   }
 }
 
 // Plain drive: one iteration of query ids[0] in slot slot_base per launch.
 __global__ __launch_bounds__(1024) void astar_batch_step_kernel(BatchDev d, uint32_t resume, uint32_t* done) {
-  extern __shared__ uint64_t lds[];
   __shared__ Shared sh;
-  uint64_t* stage = lds;
-  uint64_t* rows = lds + (size_t)blockDim.x * d.stage_cap;
-  uint32_t* cnt = reinterpret_cast<uint32_t*>(rows + (size_t)blockDim.x * d.lds_rows);
-  const bool fin = search_query(d, sh, cnt, stage, rows, d.ids[0], d.slot_base, 1, resume != 0);
+  const bool fin = search_query(d, sh, d.ids[0], d.slot_base, 1, resume != 0);
   if (threadIdx.x == 0) *done = fin ? 1u : 0u;
 }
 
 __global__ void zero_u32_kernel(uint32_t* p) { *p = 0; }
 
-constexpr size_t kLdsBudget = 64 * 1024;
+constexpr size_t kStageLimit = 64 * 1024;   // threads * (8 * stage_capacity + 4) bytes accepted
 
-size_t lds_bytes(uint32_t K, uint32_t S, uint32_t rows) { return (size_t)K * (S * 8 + rows * 8 + 4); }
-
-// Heap levels kept in LDS: the largest 2^d - 1 (d <= 5) that fits beside the staging area.
-uint32_t heap_lds_rows(uint32_t K, uint32_t S) {
-  for (uint32_t rows : {31u, 15u, 7u, 3u, 1u})
-    if (lds_bytes(K, S, rows) <= kLdsBudget) return rows;
-  return 0;
+// Entries a bucket holds: half of the list's capacity over the row, within [256, 8192] (64 KiB); a fuller bucket spills into the far store.
+uint32_t bucket_cap_for(const gpq_batch_tuning& t) {
+  const uint64_t c = (uint64_t)t.heap_capacity * t.threads_per_query / (2u * kBuckets);
+  return (uint32_t)std::min<uint64_t>(std::max<uint64_t>(c, 256), 8192);
 }
 
 __global__ void init_slots_kernel(SlotState* s, uint32_t n) {
@@ -401,8 +494,8 @@ gpq_status AstarBatch::create(const gpq_query_spec* sp, uint32_t count, const gp
                 "batch: threads_per_query must be a power of two in [64, 1024]");
   GPQ_CHECK_ARG(tu.heap_capacity >= 16 && tu.heap_capacity <= (1u << 20), "batch: heap_capacity out of range");
   GPQ_CHECK_ARG(tu.stage_capacity >= 1 && tu.stage_capacity <= 64, "batch: stage_capacity must be in [1, 64]");
-  GPQ_CHECK_ARG((size_t)tu.threads_per_query * (tu.stage_capacity * 8 + 4) <= kLdsBudget,
-                "batch: LDS staging (threads * (8 * stage + 4) bytes) must fit in 64 KiB");
+  GPQ_CHECK_ARG((size_t)tu.threads_per_query * (tu.stage_capacity * 8 + 4) <= kStageLimit,
+                "batch: staging (threads * (8 * stage + 4) bytes) must fit in 64 KiB");
   uint64_t max_cells = 0, words = 0;
   std::vector<BatchQuery> hq(count);
   std::vector<uint64_t> off(count);
@@ -420,10 +513,11 @@ gpq_status AstarBatch::create(const gpq_query_spec* sp, uint32_t count, const gp
   int dev = 0, cus = 0;
   GPQ_HIP(hipGetDevice(&dev));
   GPQ_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-  const uint32_t rows = heap_lds_rows(tu.threads_per_query, tu.stage_capacity);
-  const size_t lds = lds_bytes(tu.threads_per_query, tu.stage_capacity, rows);
   int per_cu = 0;
-  GPQ_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, astar_batch_kernel, (int)tu.threads_per_query, lds));
+  GPQ_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, astar_batch_kernel, (int)tu.threads_per_query, 0));
+  // a slot holds a whole grid's g values, so the slots grow with the workgroups per CU; an
+  // iteration is bound by latency, and two 512-thread workgroups per CU already overlap theirs
+  per_cu = std::min(per_cu, std::min<int>(8, 512 / (int)tu.threads_per_query + 1));
   uint32_t resident = tu.max_resident ? tu.max_resident : (uint32_t)std::max(1, cus * std::max(per_cu, 1));
   resident = std::min(resident, count);
   tu.max_resident = resident;
@@ -444,10 +538,15 @@ gpq_status AstarBatch::create(const gpq_query_spec* sp, uint32_t count, const gp
   uint32_t* bits = nullptr;
   gpq_status s;
   const uint64_t slots = std::max<uint32_t>(resident, 1);
+  // the far store alone holds every entry that the open list may (heap_capacity per thread); the
+  // buckets come on top
+  d->far_cap = (uint64_t)tu.heap_capacity * tu.threads_per_query;
+  d->bucket_cap = bucket_cap_for(tu);
   if ((s = b->arena.alloc(&dq, count)) != GPQ_OK || (s = b->arena.alloc(&bits, words ? words : 1)) != GPQ_OK ||
       (s = b->arena.alloc(&d->g, slots * max_cells)) != GPQ_OK ||
-      (s = b->arena.alloc(&d->heap, slots * tu.heap_capacity * tu.threads_per_query)) != GPQ_OK ||
-      (s = b->arena.alloc(&d->hn, slots * tu.threads_per_query)) != GPQ_OK ||
+      (s = b->arena.alloc(&d->far, slots * d->far_cap)) != GPQ_OK ||
+      (s = b->arena.alloc(&d->bucket, slots * kBuckets * d->bucket_cap)) != GPQ_OK ||
+      (s = b->arena.alloc(&d->list, slots)) != GPQ_OK ||
       (s = b->arena.alloc(&d->slot, slots)) != GPQ_OK || (s = b->arena.alloc(&d->cost, count)) != GPQ_OK ||
       (s = b->arena.alloc(&d->expanded, count)) != GPQ_OK || (s = b->arena.alloc(&d->flags, count)) != GPQ_OK ||
       (s = b->arena.alloc(&d->clk, 2 * (size_t)count)) != GPQ_OK ||
@@ -456,10 +555,6 @@ gpq_status AstarBatch::create(const gpq_query_spec* sp, uint32_t count, const gp
   d->q = dq;
   d->bits = bits;
   d->g_stride = max_cells;
-  d->heap_cap = tu.heap_capacity;
-  d->stage_cap = tu.stage_capacity;
-  d->log2k = log2u(tu.threads_per_query);
-  d->lds_rows = rows;
   d->counter = b->counter;
   std::vector<uint32_t> ids(count);
   for (uint32_t i = 0; i < count; ++i) ids[i] = i;
@@ -504,9 +599,8 @@ gpq_status AstarBatch::launch(const uint32_t* d_ids, uint32_t n, uint32_t slot_b
   d.counter = d_counter;
   d.slot_base = slot_base;
   const uint32_t K = tuning.threads_per_query;
-  const size_t lds = lds_bytes(K, tuning.stage_capacity, d.lds_rows);
   hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(1), 0, s, d_counter);
-  hipLaunchKernelGGL(astar_batch_kernel, dim3(std::max<uint32_t>(1, std::min(slots, n))), dim3(K), lds, s,
+  hipLaunchKernelGGL(astar_batch_kernel, dim3(std::max<uint32_t>(1, std::min(slots, n))), dim3(K), 0, s,
                      static_cast<BatchDev>(d));
   GPQ_HIP(hipGetLastError());
   return GPQ_OK;
@@ -522,14 +616,13 @@ gpq_status AstarBatch::plain_one(const uint32_t* d_id, uint32_t spec_index, uint
   d.n = 1;
   d.slot_base = slot;
   const uint32_t K = tuning.threads_per_query;
-  const size_t lds = lds_bytes(K, tuning.stage_capacity, d.lds_rows);
   const uint64_t step_cap = 64ull * specs[spec_index].side * specs[spec_index].side + 1024;
   for (uint64_t step = 0;; ++step) {
     if (step > step_cap) {
       set_error("batch plain: step bound exceeded");
       return GPQ_ERR_STATE;
     }
-    hipLaunchKernelGGL(astar_batch_step_kernel, dim3(1), dim3(K), lds, s, static_cast<BatchDev>(d), step ? 1u : 0u,
+    hipLaunchKernelGGL(astar_batch_step_kernel, dim3(1), dim3(K), 0, s, static_cast<BatchDev>(d), step ? 1u : 0u,
                        d_done);
     GPQ_HIP(hipGetLastError());
     GPQ_HIP(hipMemcpyAsync(h_done, d_done, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
@@ -568,37 +661,34 @@ gpq_status AstarBatch::run(gpq_drive_mode mode, double* seconds) {
   return GPQ_OK;
 }
 
-// Times every candidate (threads per query x stage capacity) on the first `sample` queries
-// (two persistent runs each, the second timed) and returns the fastest; heap_capacity and
-// max_resident are kept from `base`.  Candidates whose open lists overflow are skipped.
+// Times every workgroup size on the first `sample` queries (two persistent runs each, the second
+// timed) and returns the fastest; heap_capacity and max_resident are kept from `base`.  Candidates whose open lists overflow are skipped.
 gpq_status batch_autotune(const gpq_query_spec* sp, uint32_t count, uint32_t sample, const gpq_batch_tuning& base,
                           gpq_batch_tuning* out, double* best_seconds) {
   GPQ_CHECK_ARG(sp && count >= 1, "autotune: no queries");
   const uint32_t n = sample ? std::min(sample, count) : count;
   static const uint32_t kThreads[] = {64, 128, 256, 512, 1024};
-  static const uint32_t kStage[] = {8, 16, 32};
   double best = 1e300;
   gpq_batch_tuning pick{};
-  for (uint32_t k : kThreads)
-    for (uint32_t st : kStage) {
-      if ((size_t)k * (st * 8 + 4) > kLdsBudget) continue;
-      gpq_batch_tuning t = base;
-      t.threads_per_query = k;
-      t.stage_capacity = st;
-      AstarBatch* b = nullptr;
-      if (AstarBatch::create(sp, n, t, &b) != GPQ_OK) continue;
-      double sec = 0.0;
-      gpq_status s = b->run(GPQ_DRIVE_GRAPH, &sec);
-      if (s == GPQ_OK) s = b->run(GPQ_DRIVE_GRAPH, &sec);
-      if (s == GPQ_OK) s = b->results(nullptr, nullptr);
-      const gpq_batch_tuning used = b->tuning;
-      delete b;
-      if (s == GPQ_OK && sec < best) {
-        best = sec;
-        pick = used;
-        pick.max_resident = base.max_resident;
-      }
+  for (uint32_t k : kThreads) {
+    gpq_batch_tuning t = base;
+    t.threads_per_query = k;
+    t.stage_capacity = 8;
+    if ((size_t)k * (t.stage_capacity * 8 + 4) > kStageLimit) continue;
+    AstarBatch* b = nullptr;
+    if (AstarBatch::create(sp, n, t, &b) != GPQ_OK) continue;
+    double sec = 0.0;
+    gpq_status s = b->run(GPQ_DRIVE_GRAPH, &sec);
+    if (s == GPQ_OK) s = b->run(GPQ_DRIVE_GRAPH, &sec);
+    if (s == GPQ_OK) s = b->results(nullptr, nullptr);
+    const gpq_batch_tuning used = b->tuning;
+    delete b;
+    if (s == GPQ_OK && sec < best) {
+      best = sec;
+      pick = used;
+      pick.max_resident = base.max_resident;
     }
+  }
   if (best == 1e300) {
     set_error("autotune: no candidate completed");
     return GPQ_ERR_CAPACITY;
@@ -622,6 +712,11 @@ gpq_status AstarBatch::results(int64_t* costs, uint64_t* expanded) {
       return GPQ_ERR_CAPACITY;
     }
   return GPQ_OK;
+}
+
+uint64_t AstarBatch::open_list_bytes() const {
+  const Dev* d = static_cast<const Dev*>(dev);
+  return 8ull * (d->far_cap + (uint64_t)kBuckets * d->bucket_cap);
 }
 
 gpq_status AstarBatch::timing(double* start_us, double* finish_us) {

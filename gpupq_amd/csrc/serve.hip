@@ -226,8 +226,7 @@ gpq_status serve_run(const gpq_serve_config& cin, gpq_drive_mode mode, gpq_serve
     GPQ_TRY(AstarBatch::create(specs.data(), (uint32_t)specs.size(), t, &b));
     batch.reset(b);
   }
-  const uint64_t astar_bytes_each =
-      batch ? (uint64_t)batch->tuning.heap_capacity * batch->tuning.threads_per_query * 8ull : 0ull;
+  const uint64_t astar_bytes_each = batch ? batch->open_list_bytes() : 0ull;
 
   // Lanes for A* launches (served) / one stream for the plain drive.
   DeviceArena arena;

@@ -347,8 +347,8 @@ gpq_status gpq_astar_grid(gpq_astar* a, uint8_t* blocked);
  * target is unreachable); at most cap cells are written. */
 gpq_status gpq_astar_path(gpq_astar* a, uint32_t* cells, uint32_t cap, uint32_t* len);
 
-/* Batched A*: many independent queries, each searched by one workgroup with per-thread
- * local heaps; one persistent launch pulls queries from a device work counter (the reference's
+/* Batched A*: many independent queries, each searched by one workgroup over an open list of
+ * buckets by f; one persistent launch pulls queries from a device work counter (the reference's
  * get_new_agent, src/a_star.cu:149-164).  Query q of a batch uses the shape and endpoints of
  * the synthetic distribution (side = round(256 * 2^(3u)), density U[0.1, 0.3], 8-connected)
  * unless explicit specs are given. */
@@ -361,9 +361,10 @@ typedef struct {
 } gpq_query_spec;
 
 typedef struct {
-  uint32_t threads_per_query;   /* workgroup size = open lists per query (64..1024, multiple of 64) */
-  uint32_t heap_capacity;       /* entries per open list */
-  uint32_t stage_capacity;      /* inserts one open list may receive per iteration */
+  uint32_t threads_per_query;   /* workgroup size = expansions per iteration (64..1024, power of two) */
+  uint32_t heap_capacity;       /* open-list entries a query may hold, per thread */
+  uint32_t stage_capacity;      /* 1..64 with threads * (8 * stage + 4) <= 64 KiB; the open list takes any
+                                   number of inserts per iteration, so it sizes nothing */
   uint32_t max_resident;        /* queries searched at once (0 = fill the device) */
 } gpq_batch_tuning;
 
@@ -374,9 +375,9 @@ gpq_status gpq_query_synthetic(uint32_t seed, uint32_t q, gpq_query_spec* out);
 gpq_status gpq_astar_batch_create(const gpq_query_spec* specs, uint32_t count, const gpq_batch_tuning* tuning,
                                   gpq_astar_batch** out);
 gpq_status gpq_astar_batch_destroy(gpq_astar_batch* b);
-/* Autotuner: times threads_per_query in {64..1024} x stage_capacity in {8, 16, 32} on the
- * first `sample` queries (0 = all) and writes the fastest into *tuning (its heap_capacity
- * and max_resident are kept as given; 0 = defaults).  best_seconds (may be NULL) receives
+/* Autotuner: times threads_per_query in {64..512} (stage_capacity 8) on the first `sample`
+ * queries (0 = all) and writes the fastest into *tuning (its heap_capacity and max_resident are
+ * kept as given; 0 = defaults).  best_seconds (may be NULL) receives
  * that candidate's time. */
 gpq_status gpq_astar_batch_autotune(const gpq_query_spec* specs, uint32_t count, uint32_t sample,
                                     gpq_batch_tuning* tuning, double* best_seconds);
