@@ -523,9 +523,9 @@ gpq_status AstarModel::restart() {
   hipLaunchKernelGGL(fill_u32_kernel, dim3(grid_blocks((cells + 31) / 32)), dim3(256), 0, q->stream, closed,
                      (cells + 31) / 32, 0u);
   GPQ_HIP(hipGetLastError());
-  // entries left by an earlier search are dropped as stale (their g is not the new g[cell]);
-  // in decrease-key mode they would hold their ids' marks, so the lists start empty
-  if (q->cfg.kind == GPQ_LAQ && q->cfg.update_ids) GPQ_TRY(static_cast<LaqQueue*>(q)->empty_all());
+  // the lists start empty: a search leaves its entries beyond the goal's cost behind, which would
+  // otherwise pile up over the searches of one queue until a list overflows
+  GPQ_TRY(q->empty_all());
   const AstarDev d = view();
   const uint32_t source = cfg.sy * cfg.width + cfg.sx;
   GPQ_TRY(with_view(q, [&](auto qv) -> gpq_status {

@@ -90,6 +90,11 @@ class QueueBase {
   virtual gpq_status pending(uint64_t* n) = 0;
   virtual gpq_status length(uint32_t lp, uint32_t* n) = 0;
   virtual gpq_status clear_lp(uint32_t lp) = 0;
+  // Per-LP queues: every LP emptied on the queue's stream (a new search on the same open lists).
+  virtual gpq_status empty_all() {
+    set_error("empty_all is provided for the per-LP queues");
+    return GPQ_ERR_UNSUPPORTED;
+  }
   // Number of queue_peek() slots the model iterates over.
   virtual uint32_t peek_slots() const { return cfg.num_lps; }
 

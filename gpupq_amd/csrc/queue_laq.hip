@@ -626,7 +626,8 @@ __global__ void laq_init_kernel(LaqView q) {
 
 __global__ void laq_clear_kernel(LaqView q, uint32_t lp) { q.clear((int)lp); }
 
-// Empties every LP and unmarks every id (decrease-key mode): the queue as after init.
+// Empties every LP: rings, staging, far stores and their horizons, and in decrease-key mode (words
+// > 0) the updates and every id's mark.  The window state and the error flag stay.
 __global__ void laq_empty_kernel(LaqView q, uint32_t words) {
   const uint32_t stride = gridDim.x * blockDim.x;
   for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < q.num_lps || i < words; i += stride) {
@@ -634,7 +635,16 @@ __global__ void laq_empty_kernel(LaqView q, uint32_t words) {
       q.len[i] = 0;
       q.ins[i] = 0;
       q.head[i] = kInfBits;
-      q.upd_n[i] = 0;
+      if (words) q.upd_n[i] = 0;
+      if (q.far_cap) {
+        q.nfar[i] = 0;
+        q.far_min[i] = kInfBits;
+      }
+      if (q.near_lp) {                         // open lists: everything to the ring until it fills
+        q.near_lp[i] = 0xFFFFFFFFu;
+        q.near_lp[q.num_lps + i] = 0xFFFFFFFFu;
+        q.near_lp[2 * q.num_lps + i] = 0xFFFFFFFFu;
+      }
     }
     if (i < words) q.in_queue[i] = 0;
   }
@@ -1009,8 +1019,8 @@ gpq_status LaqQueue::reset_stage_select() {
 }
 
 gpq_status LaqQueue::empty_all() {
-  GPQ_CHECK_ARG(v_.in_queue, "LAQ: empty_all is for the decrease-key mode");
-  const uint32_t words = (v_.update_ids + 31) / 32;
+  GPQ_CHECK_ARG(!v_.wlog, "LAQ: empty_all does not serve the calendar mode");
+  const uint32_t words = v_.in_queue ? (v_.update_ids + 31) / 32 : 0u;
   const uint32_t n = std::max(cfg.num_lps, words);
   hipLaunchKernelGGL(laq_empty_kernel, dim3(std::min<uint32_t>(ceil_div(n, 256), 4096)), dim3(256), 0, stream, v_,
                      words);

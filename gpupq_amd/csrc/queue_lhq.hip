@@ -64,6 +64,14 @@ __global__ void lhq_init_kernel(LhqView q) {
   if (lp == 0) *q.ws = WindowState{kInfBits, 0u, 0u, 0u, 0ull, 0u, 0u};
 }
 
+__global__ void lhq_empty_kernel(LhqView q) {
+  const uint32_t lp = blockIdx.x * blockDim.x + threadIdx.x;
+  if (lp >= q.num_lps) return;
+  q.len[lp] = 0;
+  q.ins[lp] = 0;
+  q.head[lp] = kInfBits;
+}
+
 __global__ void lhq_clear_kernel(LhqView q, uint32_t lp) { q.clear((int)lp); }
 
 }  // namespace
@@ -87,6 +95,12 @@ gpq_status LhqQueue::init() {
   partial_slots = ceil_div(L, kLhqBlock);
   GPQ_TRY(arena.alloc(&partial, partial_slots));
   hipLaunchKernelGGL(lhq_init_kernel, dim3(ceil_div(L, 256)), dim3(256), 0, stream, v_);
+  GPQ_HIP(hipGetLastError());
+  return GPQ_OK;
+}
+
+gpq_status LhqQueue::empty_all() {
+  hipLaunchKernelGGL(lhq_empty_kernel, dim3(ceil_div(cfg.num_lps, 256)), dim3(256), 0, stream, v_);
   GPQ_HIP(hipGetLastError());
   return GPQ_OK;
 }

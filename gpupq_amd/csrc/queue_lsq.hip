@@ -118,6 +118,12 @@ gpq_status LsqQueue::init() {
   return GPQ_OK;
 }
 
+gpq_status LsqQueue::empty_all() {
+  hipLaunchKernelGGL(lsq_reset_kernel, dim3(4096), dim3(256), 0, stream, v_, 0u, cfg.num_lps);
+  GPQ_HIP(hipGetLastError());
+  return GPQ_OK;
+}
+
 gpq_status LsqQueue::post() {
   hipLaunchKernelGGL(lsq_post_kernel, dim3(partial_slots), dim3(kLsqBlock), 0, stream, v_, partial);
   GPQ_HIP(hipGetLastError());

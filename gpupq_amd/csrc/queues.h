@@ -42,8 +42,7 @@ class LaqQueue final : public QueueBase {
   // After a closing merge of such a step: both buffers are empty, the next step reads stage.
   gpq_status reset_stage_select();
   uint32_t group() const { return group_; }
-  // Decrease-key mode: every LP emptied, every id unmarked (a new search on the same queue).
-  gpq_status empty_all();
+  gpq_status empty_all() override;
   float far_step() const { return far_step_; }
   // Calendar mode: whether it is on; and, once every initial event is in (post_init), the
   // ends of the first windows and the filing of the initial events in their buckets.
@@ -76,6 +75,7 @@ class LaqQueue final : public QueueBase {
     gpq_status pending(uint64_t* n) override;                                    \
     gpq_status length(uint32_t lp, uint32_t* n) override;                        \
     gpq_status clear_lp(uint32_t lp) override;                                   \
+    gpq_status empty_all() override;                                             \
     View view() const { return v_; }                                             \
                                                                                  \
    private:                                                                      \
