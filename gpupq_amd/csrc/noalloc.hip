@@ -2,16 +2,16 @@
 // HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).
 //
 // gpq_sort_events_noalloc sorts caller-owned device records with the same kernels as
-// gpq_selftest_sort (one bitonic tile sort, then merge-path passes), but its ping-pong
-// partner buffer and its device-side record count live in `scratch`, a file-scope device
-// array of kScratchBytes that every GPU the library runs on holds until the process ends.
+// gpq_selftest_sort (one tile sort, then levels of up to 128-way merges), but its ping-pong
+// partner buffer and its sample order live in `scratch`, a file-scope device array of
+// kScratchBytes that every GPU the library runs on holds until the process ends.
 // The array's address on the current device is looked up once per device with
 // hipGetSymbolAddress and kept; host code only ever passes that address to kernels.
 //
 // Every call on one GPU shares that GPU's array, so calls that overlap on one GPU (on
 // different streams, or from different host threads) race on it and must be serialised by
-// the caller.  The array keeps the last call's contents; the count word is rewritten by each
-// call and the partner buffer is written before it is read, so nothing needs clearing.
+// the caller.  The array keeps the last call's contents; every word that a call reads it has
+// written before, so nothing needs clearing.
 #include <array>
 #include <mutex>
 
@@ -21,8 +21,8 @@ namespace gpq {
 namespace {
 
 constexpr uint32_t kNoAllocMaxRecords = 1u << 20;       // 16 MiB of partner buffer
-constexpr size_t kScratchHeader = 256;                  // the record count, padded to 256 B
-constexpr size_t kScratchBytes = kScratchHeader + sizeof(Event) * (size_t)kNoAllocMaxRecords;
+constexpr size_t kOrderBytes = 128 * 1024 + 256;        // sample order: a word per 32 records and one more
+constexpr size_t kScratchBytes = kOrderBytes + sizeof(Event) * (size_t)kNoAllocMaxRecords;
 constexpr int kMaxDevices = 64;
 
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
@@ -44,10 +44,6 @@ gpq_status scratch_on_current_device(unsigned char** out) {
   }
   *out = g_scratch_ptr[dev];
   return GPQ_OK;
-}
-
-__global__ void noalloc_set_count_kernel(uint32_t* count, uint32_t n) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) *count = n;
 }
 
 }  // namespace
@@ -77,23 +73,11 @@ extern "C" gpq_status gpq_sort_events_noalloc(const gpq_event* d_in, uint32_t n,
   }
   unsigned char* base = nullptr;
   GPQ_TRY(gpq::scratch_on_current_device(&base));
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  uint32_t* d_n = reinterpret_cast<uint32_t*>(base);
-  Event* partner = reinterpret_cast<Event*>(base + gpq::kScratchHeader);
-  hipLaunchKernelGGL(gpq::noalloc_set_count_kernel, dim3(1), dim3(64), 0, s, d_n, n);
-  GPQ_HIP(hipGetLastError());
-  // The tile sort writes its first buffer and each merge pass swaps the two; with the pass
-  // count's parity the sorted run ends in the caller's output array.
-  uint32_t passes = 0;
-  for (uint64_t w = gpq::kSortTile; w < n; w *= 2) ++passes;
-  Event* out = reinterpret_cast<Event*>(d_out);
-  Event* first = (passes & 1u) ? partner : out;
-  Event* second = (passes & 1u) ? out : partner;
-  Event* sorted = nullptr;
-  GPQ_TRY(gpq::sort_records(reinterpret_cast<const Event*>(d_in), first, second, d_n, n, s, &sorted));
-  if (sorted != out) {
-    gpq::set_error("sort_events_noalloc: sorted run left in the scratch buffer");
+  Event* partner = reinterpret_cast<Event*>(base + gpq::kOrderBytes);
+  if (sizeof(uint32_t) * gpq::sort_order_words(n) > gpq::kOrderBytes) {
+    gpq::set_error("sort_events_noalloc: sample order exceeds its scratch");
     return GPQ_ERR_STATE;
   }
-  return GPQ_OK;
+  return gpq::sort_records(reinterpret_cast<const Event*>(d_in), reinterpret_cast<Event*>(d_out), partner,
+                           reinterpret_cast<uint32_t*>(base), nullptr, n, static_cast<hipStream_t>(stream));
 }

@@ -2,7 +2,7 @@
 //   queue_pre : one safe event per LP selected from the sorted array (parallel prefix
 //               search + per-LP atomicMin + stable compaction), where the reference runs
 //               a single-thread scan (mark_safe_events, src/global_array_queue.cu:147-179).
-//   queue_post: the step's inserts are sorted (tile sort + merge passes) and merged with
+//   queue_post: the step's inserts are sorted (tile sort + 128-way merges) and merged with
 //               the array minus the selected records into the other buffer; the reference
 //               appends them and mergesorts the whole array (src/global_array_queue.cu:62-74,
 //               229-262).  Both are device-resident: no host reads between kernels.
@@ -93,7 +93,7 @@ gpq_status GaqQueue::init() {
   const uint64_t enq_cap = (uint64_t)cfg.num_lps * cfg.stage_per_lp;
   GPQ_CHECK_ARG(enq_cap < (1ull << 31), "GAQ: num_lps * stage_per_lp must be < 2^31");
   cap_ = (uint32_t)cap;
-  tile_ = cfg.sort_tile ? cfg.sort_tile : kSortTile;
+  tile_ = cfg.sort_tile ? cfg.sort_tile : kMergeTile;
   GPQ_CHECK_ARG(valid_sort_tile(tile_), "GAQ: sort_tile must be 0, 1024, 2048 or 4096");
   v_.num_lps = cfg.num_lps;
   v_.enq_cap = (uint32_t)enq_cap;
@@ -107,6 +107,7 @@ gpq_status GaqQueue::init() {
   GPQ_HIP(hipMemsetAsync(v_.seg_m, 0, sizeof(uint32_t) * kStripeCounterWords, stream));
   GPQ_TRY(arena.alloc(&sort_[0], enq_cap));
   GPQ_TRY(arena.alloc(&sort_[1], enq_cap));
+  GPQ_TRY(arena.alloc(&order_, sort_order_words(enq_cap)));
   GPQ_TRY(arena.alloc(&v_.deq, cfg.num_lps));
   GPQ_TRY(arena.alloc(&v_.st, 1));
   GPQ_TRY(arena.alloc(&task_, 1));
@@ -134,10 +135,10 @@ gpq_status GaqQueue::pre() {
 }
 
 gpq_status GaqQueue::post() {
-  Event* sorted = nullptr;
+  Event* sorted = sort_[0];
   GPQ_TRY(gather_inserts(v_.seg_m, v_.seg_cap, v_.enq_cap, v_.enq_cap, seg_pre_, &v_.st->m, ws, stream));
-  GPQ_TRY(sort_records(v_.enq, sort_[0], sort_[1], &v_.st->m, v_.enq_cap, stream, &sorted, tile_,
-                       acct(kStatSorted), seg_pre_, v_.seg_cap));
+  GPQ_TRY(sort_records(v_.enq, sort_[0], sort_[1], order_, &v_.st->m, v_.enq_cap, stream, acct(kStatSorted), seg_pre_,
+                       v_.seg_cap));
   hipLaunchKernelGGL(gaq_plan_kernel, dim3(1), dim3(1), 0, stream, v_.st, task_, sorted, rest_, cap_, v_.enq_cap, ws);
   GPQ_HIP(hipGetLastError());
   GPQ_TRY(merge_tasks(task_, 1, (uint64_t)cap_, stream, tile_, acct(kStatMerged), splits_, split_stride_));

@@ -312,7 +312,7 @@ gpq_status HqQueue::init() {
   const uint64_t nodes = cfg.heap_nodes ? cfg.heap_nodes : (total + cfg.node_size - 1) / cfg.node_size + 1;
   GPQ_CHECK_ARG(nodes >= 1 && nodes < (1u << 20), "HQ: bad heap_nodes");
   r_ = cfg.node_size;
-  tile_ = cfg.sort_tile ? cfg.sort_tile : kSortTile;
+  tile_ = cfg.sort_tile ? cfg.sort_tile : kMergeTile;
   GPQ_CHECK_ARG(valid_sort_tile(tile_), "HQ: sort_tile must be 0, 1024, 2048 or 4096");
   nodes_ = (uint32_t)nodes;
   // every heap takes a whole step's inserts (the events of one step may all go to one heap)
@@ -343,6 +343,7 @@ gpq_status HqQueue::init() {
   tasks_n_ = 3 * (size_t)slots_ + 8;
   GPQ_TRY(arena.alloc(&sort_[0], (size_t)heaps_ * enq_cap));
   GPQ_TRY(arena.alloc(&sort_[1], (size_t)heaps_ * enq_cap));
+  GPQ_TRY(arena.alloc(&order_, (size_t)heaps_ * sort_order_words(enq_cap)));
   GPQ_TRY(arena.alloc(&merged_, (size_t)heaps_ * mcap_));
   GPQ_TRY(arena.alloc(&rest_, (size_t)heaps_ * mcap_));
   GPQ_TRY(arena.alloc(&carry_, (size_t)heaps_ * mcap_));
@@ -416,13 +417,13 @@ gpq_status HqQueue::step(bool select) {
 gpq_status HqQueue::merge_root(uint32_t h, hipStream_t s) {
   HqState* st = v_.st + h;
   MergeTask* t = tasks_ + (size_t)h * tasks_n_;
-  Event* sorted = nullptr;
+  Event* sorted = sort_[0] + (size_t)h * v_.enq_cap;
   uint32_t* pre = seg_pre_ + (size_t)h * (kInsertStripes + 2);
   GPQ_TRY(gather_inserts(v_.seg_m + (size_t)h * kStripeCounterWords, v_.seg_cap, v_.enq_cap, v_.enq_cap, pre, &st->m,
                          ws, s));
-  GPQ_TRY(sort_records(v_.enq + (size_t)h * v_.area, sort_[0] + (size_t)h * v_.enq_cap,
-                       sort_[1] + (size_t)h * v_.enq_cap, &st->m, v_.enq_cap, s, &sorted, tile_,
-                       acct(kStatSorted), pre, v_.seg_cap));
+  GPQ_TRY(sort_records(v_.enq + (size_t)h * v_.area, sorted, sort_[1] + (size_t)h * v_.enq_cap,
+                       order_ + (size_t)h * sort_order_words(v_.enq_cap), &st->m, v_.enq_cap, s, acct(kStatSorted), pre,
+                       v_.seg_cap));
   hipLaunchKernelGGL(hq_plan_merge_root, dim3(1), dim3(1), 0, s, st, counts_ + (size_t)h * nodes_,
                      nodes_buf_ + (size_t)h * nodes_ * r_, sorted, merged_ + (size_t)h * mcap_, v_.enq_cap, t);
   GPQ_TRY(merge_tasks(t, 1, mcap_, s, tile_, acct(kStatMerged), splits_of(t), split_stride_));

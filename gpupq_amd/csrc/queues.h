@@ -104,6 +104,7 @@ class GaqQueue final : public QueueBase {
   Event* fel_[2] = {nullptr, nullptr};
   Event* rest_ = nullptr;
   Event* sort_[2] = {nullptr, nullptr};
+  uint32_t* order_ = nullptr;   // sample order of the insert sort
   MergeTask* task_ = nullptr;
   uint32_t* first_ = nullptr;
   uint32_t* scratch_ = nullptr;
@@ -111,7 +112,7 @@ class GaqQueue final : public QueueBase {
   uint32_t split_stride_ = 0;
   uint32_t* seg_pre_ = nullptr; // segment offsets of the step's striped inserts
   uint32_t cap_ = 0;
-  uint32_t tile_ = kSortTile;   // records per sort / merge block
+  uint32_t tile_ = kMergeTile;  // records per merge block
 };
 
 class HqQueue final : public QueueBase {
@@ -144,6 +145,7 @@ class HqQueue final : public QueueBase {
   uint32_t* counts_ = nullptr;
   uint8_t* dirty_ = nullptr;
   Event* sort_[2] = {nullptr, nullptr};
+  uint32_t* order_ = nullptr;   // sample order of the insert sort
   Event* merged_ = nullptr;
   Event* rest_ = nullptr;
   Event* carry_ = nullptr;
@@ -157,7 +159,7 @@ class HqQueue final : public QueueBase {
   uint32_t split_stride_ = 0;
   uint32_t* seg_pre_ = nullptr; // per heap, segment offsets of the step's striped inserts
   uint64_t* sum_ = nullptr;
-  uint32_t tile_ = kSortTile;   // records per sort / merge block
+  uint32_t tile_ = kMergeTile;  // records per merge block
   // the split buffer of task slot t (tasks_ + t)
   uint32_t* splits_of(const MergeTask* t) const { return splits_ + (size_t)(t - tasks_) * split_stride_; }
 };

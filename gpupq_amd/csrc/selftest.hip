@@ -57,20 +57,19 @@ struct DevBuf {
 extern "C" gpq_status gpq_selftest_sort(const gpq_event* in, uint32_t n, gpq_event* out) {
   using gpq::Event;
   if (!in || !out || n == 0 || n >= (1u << 30)) { gpq::set_error("bad selftest_sort args"); return GPQ_ERR_INVALID; }
-  DevBuf a, b0, b1, dn;
+  DevBuf a, b0, b1, dn, ord;
   GPQ_HIP(hipMalloc(&a.p, sizeof(Event) * n));
   GPQ_HIP(hipMalloc(&b0.p, sizeof(Event) * n));
   GPQ_HIP(hipMalloc(&b1.p, sizeof(Event) * n));
   GPQ_HIP(hipMalloc(&dn.p, sizeof(uint32_t)));
   GPQ_HIP(hipMemcpy(a.p, in, sizeof(Event) * n, hipMemcpyHostToDevice));
   GPQ_HIP(hipMemcpy(dn.p, &n, sizeof(uint32_t), hipMemcpyHostToDevice));
-  // A capacity above n, as the queues pass it: the merge passes whose width already covers n
-  // are skipped or reduced to one copy, by the parity of their number.
+  // a capacity above n, as the queues pass it: the levels that n does not need do nothing
   const uint32_t cap = n <= (1u << 28) ? 6u * n : n;
-  Event* res = nullptr;
+  GPQ_HIP(hipMalloc(&ord.p, sizeof(uint32_t) * gpq::sort_order_words(cap)));
   GPQ_TRY(gpq::sort_records(static_cast<Event*>(a.p), static_cast<Event*>(b0.p), static_cast<Event*>(b1.p),
-                            static_cast<uint32_t*>(dn.p), cap, 0, &res));
-  GPQ_HIP(hipMemcpy(out, res, sizeof(Event) * n, hipMemcpyDeviceToHost));
+                            static_cast<uint32_t*>(ord.p), static_cast<uint32_t*>(dn.p), cap, 0));
+  GPQ_HIP(hipMemcpy(out, b0.p, sizeof(Event) * n, hipMemcpyDeviceToHost));
   return GPQ_OK;
 }
 

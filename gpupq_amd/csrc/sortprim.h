@@ -9,13 +9,10 @@
 
 namespace gpq {
 
-// Tiles of the sort and merge kernels: 1024, 2048 (the default) or 4096 records per block
-// (128, 256 or 512 threads x 8 records), chosen per queue (gpq_queue_config.sort_tile).
+// Tiles of the merge kernels: 1024, 2048 (the default) or 4096 records per block (128, 256 or 512
+// threads x 8 records), chosen per queue (gpq_queue_config.sort_tile).
 constexpr uint32_t kMergeTile = 2048;   // default outputs per merge block
-constexpr uint32_t kSortTile = 2048;    // default records per tile-sort block
 bool valid_sort_tile(uint32_t tile);
-// Merge passes of a sort of up to cap records with tiles of `tile` records.
-uint32_t sort_passes(uint32_t cap, uint32_t tile);
 
 // Stable merge of A = a1[0:n_a1) ++ a2[0:n_a2) (both parts sorted, a1 before a2) with
 // sorted B (ties take A first).  Output rank o goes to out[s][o - start_s], where segment
@@ -31,15 +28,18 @@ struct MergeTask {
   uint32_t end[3];
 };
 
-// Sorts *d_n (<= cap) records of `in` (not modified) into buf0/buf1; returns the buffer
-// holding the sorted run.  Passes: one tile sort, then ceil(log2(cap / tile)) merge passes.
+// Sorts *d_n (<= cap; cap records when d_n is null) records of `in` by (ts, src, seq) into buf0, with buf1 as the partner buffer
+// and `order` (sort_order_words(cap) words) for the sample order.  `in` is not modified unless it
+// is buf0 (sorting in place).  One tile sort, then two launches per level of up to 128-way merges;
+// the levels that *d_n records do not need do nothing.
 // `acct` (optional): a device counter that receives the records sorted (*d_n), for the
 // algorithmic-byte accounting of queues created with collect_stats.
 // `seg_pre` (optional): `in` is a striped insert area (core.cuh) with seg_cap-record stripes,
 // its segments' records laid out by gather_inserts (*d_n = their total).
-gpq_status sort_records(const Event* in, Event* buf0, Event* buf1, const uint32_t* d_n, uint32_t cap,
-                        hipStream_t stream, Event** sorted, uint32_t tile = kSortTile,
-                        unsigned long long* acct = nullptr, const uint32_t* seg_pre = nullptr, uint32_t seg_cap = 0);
+gpq_status sort_records(const Event* in, Event* buf0, Event* buf1, uint32_t* order, const uint32_t* d_n, uint32_t cap,
+                        hipStream_t stream, unsigned long long* acct = nullptr, const uint32_t* seg_pre = nullptr,
+                        uint32_t seg_cap = 0);
+size_t sort_order_words(uint64_t cap);
 
 // Records per stripe of an insert area for `enq_cap` inserts per step: twice an even share, at
 // least 1024 (a stripe that fills up spills into the shared segment of enq_cap records).

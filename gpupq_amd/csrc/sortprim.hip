@@ -1,13 +1,15 @@
-// sortprim.hip -- record sort (bitonic tile sort in LDS + merge-path merge passes),
+// sortprim.hip -- record sort (tile sort in LDS, then levels of up to 128-way merges),
 // multi-task merge-path merges, and the parallel one-safe-event-per-LP selection.
+#include <algorithm>
+
 #include "sortprim.h"
 
 namespace gpq {
 namespace {
 
-constexpr int kThreads = 256;                       // selection blocks; sort and merge blocks: kT of
-                                                    // 128, 256 or 512 threads (tiles of 8 kT records)
-constexpr int kPerThread = 8;                       // records per thread in the tile sort and merge
+constexpr int kThreads = 256;                       // selection blocks; merge blocks: kT of 128, 256 or
+                                                    // 512 threads (tiles of 8 kT records)
+constexpr int kPerThread = 8;                       // records per thread in the merge
 constexpr uint32_t kSelectTile = 1024;              // records per selection block (256 x 4)
 constexpr uint32_t kSplitLanes = 8;                 // lanes per tile boundary in the merge partition
 
@@ -164,118 +166,441 @@ __device__ __forceinline__ void merge_tile(const ASrc& A, uint32_t na, const Eve
   for (uint32_t x = threadIdx.x; x < len; x += kT) store_event(out.at(t0 + x), s[pad8(x)]);
 }
 
-__device__ __forceinline__ void compare_swap(Event& a, Event& b, bool up) {
-  if (up ? key_less(b, a) : key_less(a, b)) {
-    const Event t = a;
-    a = b;
-    b = t;
-  }
+// --- sort -------------------------------------------------------------------------
+//
+// A run of up to kRun records is sorted by one block (tile_sort_kernel); a level then merges up to
+// kFan sorted runs at once: every kSampleth record of a run is a sample (from an offset of the run's
+// own: the same quantiles sampled in every run would leave gaps without samples, and blocks with
+// three times the others' records), sample_rank_kernel ranks
+// all samples of the runs against each other, and bucket_merge_kernel takes kBucketSamples
+// consecutive samples' worth of records per block -- its share of every run, found by searching
+// each run for two samples -- and merges the shares in LDS.  Between two samples of a run lie fewer
+// than kSample records, so a block's shares hold at most (kBucketSamples + kFan) * kSample =
+// kBucketCap records whatever the data.  One level sorts 2^17 records, two 2^24.
+//
+// What bounds it at the global queues' sizes (10^4 to 10^6 records) is the chain of launches and
+// of dependent LDS and L2 accesses, not bytes: 100,003 records took 59 us in a bitonic tile sort
+// of 66 stages and 10 us in each of six pairwise merge passes, 120 us in all; the three launches
+// here take 16, 9 and 28 us, 52 us in all.
+// Tiles and buckets are small (1024 records, two or one per thread) so that they spread over the
+// CUs: with tiles and buckets of 2048 records and eight or four per thread the launches took 38
+// and 39 us, most of it LDS reads and index arithmetic of one wave per SIMD.
+//
+// Order: (ts, src, seq), then dst, so that records compare equal only if they are identical.
+constexpr uint32_t kRun = 1024;
+constexpr uint32_t kTilePer = 2;
+constexpr int kTileThreads = kRun / kTilePer;
+constexpr uint32_t kFan = 128;
+constexpr uint32_t kSample = 32;
+constexpr uint32_t kBucketSamples = 24;
+constexpr uint32_t kBucketCap = (kBucketSamples + kFan) * kSample;
+constexpr int kBucketThreads = 1024;
+constexpr uint32_t kBucketPer = (kBucketCap + kBucketThreads - 1) / kBucketThreads;
+constexpr uint32_t kFindLanes = kBucketThreads / (2 * kFan);   // lanes that search one run for one sample
+static_assert(kRun % kSample == 0, "whole runs have the same number of samples");
+
+// Samples of run r (in its group): records off, off + kSample, ... with off = sample_offset(r).
+__device__ __forceinline__ uint32_t sample_offset(uint32_t r) { return (r * 21u + 5u) % kSample; }
+__device__ __forceinline__ uint32_t samples_of(uint32_t r, uint32_t len) {
+  const uint32_t off = sample_offset(r);
+  return len > off ? (len - off - 1u) / kSample + 1u : 0u;
+}
+// Record index of sample s of a level's input: the samples of whole runs are numbered run by run.
+__device__ __forceinline__ uint32_t sample_record(uint32_t s, uint32_t w) {
+  const uint32_t run = s / (w / kSample);
+  return run * w + (s % (w / kSample)) * kSample + sample_offset(run % kFan);
 }
 
-// Bitonic sort of one kSortTile-record tile.  Thread t holds records 8t .. 8t+7 in registers,
-// so every stage with partner distance j < 8 (30 of the 66) runs in registers with no barrier;
-// the stages with j >= 8 run in LDS, each thread exchanging 4 of the tile's 1024 pairs.  The
-// LDS tile is padded one record per 8 (pad8) so that the 8-record runs of neighbouring threads
-// start in different banks.
+// A record as two words whose pair order is the sort order.
+struct Rec {
+  uint64_t hi, lo;
+};
+__device__ __forceinline__ Rec load_rec(const Event* p) {
+  const Event e = load_event(p);
+  return Rec{((uint64_t)e.ts << 32) | e.src, ((uint64_t)e.seq << 32) | e.dst};
+}
+__device__ __forceinline__ bool rec_less(uint64_t ahi, uint64_t alo, uint64_t bhi, uint64_t blo) {
+  return ahi != bhi ? ahi < bhi : alo < blo;
+}
+
+// Records in LDS by word: searches read timestamps alone (4-byte reads, 32-bit comparisons), and
+// the other words only where timestamps tie.  One pad word per 32: the probes of a binary search
+// lie powers of two apart, which would put them all in one bank.
+template <uint32_t N>
+struct LdsRecs {
+  static constexpr uint32_t kSize = N + N / 32u;
+  uint64_t lo[kSize];
+  uint32_t ts[kSize], src[kSize];
+  static __device__ __forceinline__ uint32_t at(uint32_t i) { return i + (i >> 5); }
+  __device__ __forceinline__ uint32_t time(uint32_t i) const { return ts[at(i)]; }
+  __device__ __forceinline__ void put(uint32_t i, uint64_t h, uint64_t l) {
+    const uint32_t a = at(i);
+    ts[a] = (uint32_t)(h >> 32);
+    src[a] = (uint32_t)h;
+    lo[a] = l;
+  }
+  __device__ __forceinline__ Event get(uint32_t i) const {
+    const uint32_t a = at(i);
+    const uint64_t l = lo[a];
+    return Event{ts[a], (uint32_t)l, src[a], (uint32_t)(l >> 32)};
+  }
+  // record i comes before (h, l), or equals it with `equal`
+  __device__ __forceinline__ bool before(uint32_t i, uint64_t h, uint64_t l, bool equal) const {
+    const uint32_t a = at(i);
+    const uint64_t oh = ((uint64_t)ts[a] << 32) | src[a], ol = lo[a];
+    return oh != h ? oh < h : (equal ? ol <= l : ol < l);
+  }
+};
+
+// Blocks of bucket_merge_kernel per group of kFan runs of w records.
+__host__ __device__ __forceinline__ uint64_t buckets_per_group(uint64_t w) {
+  return (w * kFan / kSample + kBucketSamples - 1) / kBucketSamples;
+}
+
+// Levels that n records take.
+__host__ __device__ __forceinline__ uint32_t sort_levels(uint64_t n) {
+  uint32_t k = 0;
+  for (uint64_t w = kRun; w < n; w *= kFan) ++k;
+  return k;
+}
+
+// Sorted runs of kRun records; written to buf1 when the levels that follow are odd in number, to
+// buf0 otherwise, so that the last level leaves the result in buf0.
 // seg_pre (optional): `in` is a striped insert area (core.cuh) whose segment k holds records
-// [seg_pre[k], seg_pre[k + 1]) of the run (k < kInsertStripes: at k * seg_cap; the spill
+// [seg_pre[k], seg_pre[k + 1]) of the input (k < kInsertStripes: at k * seg_cap; the spill
 // segment k = kInsertStripes after the stripes).
-template <int kT>
-__global__ __launch_bounds__(kT) void tile_sort_kernel(const Event* in, Event* out, const uint32_t* d_n,
-                                                       const uint32_t* seg_pre, uint32_t seg_cap) {
-  constexpr uint32_t kTile = kT * kPerThread;
-  __shared__ Event s[kTile + kTile / 8];
+__global__ __launch_bounds__(kTileThreads) void tile_sort_kernel(const Event* in, Event* buf0, Event* buf1,
+                                                                 const uint32_t* d_n, uint32_t cap,
+                                                                 const uint32_t* seg_pre, uint32_t seg_cap) {
+  __shared__ LdsRecs<kRun> s;
   __shared__ uint32_t s_pre[kInsertStripes + 2];
-  const uint32_t n = *d_n;
-  const uint32_t base = blockIdx.x * kTile;
+  const uint32_t n = d_n ? *d_n : cap;
+  const uint32_t base = blockIdx.x * kRun;
   if (base >= n) return;
   if (seg_pre) {
-    for (uint32_t k = threadIdx.x; k < kInsertStripes + 2u; k += kT) s_pre[k] = seg_pre[k];
+    for (uint32_t k = threadIdx.x; k < kInsertStripes + 2u; k += kTileThreads) s_pre[k] = seg_pre[k];
     __syncthreads();
   }
-  for (uint32_t i = threadIdx.x; i < kTile; i += kT) {
-    const uint32_t g = base + i;
-    if (g >= n) {
-      s[pad8(i)] = sentinel();
-    } else if (!seg_pre) {
-      s[pad8(i)] = load_event(in + g);
-    } else {
-      uint32_t lo = 0, hi = kInsertStripes;          // the last segment k with s_pre[k] <= g
-      while (lo < hi) {
-        const uint32_t mid = (lo + hi + 1u) >> 1;
-        if (s_pre[mid] <= g) lo = mid; else hi = mid - 1u;
+  const uint32_t have = n - base < kRun ? n - base : kRun;
+  uint64_t hi[kTilePer], lo[kTilePer];
+  uint32_t pos[kTilePer];
+#pragma unroll
+  for (uint32_t q = 0; q < kTilePer; ++q) {
+    pos[q] = threadIdx.x * kTilePer + q;
+    hi[q] = lo[q] = ~0ull;                            // past the end: never placed or looked at
+    if (pos[q] < have) {
+      const uint32_t g = base + pos[q];
+      const Event* p = in + g;
+      if (seg_pre) {
+        uint32_t a = 0, b = kInsertStripes;           // the last segment k with s_pre[k] <= g
+        while (a < b) {
+          const uint32_t mid = (a + b + 1u) >> 1;
+          if (s_pre[mid] <= g) a = mid; else b = mid - 1u;
+        }
+        p = in + (size_t)a * seg_cap + (g - s_pre[a]);
       }
-      s[pad8(i)] = load_event(in + (size_t)lo * seg_cap + (g - s_pre[lo]));
+      const Rec r = load_rec(p);
+      hi[q] = r.hi;
+      lo[q] = r.lo;
     }
   }
+  static_assert(kTilePer == 2, "one exchange sorts a thread's records");
+  if (rec_less(hi[1], lo[1], hi[0], lo[0])) {
+    const uint64_t h = hi[0], l = lo[0];
+    hi[0] = hi[1]; lo[0] = lo[1];
+    hi[1] = h; lo[1] = l;
+  }
+#pragma unroll
+  for (uint32_t q = 0; q < kTilePer; ++q)
+    if (pos[q] < have) s.put(pos[q], hi[q], lo[q]);
   __syncthreads();
-  const uint32_t t0 = threadIdx.x * 8u;
-  Event r[8];
+  // runs of w pair up: a record's place is its place in its run plus its rank in the other
+  for (uint32_t w = kTilePer; w < kRun; w *= 2) {
+    uint32_t cnt[kTilePer];
+    const uint32_t own = threadIdx.x * kTilePer & ~(w - 1u);   // the thread's records lie in one run
+    const uint32_t other = own ^ w;
+    const uint32_t len = other < have ? (have - other < w ? have - other : w) : 0u;
+    const bool right = (own & w) != 0;                // ties: the left run's records first
 #pragma unroll
-  for (int q = 0; q < 8; ++q) r[q] = s[pad8(t0 + q)];
+    for (uint32_t q = 0; q < kTilePer; ++q) cnt[q] = 0;
+    for (uint32_t bit = w; bit; bit >>= 1) {
+      uint32_t ot[kTilePer];
+      bool tie = false;
 #pragma unroll
-  for (uint32_t k = 2; k <= 8; k <<= 1)
+      for (uint32_t q = 0; q < kTilePer; ++q) {       // a probe past the run reads slot 0 and is not used
+        const uint32_t c = cnt[q] + bit;
+        ot[q] = s.time(c <= len ? other + c - 1u : 0u);
+      }
 #pragma unroll
-    for (uint32_t j = k >> 1; j > 0; j >>= 1)
+      for (uint32_t q = 0; q < kTilePer; ++q) tie |= cnt[q] + bit <= len && ot[q] == (uint32_t)(hi[q] >> 32);
+      if (__any(tie)) {                               // a branch of the whole wave, rarely taken
 #pragma unroll
-      for (uint32_t a = 0; a < 8; ++a)
-        if ((a & j) == 0) compare_swap(r[a], r[a | j], ((t0 + a) & k) == 0);
-  for (uint32_t k = 16; k <= kTile; k <<= 1) {
+        for (uint32_t q = 0; q < kTilePer; ++q) {
+          const uint32_t c = cnt[q] + bit;
+          if (c <= len && s.before(other + c - 1u, hi[q], lo[q], right)) cnt[q] = c;
+        }
+      } else {
 #pragma unroll
-    for (int q = 0; q < 8; ++q) s[pad8(t0 + q)] = r[q];
+        for (uint32_t q = 0; q < kTilePer; ++q) {
+          const uint32_t c = cnt[q] + bit;
+          if (c <= len && ot[q] < (uint32_t)(hi[q] >> 32)) cnt[q] = c;
+        }
+      }
+    }
     __syncthreads();
-    for (uint32_t j = k >> 1; j >= 8; j >>= 1) {
+    const uint32_t pair = own & ~(2u * w - 1u);
 #pragma unroll
-      for (uint32_t q = 0; q < kTile / 2 / kT; ++q) {
-        const uint32_t pr = threadIdx.x + q * kT;
-        const uint32_t i = ((pr & ~(j - 1u)) << 1) | (pr & (j - 1u));   // pair (i, i + j), bit j of i clear
-        Event x = s[pad8(i)], y = s[pad8(i | j)];
-        compare_swap(x, y, (i & k) == 0);
-        s[pad8(i)] = x;
-        s[pad8(i | j)] = y;
+    for (uint32_t q = 0; q < kTilePer; ++q) {
+      if (pos[q] < have) {
+        pos[q] = pair + (pos[q] - own) + cnt[q];
+        s.put(pos[q], hi[q], lo[q]);
       }
-      __syncthreads();
     }
-#pragma unroll
-    for (int q = 0; q < 8; ++q) r[q] = s[pad8(t0 + q)];
-    const bool up = (t0 & k) == 0;   // bit k >= 16 of i is that of t0 for all eight
-#pragma unroll
-    for (uint32_t j = 4; j > 0; j >>= 1)
-#pragma unroll
-      for (uint32_t a = 0; a < 8; ++a)
-        if ((a & j) == 0) compare_swap(r[a], r[a | j], up);
+    __syncthreads();
   }
-  __syncthreads();   // every thread's last LDS stage reads are done
-#pragma unroll
-  for (int q = 0; q < 8; ++q) s[pad8(t0 + q)] = r[q];
-  __syncthreads();
-  for (uint32_t i = threadIdx.x; i < kTile; i += kT)
-    if (base + i < n) store_event(out + base + i, s[pad8(i)]);
+  Event* out = (sort_levels(n) & 1u) ? buf1 : buf0;
+  for (uint32_t i = threadIdx.x; i < kRun; i += kTileThreads)
+    if (base + i < n) store_event(out + base + i, s.get(i));
 }
 
-// Merges adjacent sorted runs of width w (2w is a multiple of kMergeTile); pass `pass` of
-// `passes`.  Once w >= n every remaining pass would only copy the one run, so those passes
-// do nothing when their number is even (the run already sits in the final buffer) and the
-// first of them copies when it is odd.
-template <int kT>
-__global__ __launch_bounds__(kT) void merge_pass_kernel(const Event* in, Event* out, const uint32_t* d_n,
-                                                        uint32_t w, uint32_t pass, uint32_t passes) {
-  constexpr uint32_t kTile = kT * kPerThread;
-  const uint32_t n = *d_n;
-  const uint32_t t0 = blockIdx.x * kTile;
-  if (t0 >= n) return;
-  if (w >= n) {
-    uint32_t first = 0;   // the first pass whose width covers n
-    while (((uint64_t)kTile << first) < n) ++first;
-    if (((passes - first) & 1u) == 0 || pass != first) return;
+// Number of the cnt elements a[0], a[stride], ... that come before (hi, lo) -- or equal it, with
+// `equal` -- in a sorted sequence.
+__device__ __forceinline__ uint32_t count_before(const Event* a, uint32_t cnt, uint32_t stride, uint64_t hi, uint64_t lo,
+                                                 bool equal) {
+  uint32_t c = 0;
+  for (uint32_t bit = cnt ? 1u << (31 - __builtin_clz(cnt)) : 0u; bit; bit >>= 1) {
+    const uint32_t t = c + bit;
+    if (t > cnt) continue;
+    const Rec r = load_rec(a + (size_t)(t - 1u) * stride);
+    if (rec_less(r.hi, r.lo, hi, lo) || (equal && r.hi == hi && r.lo == lo)) c = t;
   }
-  const uint32_t base = t0 / (2u * w) * (2u * w);
-  const uint32_t na = n - base < w ? n - base : w;
-  const uint32_t rest = n - base - na;
-  const uint32_t nb = rest < w ? rest : w;
-  const ASrc A{in + base, in + base, na};
-  OutMap om{{out + base, out + base, out + base}, {0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu}};
-  merge_tile<kT>(A, na, in + base + na, nb, t0 - base, om);
+  return c;
+}
+
+// The same count for stride 1 by a group of kFindLanes lanes (all of them call with the same
+// arguments): each round probes kFindLanes points that cut the remaining range evenly.
+__device__ __forceinline__ uint32_t count_before_lanes(const Event* a, uint32_t cnt, uint64_t hi, uint64_t lo, bool equal) {
+  const uint32_t lane = (uint32_t)lane_id(), k = lane % kFindLanes, first = lane - k;
+  uint32_t from = 0, to = cnt;                                     // the count lies in [from, to]
+  while (__ballot(from < to)) {
+    const uint32_t len = to - from;
+    bool before = false;
+    if (len) {
+      const Rec r = load_rec(a + from + len * (k + 1u) / (kFindLanes + 1u));
+      before = rec_less(r.hi, r.lo, hi, lo) || (equal && r.hi == hi && r.lo == lo);
+    }
+    const uint32_t m = (uint32_t)__popcll((__ballot(before) >> first) & ((1ull << kFindLanes) - 1ull));
+    if (len) {
+      const uint32_t f = from;
+      if (m < kFindLanes) to = f + len * (m + 1u) / (kFindLanes + 1u);
+      if (m) from = f + len * m / (kFindLanes + 1u) + 1u;
+    }
+  }
+  return from;
+}
+
+// Source and destination of level `level` (1, 2, ...) for n records; false when n needs fewer.
+__device__ __forceinline__ bool level_buffers(uint32_t n, uint32_t level, Event* buf0, Event* buf1, const Event** src,
+                                              Event** dst) {
+  const uint32_t k = sort_levels(n);
+  if (level > k) return false;
+  const bool odd = ((k - level) & 1u) != 0;
+  *dst = odd ? buf1 : buf0;
+  *src = odd ? buf0 : buf1;
+  return true;
+}
+
+// Level input: runs of w records, groups of kFan runs.  Every sample is ranked
+// among the samples of its group, a lane per run of the group (the lanes per sample rounded up to
+// a power of two, at most a wave's, which then takes two runs each), and order[group's first
+// sample + rank] = the sample's index.
+__global__ __launch_bounds__(256) void sample_rank_kernel(Event* buf0, Event* buf1, const uint32_t* d_n, uint32_t cap,
+                                                          uint32_t level, uint32_t w, uint32_t* order) {
+  const uint32_t n = d_n ? *d_n : cap;
+  const Event* in;
+  Event* out;
+  if (!level_buffers(n, level, buf0, buf1, &in, &out)) return;
+  const uint32_t ns = (n + kSample - 1u) / kSample;
+  const uint64_t group = (uint64_t)w * kFan;                       // records per group
+  uint32_t lanes = 1;                                              // lanes per sample
+  while (lanes < (uint32_t)kWave && (uint64_t)lanes * w < n) lanes *= 2;
+  const uint32_t t = blockIdx.x * 256u + threadIdx.x;
+  const uint64_t s = (uint64_t)t / lanes;
+  const uint32_t k = t % lanes;
+  if (((uint64_t)t & ~63ull) / lanes >= ns) return;                // the whole wave is past the samples
+  uint32_t rank = 0;
+  const uint32_t i = sample_record((uint32_t)s, w);
+  const uint32_t g0 = (uint32_t)(i / group * group);               // first record of its group
+  const bool is = s < ns && i < n;                                 // the last run may be short of its last sample
+  if (is) {
+    const uint32_t own = (i - g0) / w;
+    const Rec me = load_rec(in + i);
+    for (uint32_t r = k; r < kFan; r += lanes) {
+      const uint64_t r0 = (uint64_t)g0 + (uint64_t)r * w;          // first record of run r
+      if (r0 >= n) break;
+      const uint32_t len = (uint32_t)(n - r0 < w ? n - r0 : w);
+      rank += r == own ? (uint32_t)(i - r0) / kSample
+                       : count_before(in + r0 + sample_offset(r), samples_of(r, len), kSample, me.hi, me.lo, r < own);
+    }
+  }
+  for (uint32_t off = lanes / 2u; off > 0; off >>= 1) rank += (uint32_t)__shfl_xor((int)rank, (int)off, kWave);
+  if (is && k == 0) order[g0 / kSample + rank] = (uint32_t)s;
+}
+
+// A block merges, for kBucketSamples samples of its group from rank b0 on (in sample order), the
+// records from the first of them up to the first of the next block (the group's first block:
+// from its first record; the last: to its end).
+__global__ __launch_bounds__(kBucketThreads) void bucket_merge_kernel(Event* buf0, Event* buf1, const uint32_t* d_n,
+                                                                      uint32_t cap, uint32_t level, uint32_t w,
+                                                                      const uint32_t* order) {
+  __shared__ LdsRecs<kBucketCap> s;
+  __shared__ uint32_t s_from[kFan], s_off[kFan + 1];
+  const uint32_t n = d_n ? *d_n : cap;
+  const Event* in;
+  Event* out;
+  if (!level_buffers(n, level, buf0, buf1, &in, &out)) return;
+  const uint64_t group = (uint64_t)w * kFan;
+  const uint64_t per = buckets_per_group(w);
+  const uint64_t start = blockIdx.x / per * group;                 // first record of the block's group
+  if (start >= n) return;
+  const uint32_t g0 = (uint32_t)start;
+  const uint32_t glen = (uint32_t)(n - g0 < group ? n - g0 : group);
+  const uint32_t runs = (glen + w - 1u) / w;
+  const uint32_t last = (runs - 1u) * w;                           // the group's last run may be short
+  const uint32_t gs = last / kSample + samples_of(runs - 1u, glen - last);   // samples of the group
+  const uint32_t b0 = (uint32_t)(blockIdx.x % per) * kBucketSamples;
+  if (b0 && b0 >= gs) return;
+  // kFindLanes lanes each: the block's first record in run r, and the record past its last
+  {
+    const uint32_t job = threadIdx.x / kFindLanes, r = job >> 1, at = b0 + (job & 1u) * kBucketSamples;
+    const uint32_t r0 = g0 + r * w;
+    const uint32_t len = r < runs ? (n - r0 < w ? n - r0 : w) : 0u;
+    uint32_t c = at ? len : 0u, find = 0;
+    Rec me{0, 0};
+    uint32_t own = 0;
+    if (at && at < gs) {
+      const uint32_t i = sample_record(order[g0 / kSample + at], w);   // the splitting record
+      own = (i - g0) / w;
+      if (r == own) {
+        c = i - r0;
+      } else {
+        me = load_rec(in + i);
+        find = len;
+      }
+    }
+    const uint32_t f = count_before_lanes(in + r0, find, me.hi, me.lo, r < own);
+    if (find) c = f;
+    const uint32_t end = (uint32_t)__shfl_xor((int)c, (int)kFindLanes, kWave);
+    if (threadIdx.x % (2u * kFindLanes) == 0) {
+      s_from[r] = c;
+      s_off[r + 1] = end - c;
+    }
+  }
+  __syncthreads();
+  // the run shares one after the other; the records of the group before the block's
+  __shared__ uint32_t s_before;
+  if (threadIdx.x < (uint32_t)kWave) {
+    static_assert(kFan == 2 * kWave, "two runs per lane");
+    const uint32_t r = 2u * threadIdx.x;
+    const uint32_t l0 = s_off[r + 1], l1 = s_off[r + 2];
+    uint32_t x = l0 + l1;
+#pragma unroll
+    for (int off = 1; off < kWave; off <<= 1) {
+      const uint32_t y = (uint32_t)__shfl_up((int)x, off, kWave);
+      if ((int)threadIdx.x >= off) x += y;
+    }
+    s_off[r + 1] = x - l1;
+    s_off[r + 2] = x;
+    const uint32_t f = wave_sum_u32(s_from[r] + s_from[r + 1]);
+    if (threadIdx.x == 0) {
+      s_off[0] = 0;
+      s_before = f;
+    }
+  }
+  __syncthreads();
+  const uint32_t total = s_off[kFan];
+  // records per thread, nearly always 1 (a uniform value, so that the loops over them branch as a wave)
+  const uint32_t slots = __builtin_amdgcn_readfirstlane((total + kBucketThreads - 1u) / kBucketThreads);
+  uint64_t hi[kBucketPer], lo[kBucketPer];
+  uint32_t pos[kBucketPer], run[kBucketPer];
+#pragma unroll
+  for (uint32_t q = 0; q < kBucketPer; ++q) {
+    if (q >= slots) break;
+    const uint32_t i = threadIdx.x + q * kBucketThreads;
+    pos[q] = i;
+    run[q] = 0;
+    hi[q] = lo[q] = ~0ull;
+    if (i < total) {
+      uint32_t a = 0, b = kFan - 1u;                               // the run r with s_off[r] <= i < s_off[r + 1]
+      while (a < b) {
+        const uint32_t mid = (a + b) >> 1;
+        if (s_off[mid + 1] > i) b = mid; else a = mid + 1u;
+      }
+      run[q] = a;
+      const Rec r = load_rec(in + g0 + (size_t)a * w + s_from[a] + (i - s_off[a]));
+      hi[q] = r.hi;
+      lo[q] = r.lo;
+      s.put(i, r.hi, r.lo);
+    }
+  }
+  __syncthreads();
+  for (uint32_t m = 0; (1u << m) < runs; ++m) {                    // 2^m runs' shares are merged so far
+    uint32_t cnt[kBucketPer], from[kBucketPer], len[kBucketPer], top = 0;
+    bool right[kBucketPer];
+#pragma unroll
+    for (uint32_t q = 0; q < kBucketPer; ++q) {
+      if (q >= slots) break;
+      const uint32_t g = run[q] >> m, a = (g ^ 1u) << m, b = a + (1u << m);   // kFan is a power of two
+      from[q] = s_off[a];
+      len[q] = pos[q] < total ? s_off[b] - s_off[a] : 0u;
+      right[q] = (g & 1u) != 0;
+      cnt[q] = 0;
+      top = len[q] > top ? len[q] : top;
+    }
+    for (uint32_t bit = top ? 1u << (31 - __builtin_clz(top)) : 0u; bit; bit >>= 1) {
+      uint32_t ot[kBucketPer];
+      bool tie = false;
+#pragma unroll
+      for (uint32_t q = 0; q < kBucketPer; ++q) {      // a probe past the share reads slot 0 and is not used
+        if (q >= slots) break;
+        const uint32_t c = cnt[q] + bit;
+        ot[q] = s.time(c <= len[q] ? from[q] + c - 1u : 0u);
+      }
+#pragma unroll
+      for (uint32_t q = 0; q < kBucketPer; ++q) {
+        if (q >= slots) break;
+        tie |= cnt[q] + bit <= len[q] && ot[q] == (uint32_t)(hi[q] >> 32);
+      }
+      if (__any(tie)) {                                // a branch of the whole wave, rarely taken
+#pragma unroll
+        for (uint32_t q = 0; q < kBucketPer; ++q) {
+          if (q >= slots) break;
+          const uint32_t c = cnt[q] + bit;
+          if (c <= len[q] && s.before(from[q] + c - 1u, hi[q], lo[q], right[q])) cnt[q] = c;
+        }
+      } else {
+#pragma unroll
+        for (uint32_t q = 0; q < kBucketPer; ++q) {
+          if (q >= slots) break;
+          const uint32_t c = cnt[q] + bit;
+          if (c <= len[q] && ot[q] < (uint32_t)(hi[q] >> 32)) cnt[q] = c;
+        }
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (uint32_t q = 0; q < kBucketPer; ++q) {
+      if (q >= slots) break;
+      if (pos[q] < total) {
+        // the left share's records move by those of the right one before them, and vice versa
+        pos[q] = right[q] ? pos[q] - len[q] + cnt[q] : pos[q] + cnt[q];
+        s.put(pos[q], hi[q], lo[q]);
+      }
+    }
+    __syncthreads();
+  }
+  Event* to = out + g0 + s_before;
+  for (uint32_t i = threadIdx.x; i < total; i += kBucketThreads) store_event(to + i, s.get(i));
 }
 
 // splits (optional): task y's splits at splits[y * stride + x], for tile x's first output rank
@@ -537,53 +862,28 @@ __global__ __launch_bounds__(256) void acct_tasks_kernel(const MergeTask* tasks,
 
 }  // namespace
 
-namespace {
-template <int kT>
-gpq_status sort_records_t(const Event* in, Event* buf0, Event* buf1, const uint32_t* d_n, uint32_t cap,
-                          hipStream_t stream, Event** sorted, const uint32_t* seg_pre, uint32_t seg_cap) {
-  constexpr uint32_t kTile = kT * kPerThread;
-  hipLaunchKernelGGL(tile_sort_kernel<kT>, dim3(grid_of(cap, kTile)), dim3(kT), 0, stream, in, buf0, d_n, seg_pre,
-                     seg_cap);
-  GPQ_HIP(hipGetLastError());
-  Event* cur = buf0;
-  Event* other = buf1;
-  uint32_t passes = 0;
-  for (uint64_t w = kTile; w < cap; w *= 2) ++passes;
-  uint32_t pass = 0;
-  for (uint64_t w = kTile; w < cap; w *= 2, ++pass) {
-    hipLaunchKernelGGL(merge_pass_kernel<kT>, dim3(grid_of(cap, kTile)), dim3(kT), 0, stream, cur, other, d_n,
-                       (uint32_t)w, pass, passes);
-    GPQ_HIP(hipGetLastError());
-    Event* t = cur;
-    cur = other;
-    other = t;
-  }
-  *sorted = cur;
-  return GPQ_OK;
-}
-}  // namespace
-
 bool valid_sort_tile(uint32_t tile) { return tile == 1024 || tile == 2048 || tile == 4096; }
 
-uint32_t sort_passes(uint32_t cap, uint32_t tile) {
-  uint32_t passes = 0;
-  for (uint64_t w = tile; w < cap; w *= 2) ++passes;
-  return passes;
-}
+size_t sort_order_words(uint64_t cap) { return (size_t)((cap + kSample - 1) / kSample) + 1; }
 
-gpq_status sort_records(const Event* in, Event* buf0, Event* buf1, const uint32_t* d_n, uint32_t cap,
-                        hipStream_t stream, Event** sorted, uint32_t tile, unsigned long long* acct,
-                        const uint32_t* seg_pre, uint32_t seg_cap) {
-  gpq_status s;
-  switch (tile) {
-    case 1024: s = sort_records_t<128>(in, buf0, buf1, d_n, cap, stream, sorted, seg_pre, seg_cap); break;
-    case 2048: s = sort_records_t<256>(in, buf0, buf1, d_n, cap, stream, sorted, seg_pre, seg_cap); break;
-    case 4096: s = sort_records_t<512>(in, buf0, buf1, d_n, cap, stream, sorted, seg_pre, seg_cap); break;
-    default:
-      set_error("sort tile must be 1024, 2048 or 4096 records");
-      return GPQ_ERR_INVALID;
+gpq_status sort_records(const Event* in, Event* buf0, Event* buf1, uint32_t* order, const uint32_t* d_n, uint32_t cap,
+                        hipStream_t stream, unsigned long long* acct, const uint32_t* seg_pre, uint32_t seg_cap) {
+  hipLaunchKernelGGL(tile_sort_kernel, dim3(grid_of(cap, kRun)), dim3(kTileThreads), 0, stream, in, buf0, buf1,
+                     d_n, cap, seg_pre, seg_cap);
+  uint64_t w = kRun;
+  for (uint32_t level = 1; level <= sort_levels(cap); ++level, w *= kFan) {
+    const uint64_t runs = std::min<uint64_t>((cap + w - 1) / w, kWave);
+    const uint64_t lanes = 1ull << log2u(runs);
+    hipLaunchKernelGGL(sample_rank_kernel, dim3(grid_of(((uint64_t)cap + kSample - 1) / kSample * lanes, 256)), dim3(256),
+                       0, stream, buf0, buf1, d_n, cap, level, (uint32_t)w, order);
+    // whole groups take buckets_per_group blocks each, the last one as many as its records need
+    const uint64_t groups = cap / (w * kFan), rest = cap % (w * kFan);
+    const uint64_t blocks = groups * buckets_per_group(w) + grid_of(rest, kSample * kBucketSamples);
+    hipLaunchKernelGGL(bucket_merge_kernel, dim3((uint32_t)blocks), dim3(kBucketThreads), 0, stream,
+                       buf0, buf1, d_n, cap, level, (uint32_t)w, order);
   }
-  if (s != GPQ_OK || !acct) return s;
+  GPQ_HIP(hipGetLastError());
+  if (!acct) return GPQ_OK;
   hipLaunchKernelGGL(acct_count_kernel, dim3(1), dim3(64), 0, stream, d_n, cap, acct);
   GPQ_HIP(hipGetLastError());
   return GPQ_OK;

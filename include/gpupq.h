@@ -93,7 +93,7 @@ typedef struct {
                                 the logs of the window it commits.  Events beyond the calendar wait in
                                 two lists, and events at or past the horizon in a parked list, of
                                 num_lps * far_per_lp records each.  Same committed trace. */
-  uint32_t sort_tile;         /* GAQ / HQ: records per block of the record sort and merge kernels:
+  uint32_t sort_tile;         /* GAQ / HQ: records per block of the merge kernels:
                                 1024, 2048 or 4096 (0 = 2048); gpq_queue_autotune_sort picks one */
 } gpq_queue_config;
 
@@ -238,8 +238,7 @@ typedef struct {
 
 /* Sort-tile autotuner for the global queues (no reference counterpart; the reference's
  * moderngpu mergesort fixes its tile at compile time, lib/moderngpu/src/moderngpu/
- * kernel_mergesort.hxx:27-148): times the tiles 2048, 1024 and 4096 of the record sort and
- * merge kernels on the model's own workload cut to end time sample_end_time (0 = 2, at most
+ * kernel_mergesort.hxx:27-148): times the tiles 2048, 1024 and 4096 of the merge kernels on the model's own workload cut to end time sample_end_time (0 = 2, at most
  * model->end_time) through queue->kind (GPQ_GAQ or GPQ_HQ), each in a fresh queue driven by
  * GPQ_DRIVE_GRAPH, checks that every tile commits the same trace, and writes the fastest (a later
  * tile must beat the pick so far by more than 2%) into queue->sort_tile.  results (may be NULL)
@@ -507,7 +506,7 @@ gpq_status gpq_selftest_select(const gpq_event* sorted, uint32_t n, uint32_t num
  * HIP graph capture, tight serving loops, harnesses that forbid hipMalloc): sorts n device
  * records d_in by (ts, src, seq) into d_out (device; d_out == d_in sorts in place) on `stream`
  * (a hipStream_t; NULL = the default stream), with the kernels of gpq_selftest_sort.  Its
- * partner buffer and count word live in a library-owned device array of 16 MiB + 256 B that
+ * partner buffer and sample order live in a library-owned device array of 16.125 MiB + 256 B that
  * every GPU it runs on holds until the process ends; it calls no hipMalloc or hipFree.
  * n <= 2^20 (GPQ_ERR_CAPACITY above).  Calls that overlap on one GPU share that array and race:
  * the caller serialises them.  Returns once the work is queued (asynchronous). */
