@@ -19,7 +19,7 @@ from . import _lib
 from ._lib import DesReport, Event, GpqError, PholdConfig, QueueConfig, check
 
 __all__ = ["Queue", "Phold", "PholdBatch", "Astar", "AstarBatch", "autotune_batch", "query_synthetic", "serve_trace", "serve_run", "des_init",
-           "des_run", "des_finish",
+           "des_run", "des_finish", "release_kept_memory",
            "GpqError", "lib", "event_dtype"]
 
 lib = _lib.load()
@@ -34,6 +34,11 @@ def f32_bits(x):
 
 def bits_f32(u):
     return float(np.uint32(u).view(np.float32))
+
+
+def release_kept_memory():
+    """Frees the device and pinned memory kept from destroyed handles (gpq_release_kept_memory)."""
+    check(lib.gpq_release_kept_memory(), "release_kept_memory")
 
 
 def _ptr(a):

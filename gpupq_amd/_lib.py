@@ -176,6 +176,7 @@ SIGNATURES = [
     ("gpq_queue_autotune_sort", ctypes.c_int, [c_void_p, c_void_p, c_f32, c_void_p, c_u32, ctypes.POINTER(c_u32)]),
     ("gpq_queue_device_view", ctypes.c_int, [c_void_p, ctypes.POINTER(ctypes.c_int), c_void_p, c_u64]),
     ("gpq_queue_stream", ctypes.c_int, [c_void_p, ctypes.POINTER(c_void_p)]),
+    ("gpq_release_kept_memory", ctypes.c_int, []),
     ("gpq_sort_events_noalloc", ctypes.c_int, [c_void_p, c_u32, c_void_p, c_void_p]),
 ]
 

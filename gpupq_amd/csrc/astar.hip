@@ -470,6 +470,7 @@ gpq_status AstarModel::create(QueueBase* queue, const gpq_astar_config& c, Astar
   AstarModel* m = new AstarModel();
   m->cfg = c;
   m->q = queue;
+  m->arena.on(queue->stream);
   const uint64_t cells = (uint64_t)c.width * c.height;
   gpq_status s;
   if ((s = m->arena.alloc(&m->blocked, (cells + 31) / 32)) != GPQ_OK || (s = m->arena.alloc(&m->g, cells)) != GPQ_OK ||

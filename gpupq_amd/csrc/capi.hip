@@ -20,8 +20,9 @@ gpq_status QueueBase::init_common() {
                 "block_threads must be a multiple of 64 and <= 1024");
   threads = cfg.block_threads;
   GPQ_HIP(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
+  arena.on(stream);
   GPQ_TRY(arena.alloc(&ws, 1));
-  GPQ_HIP(hipHostMalloc(reinterpret_cast<void**>(&host_ws), sizeof(WindowState), hipHostMallocDefault));
+  GPQ_TRY(host_ws_block.alloc(&host_ws, 1));
   std::memset(host_ws, 0, sizeof(WindowState));
   GPQ_HIP(hipMemcpyAsync(ws, host_ws, sizeof(WindowState), hipMemcpyHostToDevice, stream));
   if (cfg.collect_stats) {

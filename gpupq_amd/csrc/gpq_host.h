@@ -7,9 +7,11 @@
 
 #include <cstdio>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "../../include/gpupq.h"
+#include "devmem.h"
 #include "gpq_device.h"
 
 namespace gpq {
@@ -37,34 +39,70 @@ const std::string& last_error();
     if (!(cond)) { ::gpq::set_error(msg); return GPQ_ERR_INVALID; }                     \
   } while (0)
 
-// Device allocation tracked by its owner; freed in the owner's destructor.
+// Device memory tracked by its owner, given back in the owner's destructor (devmem.h keeps it for
+// the next owner, whose stream knows nothing of this owner's work: the work must have ended by
+// then).  The streams named with on() are waited for; the device as a whole is not, as that
+// would break a graph capture on another host thread.
 class DeviceArena {
  public:
   ~DeviceArena() { release(); }
+  void on(hipStream_t s) { streams_.push_back(s); }
   template <class T>
   gpq_status alloc(T** p, size_t count) {
-    void* raw = nullptr;
     const size_t bytes = count * sizeof(T) > 0 ? count * sizeof(T) : 16;
-    if (hipMalloc(&raw, bytes) != hipSuccess) {
-      (void)hipGetLastError();
+    size_t size = 0;
+    void* raw = mem_get(MemKind::kDevice, bytes, &size);
+    if (!raw) {
       set_error("hipMalloc of " + std::to_string(bytes) + " bytes failed");
       return GPQ_ERR_NOMEM;
     }
-    ptrs_.push_back(raw);
+    blocks_.push_back({raw, size});
     bytes_ += bytes;
     *p = static_cast<T*>(raw);
     return GPQ_OK;
   }
   size_t bytes() const { return bytes_; }
   void release() {
-    for (void* p : ptrs_) (void)hipFree(p);
-    ptrs_.clear();
+    for (hipStream_t s : streams_) (void)hipStreamSynchronize(s);
+    streams_.clear();
+    for (const auto& b : blocks_) mem_put(MemKind::kDevice, b.first, b.second);
+    blocks_.clear();
     bytes_ = 0;
   }
 
  private:
-  std::vector<void*> ptrs_;
+  std::vector<std::pair<void*, size_t>> blocks_;
+  std::vector<hipStream_t> streams_;
   size_t bytes_ = 0;
+};
+
+// Pinned host memory of one owner, which ends every copy to or from it first.
+class PinnedBlock {
+ public:
+  PinnedBlock() = default;
+  PinnedBlock(const PinnedBlock&) = delete;
+  PinnedBlock& operator=(const PinnedBlock&) = delete;
+  ~PinnedBlock() { release(); }
+  template <class T>
+  gpq_status alloc(T** p, size_t count) {
+    release();
+    p_ = mem_get(MemKind::kPinned, count * sizeof(T) > 0 ? count * sizeof(T) : 16, &size_);
+    if (!p_) {
+      set_error("hipHostMalloc of " + std::to_string(count * sizeof(T)) + " bytes failed");
+      return GPQ_ERR_HIP;
+    }
+    *p = static_cast<T*>(p_);
+    return GPQ_OK;
+  }
+  void release() {
+    if (!p_) return;
+    mem_put(MemKind::kPinned, p_, size_);
+    p_ = nullptr;
+  }
+
+ private:
+  void* p_ = nullptr;
+  size_t size_ = 0;
 };
 
 inline uint32_t ceil_div(uint64_t a, uint64_t b) { return (uint32_t)((a + b - 1) / b); }
@@ -77,8 +115,8 @@ class QueueBase {
  public:
   explicit QueueBase(const gpq_queue_config& c) : cfg(c) {}
   virtual ~QueueBase() {
+    arena.release();                         // waits for the stream
     if (stream) (void)hipStreamDestroy(stream);
-    if (host_ws) (void)hipHostFree(host_ws);
   }
   gpq_status init_common();
 
@@ -111,6 +149,7 @@ class QueueBase {
   DeviceArena arena;
   WindowState* ws = nullptr;          // device
   WindowState* host_ws = nullptr;     // pinned mirror for polling
+  PinnedBlock host_ws_block;
   hipEvent_t profile_mark = nullptr;  // when set, recorded just before the window publication
   uint32_t* partial = nullptr;        // device, one slot per reduction block
   uint32_t partial_slots = 0;

@@ -293,6 +293,7 @@ gpq_status PholdModel::create(QueueBase* queue, const gpq_phold_config& c, Phold
   PholdModel* m = new PholdModel();
   m->cfg = c;
   m->q = queue;
+  m->arena.on(queue->stream);
   gpq_status s = GPQ_OK;
   if ((s = m->arena.alloc(&m->count, c.num_lps)) != GPQ_OK ||
       (s = m->arena.alloc(&m->hash, c.num_lps)) != GPQ_OK ||

@@ -63,6 +63,7 @@ class PholdPool {
   WindowState* h_ws_ = nullptr;          // pinned mirror of d_ws_
   uint32_t* h_count_ = nullptr;          // pinned staging of retired instances' counters, by LP
   uint64_t* h_hash_ = nullptr;           // and hashes
+  PinnedBlock h_ws_block_, h_count_block_, h_hash_block_;
   hipEvent_t done_ = nullptr;
   hipGraph_t graph_ = nullptr;
   hipGraphExec_t graph_exec_ = nullptr;

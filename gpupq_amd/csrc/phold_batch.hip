@@ -275,10 +275,9 @@ gpq_status PholdPool::create(uint32_t capacity_lps, uint32_t capacity_per_lp, ui
   if (p->far_) p->q_->set_block_windows(p->d_block_win_, p->d_ws_);
   GPQ_TRY(p->arena_.alloc(&p->d_count_, cap));
   GPQ_TRY(p->arena_.alloc(&p->d_hash_, cap));
-  GPQ_HIP(hipHostMalloc(reinterpret_cast<void**>(&p->h_ws_), sizeof(WindowState) * max_instances,
-                        hipHostMallocDefault));
-  GPQ_HIP(hipHostMalloc(reinterpret_cast<void**>(&p->h_count_), sizeof(uint32_t) * cap, hipHostMallocDefault));
-  GPQ_HIP(hipHostMalloc(reinterpret_cast<void**>(&p->h_hash_), sizeof(uint64_t) * cap, hipHostMallocDefault));
+  GPQ_TRY(p->h_ws_block_.alloc(&p->h_ws_, max_instances));
+  GPQ_TRY(p->h_count_block_.alloc(&p->h_count_, cap));
+  GPQ_TRY(p->h_hash_block_.alloc(&p->h_hash_, cap));
   GPQ_HIP(hipEventCreateWithFlags(&p->done_, hipEventDisableTiming));
   p->inst_.assign(max_instances, PoolInst{});
   p->block_used_.assign(cap / kBlk, 0);
@@ -299,9 +298,6 @@ PholdPool::~PholdPool() {
   if (graph_exec_) (void)hipGraphExecDestroy(graph_exec_);
   if (graph_) (void)hipGraphDestroy(graph_);
   if (done_) (void)hipEventDestroy(done_);
-  if (h_ws_) (void)hipHostFree(h_ws_);
-  if (h_count_) (void)hipHostFree(h_count_);
-  if (h_hash_) (void)hipHostFree(h_hash_);
   arena_.release();
   delete q_;
 }
@@ -642,7 +638,9 @@ gpq_status PholdBatch::run_calendar_union(uint32_t batch, double* seconds) {
   std::unique_ptr<LaqQueue> q(new LaqQueue(qc));
   GPQ_TRY(q->init_common());
   GPQ_TRY(q->init());
-  DeviceArena arena;
+  PinnedBlock pinned_count, pinned_hash;      // host staging of the counters and hashes
+  DeviceArena arena;                          // destroyed first, so after the stream's last work
+  arena.on(q->stream);
   PoolInst* d_inst = nullptr;
   uint32_t* d_block = nullptr;
   uint32_t* d_count = nullptr;
@@ -691,16 +689,10 @@ gpq_status PholdBatch::run_calendar_union(uint32_t batch, double* seconds) {
   GPQ_TRY(st);
   GPQ_HIP(e);
   GPQ_HIP(hipGraphInstantiate(&gg.x, gg.g, nullptr, nullptr, 0));
-  struct Pinned {              // host staging of the counters and hashes
-    void* p = nullptr;
-    ~Pinned() {
-      if (p) (void)hipHostFree(p);
-    }
-  } pc, ph;
-  GPQ_HIP(hipHostMalloc(&pc.p, sizeof(uint32_t) * total, hipHostMallocDefault));
-  GPQ_HIP(hipHostMalloc(&ph.p, sizeof(uint64_t) * total, hipHostMallocDefault));
-  uint32_t* h_count = static_cast<uint32_t*>(pc.p);
-  uint64_t* h_hash = static_cast<uint64_t*>(ph.p);
+  uint32_t* h_count = nullptr;
+  uint64_t* h_hash = nullptr;
+  GPQ_TRY(pinned_count.alloc(&h_count, total));
+  GPQ_TRY(pinned_hash.alloc(&h_hash, total));
   const auto t0 = std::chrono::steady_clock::now();
   WindowState w{};
   for (;;) {

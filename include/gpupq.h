@@ -107,6 +107,12 @@ const char* gpq_last_error(void);
 /* Library version string. */
 const char* gpq_version(void);
 
+/* Device and pinned host memory that destroyed handles gave back is kept for the next handles, at
+ * most an eighth of the device's memory and 1 GiB of pinned memory per process, because the
+ * driver wipes freed device memory at about 33 GB/s.  An allocation that fails frees what is
+ * kept and tries again; this call frees it for the process's other users. */
+gpq_status gpq_release_kept_memory(void);
+
 /* ---- host queue API (src/queue.h:86-115) ------------------------------------------------ */
 /* queue_init() (src/queue.h:87): allocates and clears the queue. */
 gpq_status gpq_queue_create(const gpq_queue_config* cfg, gpq_queue** out);
