@@ -6,9 +6,9 @@
 // queue, R. Brown, CACM 31(10), 1988, with one day per window), split by the block of LPs the
 // events are for, and an event is appended to the log of its window and LP block.  Step c is one
 // launch with two kinds of blocks that run side by side:
-//   * commit blocks, one per block of kBlock LPs: the block's log of window c is grouped by LP in
-//     LDS, each LP's events are sorted in registers and committed in key order, and their
-//     successors are appended to the logs of their windows and LP blocks (one atomic each);
+//   * commit blocks, one per block of kBlock LPs: the block's log of window c is grouped by LP and
+//     put in key order in LDS, its events are committed, and their successors are appended to the
+//     logs of their windows and LP blocks;
 //   * a few list blocks: the events beyond the calendar (over[(c + 1) & 1]) whose window the
 //     calendar now reaches move into the logs.
 // No sorted run is kept, merged or shifted, and no separate pass groups the events by LP.
@@ -36,57 +36,25 @@ namespace cal {
 // self-addressed successors, larger ones fewer blocks in flight: at 2^20 LPs 64 LPs 1.37e10,
 // 128 LPs 1.59-1.66e10, 256 LPs 1.74-1.83e10, 512 LPs 1.60e10, 1024 LPs 1.42e10 events/s.
 constexpr int kBlock = 256;
-constexpr int kRegs = 8;          // events of one LP sorted in registers by one thread (fast path)
-constexpr int kWaveCand = 64;     // events of one LP on the slow path (one per lane)
-constexpr int kLogStage = 896;    // log records whose keys a commit block may keep in LDS while grouping
+constexpr uint32_t kLpMost = 64;  // events of one LP in one window
+constexpr uint32_t kPer = 4;      // events of one thread in a pass over the log
+constexpr uint32_t kPassCap = kPer * kBlock;   // events a commit block takes at once
 constexpr int kGroupBlocks = 2048;        // blocks of the standalone filing launch
 constexpr uint32_t kStepListBlocks = 32;  // blocks of a step that move the beyond-the-calendar events
 
-struct Key {
-  uint32_t ts, src, seq;
-};
-
-__device__ __forceinline__ bool key_lt(const Key& a, const Key& b) {
-  if (a.ts != b.ts) return a.ts < b.ts;
-  if (a.src != b.src) return a.src < b.src;
-  return a.seq < b.seq;
-}
-
-// Compare-exchange of keys a and b (ascending) held as three word arrays indexed by constants,
-// so that the sort network stays in registers (a network over an array of Key structs is
-// placed in scratch memory by the compiler).
-template <int A, int B>
-__device__ __forceinline__ void cswap3(uint32_t* t, uint32_t* s, uint32_t* q) {
-  const bool lt = t[B] != t[A] ? t[B] < t[A] : (s[B] != s[A] ? s[B] < s[A] : q[B] < q[A]);
-  const uint32_t t0 = lt ? t[B] : t[A], t1 = lt ? t[A] : t[B];
-  const uint32_t s0 = lt ? s[B] : s[A], s1 = lt ? s[A] : s[B];
-  const uint32_t q0 = lt ? q[B] : q[A], q1 = lt ? q[A] : q[B];
-  t[A] = t0; t[B] = t1;
-  s[A] = s0; s[B] = s1;
-  q[A] = q0; q[B] = q1;
-}
-
-// Batcher's odd-even merge sort of eight keys (19 comparators).
-__device__ __forceinline__ void sort8(uint32_t* t, uint32_t* s, uint32_t* q) {
-  cswap3<0, 1>(t, s, q); cswap3<2, 3>(t, s, q); cswap3<4, 5>(t, s, q); cswap3<6, 7>(t, s, q);
-  cswap3<0, 2>(t, s, q); cswap3<1, 3>(t, s, q); cswap3<4, 6>(t, s, q); cswap3<5, 7>(t, s, q);
-  cswap3<1, 2>(t, s, q); cswap3<5, 6>(t, s, q);
-  cswap3<0, 4>(t, s, q); cswap3<1, 5>(t, s, q); cswap3<2, 6>(t, s, q); cswap3<3, 7>(t, s, q);
-  cswap3<2, 4>(t, s, q); cswap3<3, 5>(t, s, q);
-  cswap3<1, 2>(t, s, q); cswap3<3, 4>(t, s, q); cswap3<5, 6>(t, s, q);
-}
-
 // Window offset of timestamp bits ts: the smallest o in [o_min, n) with ts < sw[o], where
-// sw[o] is the end of window x + o; n when ts >= sw[n - 1] (beyond the windows looked at).
-__device__ __forceinline__ uint32_t find_window(const uint32_t* sw, uint32_t n, uint32_t ts, uint32_t o_min) {
+// sw[o] is the end of window x + o; n when ts >= sw[n - 1] (beyond the windows looked at).  The
+// ends lie one lookahead apart (inv = 1 / lookahead), the last ones at the end time, so the search
+// starts at the window that the difference to the first end gives: it is off by at most a
+// few, where a binary search made six dependent LDS reads at 64 windows.
+__device__ __forceinline__ uint32_t find_window(const uint32_t* sw, uint32_t n, uint32_t ts, uint32_t o_min, float inv) {
   if (!(ts < sw[n - 1])) return n;
-  uint32_t lo = o_min, hi = n - 1;
-  while (lo < hi) {
-    const uint32_t mid = (lo + hi) >> 1;
-    if (ts < sw[mid]) hi = mid;
-    else lo = mid + 1;
-  }
-  return lo;
+  const float d = (bits_to_f(ts) - bits_to_f(sw[0])) * inv;
+  uint32_t o = d > 0.0f ? (uint32_t)fminf(d, (float)(n - 1u)) + 1u : 0u;
+  o = o < o_min ? o_min : (o < n ? o : n - 1u);
+  while (o > o_min && ts < sw[o - 1u]) --o;
+  while (!(ts < sw[o])) ++o;                           // ends: ts < sw[n - 1]
+  return o;
 }
 
 // Where an event goes, seen from window x with n windows looked at: a window offset o < n
@@ -96,12 +64,12 @@ struct Route {
   static constexpr uint32_t kParked = kCalMaxWindows + 1;
   static constexpr uint32_t kNone = kCalMaxWindows + 2;   // no record
 };
-constexpr uint32_t kRemote = 0x10000u;   // flag on a window route: the event is for another block's LPs
+constexpr uint32_t kRemote = 0x1000u;    // flag on a window route: the event is for another block's LPs
 
 __device__ __forceinline__ uint32_t route_of(const uint32_t* sw, uint32_t n, uint32_t ts, uint32_t end_bits,
-                                             uint32_t o_min) {
+                                             uint32_t o_min, float inv) {
   if (!(ts < end_bits)) return Route::kParked;
-  const uint32_t o = find_window(sw, n, ts, o_min);
+  const uint32_t o = find_window(sw, n, ts, o_min, inv);
   return o < n ? o : Route::kOver;
 }
 
@@ -193,257 +161,245 @@ __device__ __forceinline__ Event successor(const FusedModel& m, uint32_t lp, uin
   return Event{f_to_bits(t_new), dst, local, m.init_per_lp + n};
 }
 
-// Slow path, one wave for one LP with more than kRegs events in window c: the block's log of the
-// window is scanned for them (lane i gets the LP's i-th; with kStage, the keys the grouping kept
-// in LDS -- st, ss, sq, and the LP's index in the block sl -- stand for the log's first
-// kLogStage records), each lane ranks its event among the others, and the successors are filed
-// by their own atomics.
-template <bool kStage>
-__device__ __forceinline__ void slow_lp(const LaqView& q, const FusedModel& m, const uint32_t* sw, uint32_t c,
-                                        uint32_t end_bits, uint32_t lp, const Event* lg, uint32_t n, Key* keys,
-                                        const uint32_t* st, const uint32_t* ss, const uint32_t* sq,
-                                        const uint8_t* sl) {
-  const int lane = lane_id();
-  const uint64_t below = (1ull << lane) - 1ull;
-  const uint32_t l = lp & (kBlock - 1u);
-  uint32_t k = 0;
-  for (uint32_t base = 0; base < n; base += kWave) {     // wave-uniform trip count
-    const uint32_t i = base + (uint32_t)lane;
-    Event x{kInfBits, 0xFFFFFFFFu, 0u, 0u};
-    if (kStage && i < n && i < (uint32_t)kLogStage) {
-      if (sl[i] == l) x = Event{st[i], lp, ss[i], sq[i]};
-    } else if (i < n) {
-      x = load_event(&lg[i]);
-    }
-    const bool mine = x.dst == lp;
-    const uint64_t mm = __ballot(mine);
-    const uint32_t pos = k + (uint32_t)__popcll(mm & below);
-    if (mine && pos < (uint32_t)kWaveCand) keys[pos] = Key{x.ts, x.src, x.seq};
-    k += (uint32_t)__popcll(mm);
-  }
-  if (k > (uint32_t)kWaveCand) {
-    if (lane == 0) atomicOr(&q.ws->error, kErrStageOverflow);
-    k = kWaveCand;
-  }
-  laq::wave_lds_sync();
-  const bool has = (uint32_t)lane < k;
-  const Key me = has ? keys[lane] : Key{kInfBits, 0u, 0u};
-  uint32_t rank = 0;
-  for (uint32_t j = 0; j < k; ++j) {
-    const Key o{(uint32_t)__shfl((int)me.ts, (int)j, kWave), (uint32_t)__shfl((int)me.src, (int)j, kWave),
-                (uint32_t)__shfl((int)me.seq, (int)j, kWave)};
-    rank += key_lt(o, me) ? 1u : 0u;
-  }
-  laq::wave_lds_sync();                                  // every lane has read its key
-  const uint32_t cnt = m.count[lp];
-  Event ne{};
-  uint32_t r = Route::kNone;
-  if (has) {
-    keys[rank] = me;
-    ne = successor(m, lp, cnt + rank, me.ts);
-    r = route_of(sw, q.cal_windows, ne.ts, end_bits, 1u);
-    if (r < kCalMaxWindows) log_append(q, c + r, ne);
-  }
-  // the list successors: one reservation per list for the wave.  Near the end time almost every
-  // successor is parked, and with an atomic per lane on the one list counter the last steps took
-  // up to 410 us instead of 110-160.
-#pragma unroll
-  for (uint32_t li = 0; li < 2u; ++li) {
-    const uint32_t route = li ? Route::kParked : Route::kOver;
-    const uint64_t mm = __ballot(r == route);
-    if (!mm) continue;                                   // uniform across the wave
-    const int leader = __builtin_ctzll(mm);
-    uint32_t base = 0;
-    if (lane == leader) base = atomicAdd(list_count(q, c & 1u, route), (uint32_t)__popcll(mm));
-    base = (uint32_t)__shfl((int)base, leader, kWave);
-    if (r == route) list_store(q, c & 1u, route, base + (uint32_t)__popcll(mm & below), make_uint4(ne.ts, ne.dst, ne.src, ne.seq));
-  }
-  laq::wave_lds_sync();
-  if (lane == 0) {
-    uint64_t h = m.hash[lp];
-    uint32_t last = m.last_ts ? m.last_ts[lp] : 0u;
-    for (uint32_t r = 0; r < k; ++r) {
-      const Key x = keys[r];
-      h = trace_step(h, x.ts, x.src, x.seq);
-      if (m.last_ts) {
-        if (x.ts < last) atomicOr(&q.ws->error, kErrBadState);
-        last = x.ts;
-      }
-    }
-    m.count[lp] = cnt + k;
-    m.hash[lp] = h;
-    if (m.last_ts) m.last_ts[lp] = last;
-  }
-  laq::wave_lds_sync();
-}
-
-// Commit block `blk` of step c (window c): the block's log of the window is grouped by LP in LDS
-// (counts, and the log index of each LP's first kRegs events).  Fast path, one thread per LP
-// with at most kRegs events: sorted in registers and committed in order.  A successor for one of
-// this block's LPs (half of them in PHOLD: the self-addressed ones) and one for a list take a
-// rank in the block's LDS count of their window or list, one thread per window and list
-// reserves the block's run, and they are written into the runs; a successor for another block
-// goes to that block's log by its own atomic, all of a thread's issued before any is waited for.
-// LPs with more events are handled afterwards, one wave each (slow_lp).  The log is emptied at
-// the end.
-// kStage: the keys of the log's first kLogStage records are kept in LDS while grouping, and the
-// commit and the slow path read them there (the instances of one calendar: 1.81 -> 1.93e10
-// events/s; one 2^20-LP instance: 2-4% slower, so it keeps kStage off).
-template <bool kStage>
-__device__ __forceinline__ void commit_block(const LaqView& q, const FusedModel& m, float end_time, uint32_t c,
+// Commit block `blk` of step c (window c).  The block's log of the window is grouped by LP in LDS
+// (a count per LP, its prefix sum, the records in LP order), and then worked on event by event, a
+// thread per event: its rank among its LP's events (compared one by one: three on average),
+// which gives its draw number, its successor and where that goes.  Only the trace hash, a chain
+// over an LP's events in key order, is left to a thread per LP; it runs while the successors' slot
+// atomics are in flight.  A successor for one of this block's LPs (half of them in PHOLD: the
+// self-addressed ones) and one for a list take a rank in the block's LDS count of their window or
+// list, one thread per window and list reserves the block's run, and they are written into
+// the runs; a successor for another block goes to that block's log by its own atomic.  The log is
+// emptied at the end.  A log of more than kPassCap records is taken in passes over ranges of LPs.
+//
+// What bounds it: the atomics on the logs' counters, which are performed at the memory side at 26.6
+// G/s whatever lines they meet on: 1.7 M per step at 2^20 LPs x 32 events, 64 us of its 126.
+// With a thread per LP and its events in eight register slots (sorted by a network), a wave ran
+// all eight slots' draws for LPs that hold three events on average, and an LP with more was
+// committed by a wave of its own afterwards: 152 us per step (and 15.7 us at 1024 LPs, now 10.1).
+// Registers do not bind: 4, 5 and 6 waves per SIMD (105, 81 and 79 registers) took the same time.
+__device__ __forceinline__ void commit_block(const LaqView& q, const FusedModel& m, float end_time, float inv, uint32_t c,
                                              uint32_t blk) {
   __shared__ uint32_t sw[kCalMaxWindows];
-  __shared__ uint32_t s_cnt[kBlock];
-  __shared__ uint16_t s_idx[kBlock][kRegs];
+  __shared__ uint32_t s_cnt[kBlock], s_off[kBlock + 1], s_fill[kBlock], s_n0[kBlock];
+  __shared__ uint32_t s_ts[kPassCap], s_src[kPassCap], s_seq[kPassCap];
+  __shared__ uint8_t s_lp[kPassCap];
+  __shared__ uint32_t s_wave[kBlock / kWave];
   __shared__ uint32_t s_lcnt[2], s_lbase[2];
   __shared__ uint32_t s_wcnt[kCalMaxWindows], s_wbase[kCalMaxWindows];
-  __shared__ uint32_t s_slow[kBlock];
-  __shared__ uint32_t s_nslow;
-  __shared__ Key s_keys[kBlock / kWave][kWaveCand];
-  constexpr int kSt = kStage ? kLogStage : 1;
-  __shared__ uint32_t s_lt[kSt], s_ls[kSt], s_lq[kSt];   // with kStage: keys of the log's first records
-  __shared__ uint8_t s_ll[kSt];                          // and their LP's index in the block
   static_assert(kBlock <= 256, "an LP's index in its block fits a byte");
+  const uint32_t t = threadIdx.x;
   const uint32_t lp0 = blk << q.cal_block_log2;
-  const uint32_t lp = lp0 + threadIdx.x;
+  const uint32_t lp = lp0 + t;
   const bool in_range = lp < q.num_lps && lp - m.base < m.lps;
   const Event* lg = log_base(q, c, blk);
-  // issued together with the window ends' load: the log's length, the LP of the log record this
-  // thread groups first (slot threadIdx.x exists: a block's log has at least kBlock slots; used
-  // only below the length) and the thread's LP state, so that their latencies overlap
+  // issued together with the window ends' load: the log's length, the first two of the thread's
+  // records (the slots exist, or the second is not read; used only below the length) and the
+  // thread's LP state, so that their latencies overlap
   const uint32_t n0 = *log_count(q, c, blk);
-  Event e0{};
-  if (kStage) e0 = load_event(&lg[threadIdx.x]);
-  const uint32_t d0 = kStage ? e0.dst : lg[threadIdx.x].dst;
+  Event e[kPer];
+  e[0] = load_event(&lg[t]);
+  e[1] = Event{};
+  if (q.cal_sub_cap >= 2u * kBlock) e[1] = load_event(&lg[t + kBlock]);
   const uint32_t cnt_pre = in_range ? m.count[lp] : 0u;
   const uint64_t h_pre = in_range ? m.hash[lp] : 0ull;
   load_windows(q, c, sw);
   const uint32_t B = q.cal_windows;
-  s_cnt[threadIdx.x] = 0u;
-  for (uint32_t i = threadIdx.x; i < B; i += kBlock) s_wcnt[i] = 0u;
-  if (threadIdx.x < 2) s_lcnt[threadIdx.x] = 0u;
-  if (threadIdx.x == 0) s_nslow = 0;
+  const uint32_t end_bits = f_to_bits(end_time);
+  s_cnt[t] = 0u;
+  s_n0[t] = cnt_pre;
   __syncthreads();
   const uint32_t n = n0 < q.cal_sub_cap ? n0 : q.cal_sub_cap;
-  for (uint32_t i = threadIdx.x; i < n; i += kBlock) {
-    Event e{};
-    if (kStage) e = i == threadIdx.x ? e0 : load_event(&lg[i]);
-    const uint32_t l = (kStage ? e.dst : (i == threadIdx.x ? d0 : lg[i].dst)) - lp0;   // < kBlock: this block's LPs only
-    if (l >= (uint32_t)kBlock) {
-      atomicOr(&q.ws->error, kErrBadState);
-      continue;
+  uint32_t l[kPer], k[kPer];
+#pragma unroll
+  for (uint32_t j = 0; j < kPer; ++j) {
+    const uint32_t i = t + j * kBlock;
+    l[j] = kBlock;
+    k[j] = 0;
+    if (i < n) {
+      if (j >= 2u) e[j] = load_event(&lg[i]);
+      l[j] = e[j].dst - lp0;                           // < kBlock: this block's LPs only
+      if (l[j] < (uint32_t)kBlock) k[j] = atomicAdd(&s_cnt[l[j]], 1u);
+      else atomicOr(&q.ws->error, kErrBadState);
     }
-    if (kStage && i < (uint32_t)kLogStage) {            // kept for the commit and the slow path
-      s_lt[i] = e.ts;
-      s_ls[i] = e.src;
-      s_lq[i] = e.seq;
-      s_ll[i] = (uint8_t)l;
-    }
-    const uint32_t k = atomicAdd(&s_cnt[l], 1u);
-    if (k < (uint32_t)kRegs) s_idx[l][k] = (uint16_t)i;
+  }
+  for (uint32_t i = t + kPassCap; i < n; i += kBlock) {
+    const uint32_t x = lg[i].dst - lp0;
+    if (x < (uint32_t)kBlock) atomicAdd(&s_cnt[x], 1u);
+    else atomicOr(&q.ws->error, kErrBadState);
   }
   __syncthreads();
-  const uint32_t end_bits = f_to_bits(end_time);
-  uint4 ne[kRegs];      // list successors as uint4: an array of the 16-byte-aligned Event goes to scratch memory
-  uint32_t route[kRegs], rank[kRegs];
-  uint32_t cn = 0;
-  if (in_range) {
-    const uint32_t k = s_cnt[threadIdx.x];
-    if (k > (uint32_t)kRegs) {
-      s_slow[atomicAdd(&s_nslow, 1u)] = lp;
-    } else if (k) {
-      cn = k;
-      uint32_t kt[kRegs], ks[kRegs], kq[kRegs];
+  const uint32_t mine = s_cnt[t];                      // events of the thread's LP
+  if (mine > kLpMost) atomicOr(&q.ws->error, kErrStageOverflow);
+  uint32_t inc = mine;
 #pragma unroll
-      for (int s = 0; s < kRegs; ++s) {
-        if ((uint32_t)s < cn) {
-          const uint32_t ix = s_idx[threadIdx.x][s];
-          if (kStage && ix < (uint32_t)kLogStage) {
-            kt[s] = s_lt[ix];
-            ks[s] = s_ls[ix];
-            kq[s] = s_lq[ix];
-          } else {
-            const Event e = load_event(&lg[ix]);
-            kt[s] = e.ts;
-            ks[s] = e.src;
-            kq[s] = e.seq;
-          }
-        } else {
-          kt[s] = ks[s] = kq[s] = 0xFFFFFFFFu;
-        }
+  for (int off = 1; off < kWave; off <<= 1) {
+    const uint32_t y = (uint32_t)__shfl_up((int)inc, off, kWave);
+    if (lane_id() >= off) inc += y;
+  }
+  if (lane_id() == kWave - 1) s_wave[t / kWave] = inc;
+  __syncthreads();
+  for (uint32_t w = 0; w < t / kWave; ++w) inc += s_wave[w];
+  s_off[t + 1u] = inc;
+  if (t == 0) s_off[0] = 0u;
+  __syncthreads();
+  const bool whole = n <= kPassCap;
+  if (whole) {                                         // the records into LP order, from registers
+#pragma unroll
+    for (uint32_t j = 0; j < kPer; ++j) {
+      if (l[j] >= (uint32_t)kBlock) continue;
+      const uint32_t p = s_off[l[j]] + k[j];
+      s_ts[p] = e[j].ts;
+      s_src[p] = e[j].src;
+      s_seq[p] = e[j].seq;
+      s_lp[p] = (uint8_t)l[j];
+    }
+  }
+  for (uint32_t first = 0; first < (uint32_t)kBlock;) {   // one pass unless the log is longer than kPassCap
+    uint32_t last = kBlock;
+    const uint32_t base = s_off[first];
+    if (!whole) {                                      // the LPs from `first` on whose events fit
+      last = first + (uint32_t)__syncthreads_count(t >= first && s_off[t + 1u] - base <= kPassCap);
+      if (last == first) {                             // an LP of more than kPassCap > kLpMost events: refused above
+        ++first;
+        continue;
       }
-      const uint32_t cnt = cnt_pre;
+      s_fill[t] = 0u;
+    }
+    const uint32_t take = s_off[last] - base;
+    for (uint32_t i = t; i < B; i += kBlock) s_wcnt[i] = 0u;
+    if (t < 2) s_lcnt[t] = 0u;
+    if (!whole) {
+      __syncthreads();
+      for (uint32_t i = t; i < n; i += kBlock) {
+        const Event x = load_event(&lg[i]);
+        const uint32_t xl = x.dst - lp0;
+        if (xl < first || xl >= last) continue;
+        const uint32_t p = s_off[xl] - base + atomicAdd(&s_fill[xl], 1u);
+        s_ts[p] = x.ts;
+        s_src[p] = x.src;
+        s_seq[p] = x.seq;
+        s_lp[p] = (uint8_t)xl;
+      }
+    }
+    __syncthreads();
+    // a thread per event: its rank among its LP's events
+    {
+      uint32_t ets[kPer], esrc[kPer], eseq[kPer], to[kPer];
+#pragma unroll
+      for (uint32_t j = 0; j < kPer; ++j) {
+        const uint32_t p = t + j * kBlock;
+        if (p >= take) continue;
+        const uint32_t el = s_lp[p], o = s_off[el] - base, kk = s_cnt[el];
+        ets[j] = s_ts[p];
+        esrc[j] = s_src[p];
+        eseq[j] = s_seq[p];
+        uint32_t rank = 0;
+        for (uint32_t i = 0; i < kk; ++i) {
+          const uint32_t ot = s_ts[o + i];
+          bool before = ot < ets[j];
+          if (ot == ets[j] && o + i != p) {            // equal times: by source, then number, then arrival
+            const uint32_t os = s_src[o + i], oq = s_seq[o + i];
+            before = os != esrc[j] ? os < esrc[j] : (oq != eseq[j] ? oq < eseq[j] : o + i < p);
+          }
+          rank += before ? 1u : 0u;
+        }
+        to[j] = o + rank;
+      }
+      __syncthreads();                                 // every rank is taken; the records move into key order
+#pragma unroll
+      for (uint32_t j = 0; j < kPer; ++j) {
+        if (t + j * kBlock >= take) continue;
+        s_ts[to[j]] = ets[j];
+        s_src[to[j]] = esrc[j];
+        s_seq[to[j]] = eseq[j];
+      }
+    }
+    __syncthreads();
+    // a thread per LP: the trace hash
+    if (in_range && mine && t >= first && t < last) {
       uint64_t h = h_pre;
-      uint32_t last = m.last_ts ? m.last_ts[lp] : 0u;
-      sort8(kt, ks, kq);
-#pragma unroll
-      for (int j = 0; j < kRegs; ++j) {
-        route[j] = Route::kNone;
-        if ((uint32_t)j < cn) {
-          h = trace_step(h, kt[j], ks[j], kq[j]);
-          if (m.last_ts) {
-            if (kt[j] < last) atomicOr(&q.ws->error, kErrBadState);
-            last = kt[j];
-          }
-          const Event sc = successor(m, lp, cnt + (uint32_t)j, kt[j]);
-          const uint32_t r = route_of(sw, B, sc.ts, end_bits, 1u);
-          route[j] = r;
-          ne[j] = make_uint4(sc.ts, sc.dst, sc.src, sc.seq);
-          if (r < kCalMaxWindows) {
-            if ((sc.dst >> q.cal_block_log2) == blk) rank[j] = atomicAdd(&s_wcnt[r], 1u);   // this block's log
-            else route[j] = r | kRemote;
-          } else {
-            rank[j] = atomicAdd(&s_lcnt[r == Route::kParked ? 1u : 0u], 1u);
-          }
+      uint32_t prev = m.last_ts ? m.last_ts[lp] : 0u;
+      const uint32_t o = s_off[t] - base;
+      for (uint32_t i = 0; i < mine; ++i) {
+        const uint32_t xt = s_ts[o + i];
+        h = trace_step(h, xt, s_src[o + i], s_seq[o + i]);
+        if (m.last_ts) {
+          if (xt < prev) atomicOr(&q.ws->error, kErrBadState);
+          prev = xt;
         }
       }
-      m.count[lp] = cnt + cn;
+      m.count[lp] = cnt_pre + mine;
       m.hash[lp] = h;
-      if (m.last_ts) m.last_ts[lp] = last;
+      if (m.last_ts) m.last_ts[lp] = prev;
     }
-  }
-  // successors for other blocks' logs: every slot atomic of the thread in flight at once
-  uint32_t pos[kRegs];
-#pragma unroll
-  for (int j = 0; j < kRegs; ++j)
-    pos[j] = (uint32_t)j < cn && (route[j] & kRemote)
-                 ? atomicAdd(log_count(q, c + (route[j] & ~kRemote), ne[j].y >> q.cal_block_log2), 1u)
-                 : 0u;
-  __syncthreads();
-  // one run per window (this block's own log) and per list for the block
-  for (uint32_t i = threadIdx.x; i < B; i += kBlock) {
-    const uint32_t t = s_wcnt[i];
-    s_wbase[i] = t ? atomicAdd(log_count(q, c + i, blk), t) : 0u;
-  }
-  if (threadIdx.x < 2) {
-    const uint32_t t = s_lcnt[threadIdx.x];
-    s_lbase[threadIdx.x] = t ? atomicAdd(list_count(q, c & 1u, threadIdx.x ? Route::kParked : Route::kOver), t) : 0u;
-  }
-#pragma unroll
-  for (int j = 0; j < kRegs; ++j) {
-    if ((uint32_t)j < cn && (route[j] & kRemote)) {
-      const uint32_t r = route[j] & ~kRemote;
-      if (pos[j] < q.cal_sub_cap) *reinterpret_cast<uint4*>(log_base(q, c + r, ne[j].y >> q.cal_block_log2) + pos[j]) = ne[j];
-      else atomicOr(&q.ws->error, kErrQueueOverflow);
+    __syncthreads();                                   // the events' words now hold their successors
+    // a thread per event, one after the other (side by side they take 108 registers, four waves per
+    // SIMD): the successor's time and destination, and its route with its rank in this
+    // block's run of that window or list
+#pragma unroll 1
+    for (uint32_t p = t; p < take; p += kBlock) {
+      const uint32_t el = s_lp[p], elp = lp0 + el;
+      uint32_t way = Route::kNone;
+      if (elp < q.num_lps && elp - m.base < m.lps) {
+        const Event sc = successor(m, elp, s_n0[el] + (p - (s_off[el] - base)), s_ts[p]);
+        const uint32_t r = route_of(sw, B, sc.ts, end_bits, 1u, inv);
+        s_ts[p] = sc.ts;
+        s_src[p] = sc.dst;
+        if (r >= kCalMaxWindows) way = r | (atomicAdd(&s_lcnt[r == Route::kParked ? 1u : 0u], 1u) << 16);
+        else if ((sc.dst >> q.cal_block_log2) == blk) way = r | (atomicAdd(&s_wcnt[r], 1u) << 16);
+        else way = r | kRemote;
+      }
+      s_seq[p] = way;
     }
-  }
-  __syncthreads();
+    // successors for other blocks' logs: every slot atomic of the thread in flight at once
+    uint32_t pos[kPer];
 #pragma unroll
-  for (int j = 0; j < kRegs; ++j) {
-    if ((uint32_t)j >= cn || (route[j] & kRemote)) continue;
-    const uint32_t r = route[j];
-    if (r < kCalMaxWindows) {
-      const uint32_t p = s_wbase[r] + rank[j];
-      if (p < q.cal_sub_cap) *reinterpret_cast<uint4*>(log_base(q, c + r, blk) + p) = ne[j];
-      else atomicOr(&q.ws->error, kErrQueueOverflow);
-    } else {
-      list_store(q, c & 1u, r, s_lbase[r == Route::kParked ? 1u : 0u] + rank[j], ne[j]);
+    for (uint32_t j = 0; j < kPer; ++j) {
+      const uint32_t p = t + j * kBlock;
+      const uint32_t way = p < take ? s_seq[p] : (uint32_t)Route::kNone;
+      pos[j] = way & kRemote ? atomicAdd(log_count(q, c + (way & 0xFFFu), s_src[p] >> q.cal_block_log2), 1u) : 0u;
     }
+    __syncthreads();
+    // one run per window (this block's own log) and per list for the block
+    for (uint32_t i = t; i < B; i += kBlock) {
+      const uint32_t x = s_wcnt[i];
+      s_wbase[i] = x ? atomicAdd(log_count(q, c + i, blk), x) : 0u;
+    }
+    if (t < 2) {
+      const uint32_t x = s_lcnt[t];
+      s_lbase[t] = x ? atomicAdd(list_count(q, c & 1u, t ? Route::kParked : Route::kOver), x) : 0u;
+    }
+    auto record = [&](uint32_t p) {
+      const uint32_t el = s_lp[p];
+      return make_uint4(s_ts[p], s_src[p], lp0 + el - m.base, m.init_per_lp + s_n0[el] + (p - (s_off[el] - base)));
+    };
+#pragma unroll
+    for (uint32_t j = 0; j < kPer; ++j) {
+      const uint32_t p = t + j * kBlock;
+      const uint32_t way = p < take ? s_seq[p] : (uint32_t)Route::kNone;
+      if (!(way & kRemote)) continue;
+      if (pos[j] < q.cal_sub_cap)
+        *reinterpret_cast<uint4*>(log_base(q, c + (way & 0xFFFu), s_src[p] >> q.cal_block_log2) + pos[j]) = record(p);
+      else
+        atomicOr(&q.ws->error, kErrQueueOverflow);
+    }
+    __syncthreads();
+    for (uint32_t p = t; p < take; p += kBlock) {
+      const uint32_t way = s_seq[p], r = way & 0xFFFu, rank = way >> 16;
+      if ((way & kRemote) || r == Route::kNone) continue;
+      if (r < kCalMaxWindows) {
+        const uint32_t i = s_wbase[r] + rank;
+        if (i < q.cal_sub_cap) *reinterpret_cast<uint4*>(log_base(q, c + r, blk) + i) = record(p);
+        else atomicOr(&q.ws->error, kErrQueueOverflow);
+      } else {
+        list_store(q, c & 1u, r, s_lbase[r == Route::kParked ? 1u : 0u] + rank, record(p));
+      }
+    }
+    first = last;
+    if (first < (uint32_t)kBlock) __syncthreads();     // the next pass clears the counts
   }
-  const uint32_t w = threadIdx.x / kWave;
-  for (uint32_t i = w; i < s_nslow; i += kBlock / kWave) slow_lp<kStage>(q, m, sw, c, end_bits, s_slow[i], lg, n, s_keys[w], s_lt, s_ls, s_lq, s_ll);
-  __syncthreads();
-  if (threadIdx.x == 0) *log_count(q, c, blk) = 0u;     // the block's log of window c is consumed
+  if (t == 0) *log_count(q, c, blk) = 0u;              // the block's log of window c is consumed
 }
 
 // The end of the step that committed window c (its logs emptied by the commit blocks): the list
@@ -488,7 +444,7 @@ __device__ __forceinline__ void block_done(const LaqView& q, float lookahead, fl
 // windows -- x .. x + B - 2, all of them beyond the window being committed and short of the
 // one whose log slot it is reading -- and go to the log of their window, on to over[(x + 1) & 1],
 // or with the parked ones.
-__device__ __forceinline__ void list_block(const LaqView& q, float end_time, uint32_t x, uint32_t blk,
+__device__ __forceinline__ void list_block(const LaqView& q, float end_time, float inv, uint32_t x, uint32_t blk,
                                            uint32_t nblk) {
   __shared__ uint32_t sw[kCalMaxWindows];
   __shared__ ListAppend la;
@@ -505,7 +461,7 @@ __device__ __forceinline__ void list_block(const LaqView& q, float end_time, uin
     const uint32_t i = base + threadIdx.x;
     const bool has = i < no;
     const Event e = has ? load_event(&ov[i]) : Event{};
-    const uint32_t r = has ? route_of(sw, B - 1u, e.ts, end_bits, 0u) : Route::kNone;
+    const uint32_t r = has ? route_of(sw, B - 1u, e.ts, end_bits, 0u, inv) : Route::kNone;
     block_file(q, x, wp, r, e, la);
   }
 }

@@ -789,7 +789,7 @@ __global__ void cal_start_kernel(LaqView q, float lookahead, float end_time) {
 
 // Files every initial event (the list over[0]) in the log of its window (windows 0 .. B - 1)
 // and LP block, in over[1] (read by the first step), or with the parked ones.
-__global__ __launch_bounds__(cal::kBlock) void cal_fill_kernel(LaqView q, float end_time) {
+__global__ __launch_bounds__(cal::kBlock) void cal_fill_kernel(LaqView q, float end_time, float inv) {
   __shared__ uint32_t sw[kCalMaxWindows];
   __shared__ cal::ListAppend la;
   cal::load_windows(q, 0u, sw);
@@ -802,7 +802,7 @@ __global__ __launch_bounds__(cal::kBlock) void cal_fill_kernel(LaqView q, float 
     const uint32_t i = base + threadIdx.x;
     const bool has = i < n;
     const Event e = has ? load_event(&src[i]) : Event{};
-    const uint32_t r = has ? cal::route_of(sw, B, e.ts, end_bits, 0u) : cal::Route::kNone;
+    const uint32_t r = has ? cal::route_of(sw, B, e.ts, end_bits, 0u, inv) : cal::Route::kNone;
     cal::block_file(q, 0u, 1u, r, e, la);
   }
 }
@@ -990,7 +990,8 @@ gpq_status LaqQueue::init_calendar() {
 gpq_status LaqQueue::calendar_start() {
   GPQ_CHECK_ARG(v_.wlog, "LAQ: calendar_start needs calendar mode");
   hipLaunchKernelGGL(cal_start_kernel, dim3(1), dim3(1), 0, stream, v_, cfg.lookahead, cfg.horizon);
-  hipLaunchKernelGGL(cal_fill_kernel, dim3(cal::kGroupBlocks), dim3(cal::kBlock), 0, stream, v_, cfg.horizon);
+  hipLaunchKernelGGL(cal_fill_kernel, dim3(cal::kGroupBlocks), dim3(cal::kBlock), 0, stream, v_, cfg.horizon,
+                     1.0f / cfg.lookahead);
   hipLaunchKernelGGL(cal_fill_done_kernel, dim3(1), dim3(1), 0, stream, v_);
   GPQ_HIP(hipGetLastError());
   return GPQ_OK;
