@@ -604,7 +604,8 @@ gpq_status PholdBatch::run_calendar_union(uint32_t batch, double* seconds) {
   uint32_t max_init = 0;
   float la = inst[0].lookahead, horizon = inst[0].end_time;
   for (uint32_t i = 0; i < n; ++i) {
-    const uint32_t blocks = (uint32_t)ceil_div(inst[i].num_lps, kCalBlk);
+    // whole units of a large calendar, so whole commit blocks of a small one
+    const uint32_t blocks = (uint32_t)ceil_div(inst[i].num_lps, cal::kUnit) * (cal::kUnit / kCalBlk);
     PoolInst& t = tab[i];
     t = PoolInst{};
     t.base = (uint32_t)total;

@@ -13,6 +13,7 @@
 #include <cmath>
 
 #include "laq_calendar.cuh"
+#include "laq_calendar_groups.cuh"
 #include "laq_merge.cuh"
 #include "phold_fused.cuh"
 #include "queues.h"
@@ -707,11 +708,16 @@ __global__ void laq_update_kernel(LaqView q, uint32_t* partial) {
 // The block reserves one run for all its LPs' staged events (one atomic per block: an atomic per
 // wave on the list counter took 192 us per launch at 2^20 LPs), and each thread writes its LP's
 // events at its prefix in the run.
-__global__ __launch_bounds__(kLaqBlock) void cal_post_init_kernel(LaqView q, uint32_t* partial) {
+__global__ __launch_bounds__(kLaqBlock) void cal_post_init_kernel(LaqView q, cal::Groups g, uint32_t* partial) {
   __shared__ uint32_t s_wave[kLaqBlock / kWave];
   __shared__ uint32_t s_base;
   const uint32_t lp = blockIdx.x * kLaqBlock + threadIdx.x;
   const int lane = lane_id(), wave = (int)threadIdx.x / kWave;
+  // the list of the LPs' group, or the one list of a small calendar
+  const uint32_t grp = g.units ? (blockIdx.x * kLaqBlock) >> g.group_shift : 0u;
+  Event* list = g.units ? g.over + (size_t)grp * g.over_cap : q.over;
+  uint32_t* list_n = g.units ? g.over_n + grp * 16u : &q.over_n[0];
+  const uint32_t list_cap = g.units ? g.over_cap : q.over_cap;
   uint32_t k0 = 0, k = 0;
   if (lp < q.num_lps) {
     k0 = q.ins[lp];
@@ -732,7 +738,7 @@ __global__ __launch_bounds__(kLaqBlock) void cal_post_init_kernel(LaqView q, uin
       s_wave[w] = tot;
       tot += t;
     }
-    s_base = tot ? atomicAdd(&q.over_n[0], tot) : 0u;
+    s_base = tot ? atomicAdd(list_n, tot) : 0u;
   }
   __syncthreads();
   const uint32_t start = s_base + s_wave[wave] + (incl - k);
@@ -740,7 +746,7 @@ __global__ __launch_bounds__(kLaqBlock) void cal_post_init_kernel(LaqView q, uin
   for (uint32_t i = 0; i < k; ++i) {
     const Event e = load_event(&q.stage[(size_t)lp * q.stage_cap + i]);
     m = e.ts < m ? e.ts : m;
-    if (start + i < q.over_cap) store_event(&q.over[start + i], e);
+    if (start + i < list_cap) store_event(&list[start + i], e);
     else atomicOr(&q.ws->error, kErrQueueOverflow);
   }
   if (k0) q.ins[lp] = 0;
@@ -863,6 +869,59 @@ __global__ void cal_gather_kernel(LaqView q, uint32_t lp, Event* out, uint32_t c
   }
 }
 
+__global__ __launch_bounds__(cal::kFileThreads) void cal_file_kernel(LaqView q, cal::Groups g, float end_time, float inv) {
+  extern __shared__ uint32_t s_file_counts[];
+  cal::file_group(q, g, end_time, inv, s_file_counts);
+}
+
+// The same two over a large calendar: the logs of the units, the groups' lists, the outboxes of the
+// last step, the parked ones and the staging slots.
+__global__ void cal_units_count_kernel(LaqView q, cal::Groups g, unsigned long long* sum) {
+  __shared__ unsigned long long s[16];
+  const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x, stride = gridDim.x * blockDim.x;
+  unsigned long long n = 0;
+  for (uint32_t i = t; i < q.num_lps; i += stride) n += min(q.ins[i], q.stage_cap);
+  for (uint32_t i = t; i < g.units * q.cal_windows; i += stride) n += min(g.wlog_n[i], g.log_cap);
+  for (uint32_t i = t; i < g.groups; i += stride) n += min(g.over_n[i * 16u], g.over_cap);
+  for (uint32_t u = t; u < g.units; u += stride)
+    for (uint32_t p = 0; p < g.npass[u]; ++p)
+      for (uint32_t i = 0; i < cal::kMaxGroups; ++i) n += g.parts[((size_t)u * g.passes + p) * cal::kMaxGroups + i] >> 16;
+  if (t == 0) n += min(*q.parked_n, q.parked_cap);
+  for (int off = 32; off > 0; off >>= 1) n += __shfl_xor(n, off, kWave);
+  if (lane_id() == 0) s[threadIdx.x / kWave] = n;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    unsigned long long tot = 0;
+    for (int w = 0; w < (int)(blockDim.x / kWave); ++w) tot += s[w];
+    if (tot) atomicAdd(sum, tot);
+  }
+}
+
+__global__ void cal_units_gather_kernel(LaqView q, cal::Groups g, uint32_t lp, Event* out, uint32_t cap, uint32_t* n) {
+  const uint32_t stride = gridDim.x * blockDim.x;
+  const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+  const uint32_t unit = lp >> cal::kUnitLog2, grp = lp >> g.group_shift;
+  for (uint32_t x = 0; x < q.cal_windows; ++x) {
+    const uint32_t c = min(*cal::unit_count(q, g, unit, x), g.log_cap);
+    const Event* lg = cal::unit_log(q, g, unit, x);
+    for (uint32_t i = t; i < c; i += stride) gather_one(&lg[i], lp, out, cap, n);
+  }
+  const uint32_t no = min(g.over_n[grp * 16u], g.over_cap);
+  for (uint32_t i = t; i < no; i += stride) gather_one(&g.over[(size_t)grp * g.over_cap + i], lp, out, cap, n);
+  for (uint32_t u = t; u < g.units; u += stride)
+    for (uint32_t p = 0; p < g.npass[u]; ++p) {
+      const size_t slot = (size_t)u * g.passes + p;
+      const uint32_t part = g.parts[slot * cal::kMaxGroups + grp], from = part & 0xFFFFu;
+      for (uint32_t i = 0; i < part >> 16; ++i) gather_one(&g.out[slot * cal::kUnitPass + from + i], lp, out, cap, n);
+    }
+  const uint32_t c = min(*q.parked_n, q.parked_cap);
+  for (uint32_t i = t; i < c; i += stride) gather_one(&q.parked[i], lp, out, cap, n);
+  if (t == 0) {
+    const uint32_t k0 = min(q.ins[lp], q.stage_cap);
+    for (uint32_t i = 0; i < k0; ++i) gather_one(&q.stage[(size_t)lp * q.stage_cap + i], lp, out, cap, n);
+  }
+}
+
 }  // namespace
 
 gpq_status LaqQueue::init() {
@@ -963,20 +1022,28 @@ gpq_status LaqQueue::init_calendar() {
   GPQ_TRY(arena.alloc(&v_.ins, L));
   GPQ_TRY(arena.alloc(&v_.head, L));
   GPQ_TRY(arena.alloc(&sum_, 1));
-  // the logs' counters (16 words apart), then over_n[2] and parked_n, each on a 128-byte line of
-  // its own: every block of a step may reserve a run on them, and a line that such atomics share
-  // with words that blocks read (or with each other) slows every access to it
-  const size_t lists_at = (((size_t)B * blocks << cal::kLogCountShift) + 31u) & ~(size_t)31u;
-  const size_t counters = lists_at + 64u;
-  GPQ_TRY(arena.alloc(&v_.wlog, (size_t)B * v_.wlog_cap));
-  GPQ_TRY(arena.alloc(&v_.wlog_n, counters));
-  v_.over_n = v_.wlog_n + lists_at;
-  GPQ_TRY(arena.alloc(&v_.over, 2 * (size_t)v_.over_cap));
+  if (L >= kGroupedMinLps) {
+    GPQ_TRY(init_calendar_groups());
+    GPQ_TRY(arena.alloc(&v_.over_n, 64));             // the list counters' places; only the parked one is used
+    v_.wlog = groups_.wlog;
+    v_.parked_n = v_.over_n + 32u;
+    GPQ_HIP(hipMemsetAsync(v_.over_n, 0, sizeof(uint32_t) * 64, stream));
+  } else {
+    // the logs' counters (16 words apart), then over_n[2] and parked_n, each on a 128-byte line of
+    // its own: every block of a step may reserve a run on them, and a line that such atomics share
+    // with words that blocks read (or with each other) slows every access to it
+    const size_t lists_at = (((size_t)B * blocks << cal::kLogCountShift) + 31u) & ~(size_t)31u;
+    const size_t counters = lists_at + 64u;
+    GPQ_TRY(arena.alloc(&v_.wlog, (size_t)B * v_.wlog_cap));
+    GPQ_TRY(arena.alloc(&v_.wlog_n, counters));
+    v_.over_n = v_.wlog_n + lists_at;
+    v_.parked_n = v_.wlog_n + lists_at + 32u;
+    GPQ_TRY(arena.alloc(&v_.over, 2 * (size_t)v_.over_cap));
+    GPQ_HIP(hipMemsetAsync(v_.wlog_n, 0, sizeof(uint32_t) * counters, stream));
+  }
   GPQ_TRY(arena.alloc(&v_.parked, (size_t)v_.parked_cap));
   GPQ_TRY(arena.alloc(&v_.cal_st, 1));
   GPQ_TRY(arena.alloc(&gather_, kGatherCap + 1));
-  v_.parked_n = v_.wlog_n + lists_at + 32u;
-  GPQ_HIP(hipMemsetAsync(v_.wlog_n, 0, sizeof(uint32_t) * counters, stream));
   GPQ_HIP(hipMemsetAsync(v_.cal_st, 0, sizeof(CalState), stream));
   v_.ws = ws;
   v_.stats = stats;
@@ -987,9 +1054,58 @@ gpq_status LaqQueue::init_calendar() {
   return GPQ_OK;
 }
 
+// Units, groups and their buffers.  A group's list holds twice its share of far_per_lp, so that
+// uniform destinations never fill it before the whole queue's bound; a pass over a log takes all
+// but the last LP's events that fit.
+gpq_status LaqQueue::init_calendar_groups() {
+  const uint32_t L = cfg.num_lps, B = cfg.calendar_windows;
+  cal::Groups& g = groups_;
+  g.units = (uint32_t)ceil_div(L, cal::kUnit);
+  g.group_shift = cal::kUnitLog2;
+  while (((L - 1u) >> g.group_shift) + 1u > cal::kMaxGroups) ++g.group_shift;
+  g.groups = ((L - 1u) >> g.group_shift) + 1u;
+  g.log_cap = cal::kUnit * cfg.capacity_per_lp;
+  g.passes = g.log_cap / (cal::kUnitPass - cal::kLpMost) + 1u;
+  const uint64_t over = 2ull * cfg.far_per_lp << g.group_shift;
+  GPQ_CHECK_ARG(over < (1ull << 32), "LAQ calendar: num_lps too large for the groups' lists");
+  g.over_cap = (uint32_t)over;
+  const size_t slots = (size_t)g.units * g.passes;
+  GPQ_TRY(arena.alloc(&g.wlog, (size_t)g.units * B * g.log_cap));
+  GPQ_TRY(arena.alloc(&g.wlog_n, (size_t)g.units * B));
+  GPQ_TRY(arena.alloc(&g.out, slots * cal::kUnitPass));
+  GPQ_TRY(arena.alloc(&g.parts, slots * cal::kMaxGroups));
+  GPQ_TRY(arena.alloc(&g.npass, g.units));
+  GPQ_TRY(arena.alloc(&g.over, (size_t)g.groups * g.over_cap));
+  GPQ_TRY(arena.alloc(&g.over_n, (size_t)g.groups * 16u));
+  GPQ_HIP(hipMemsetAsync(g.wlog_n, 0, sizeof(uint32_t) * g.units * B, stream));
+  GPQ_HIP(hipMemsetAsync(g.npass, 0, sizeof(uint32_t) * g.units, stream));
+  GPQ_HIP(hipMemsetAsync(g.parts, 0, sizeof(uint32_t) * slots * cal::kMaxGroups, stream));
+  GPQ_HIP(hipMemsetAsync(g.over_n, 0, sizeof(uint32_t) * g.groups * 16u, stream));
+  const size_t lds = sizeof(uint32_t) * ((size_t)B << (g.group_shift - cal::kUnitLog2));
+  GPQ_CHECK_ARG(lds <= 96u * 1024u, "LAQ calendar: num_lps * calendar_windows too large for the filing step's counts");
+  if (lds > 16u * 1024u)
+    GPQ_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(cal_file_kernel),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  return GPQ_OK;
+}
+
+gpq_status LaqQueue::calendar_file() {
+  const cal::Groups& g = groups_;
+  GPQ_CHECK_ARG(g.units, "LAQ: calendar_file needs a large calendar");
+  const size_t lds = sizeof(uint32_t) * ((size_t)cfg.calendar_windows << (g.group_shift - cal::kUnitLog2));
+  hipLaunchKernelGGL(cal_file_kernel, dim3(ceil_div(g.groups, cal::kXcds) * cal::kXcds), dim3(cal::kFileThreads), lds, stream, v_, g, cfg.horizon,
+                     1.0f / cfg.lookahead);
+  GPQ_HIP(hipGetLastError());
+  return GPQ_OK;
+}
+
 gpq_status LaqQueue::calendar_start() {
   GPQ_CHECK_ARG(v_.wlog, "LAQ: calendar_start needs calendar mode");
   hipLaunchKernelGGL(cal_start_kernel, dim3(1), dim3(1), 0, stream, v_, cfg.lookahead, cfg.horizon);
+  if (groups_.units) {       // the groups' lists hold every initial event
+    GPQ_HIP(hipGetLastError());
+    return calendar_file();
+  }
   hipLaunchKernelGGL(cal_fill_kernel, dim3(cal::kGroupBlocks), dim3(cal::kBlock), 0, stream, v_, cfg.horizon,
                      1.0f / cfg.lookahead);
   hipLaunchKernelGGL(cal_fill_done_kernel, dim3(1), dim3(1), 0, stream, v_);
@@ -1031,7 +1147,7 @@ gpq_status LaqQueue::empty_all() {
 
 gpq_status LaqQueue::post_init() {
   if (!v_.wlog) return merge_publish();
-  hipLaunchKernelGGL(cal_post_init_kernel, dim3(partial_slots), dim3(kLaqBlock), 0, stream, v_, partial);
+  hipLaunchKernelGGL(cal_post_init_kernel, dim3(partial_slots), dim3(kLaqBlock), 0, stream, v_, groups_, partial);
   hipLaunchKernelGGL(cal_init_publish_kernel, dim3(1), dim3(1024), 0, stream, partial, partial_slots, ws,
                      cfg.lookahead, cfg.horizon);
   GPQ_HIP(hipGetLastError());
@@ -1094,8 +1210,12 @@ gpq_status LaqQueue::enable_alt_stage() {
 gpq_status LaqQueue::pending(uint64_t* n) {
   if (v_.wlog) {
     GPQ_HIP(hipMemsetAsync(sum_, 0, sizeof(uint64_t), stream));
-    hipLaunchKernelGGL(cal_count_kernel, dim3(ceil_div(cfg.num_lps, 256)), dim3(256), 0, stream, v_,
-                       reinterpret_cast<unsigned long long*>(sum_));
+    if (groups_.units)
+      hipLaunchKernelGGL(cal_units_count_kernel, dim3(1024), dim3(256), 0, stream, v_, groups_,
+                         reinterpret_cast<unsigned long long*>(sum_));
+    else
+      hipLaunchKernelGGL(cal_count_kernel, dim3(ceil_div(cfg.num_lps, 256)), dim3(256), 0, stream, v_,
+                         reinterpret_cast<unsigned long long*>(sum_));
     GPQ_HIP(hipGetLastError());
     GPQ_HIP(hipMemcpyAsync(n, sum_, sizeof(uint64_t), hipMemcpyDeviceToHost, stream));
     GPQ_HIP(hipStreamSynchronize(stream));
@@ -1119,7 +1239,10 @@ gpq_status LaqQueue::pending(uint64_t* n) {
 gpq_status LaqQueue::calendar_gather(uint32_t lp, std::vector<Event>* out) {
   uint32_t* d_n = reinterpret_cast<uint32_t*>(gather_ + kGatherCap);
   GPQ_HIP(hipMemsetAsync(d_n, 0, sizeof(uint32_t), stream));
-  hipLaunchKernelGGL(cal_gather_kernel, dim3(1024), dim3(256), 0, stream, v_, lp, gather_, kGatherCap, d_n);
+  if (groups_.units)
+    hipLaunchKernelGGL(cal_units_gather_kernel, dim3(1024), dim3(256), 0, stream, v_, groups_, lp, gather_, kGatherCap, d_n);
+  else
+    hipLaunchKernelGGL(cal_gather_kernel, dim3(1024), dim3(256), 0, stream, v_, lp, gather_, kGatherCap, d_n);
   GPQ_HIP(hipGetLastError());
   uint32_t n = 0;
   GPQ_HIP(hipMemcpyAsync(&n, d_n, 4, hipMemcpyDeviceToHost, stream));
