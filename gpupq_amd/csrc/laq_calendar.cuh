@@ -38,7 +38,6 @@ namespace cal {
 constexpr int kBlock = 256;
 constexpr uint32_t kLpMost = 64;  // events of one LP in one window
 constexpr uint32_t kPer = 4;      // events of one thread in a pass over the log
-constexpr uint32_t kPassCap = kPer * kBlock;   // events a commit block takes at once
 constexpr int kGroupBlocks = 2048;        // blocks of the standalone filing launch
 constexpr uint32_t kStepListBlocks = 32;  // blocks of a step that move the beyond-the-calendar events
 
@@ -161,6 +160,156 @@ __device__ __forceinline__ Event successor(const FusedModel& m, uint32_t lp, uin
   return Event{f_to_bits(t_new), dst, local, m.init_per_lp + n};
 }
 
+// ---- the parts of a commit that every size of calendar shares ---------------------------------
+// U threads, one per LP, take a window's events from one log, U * PER at a time.
+template <int U, uint32_t PER>
+struct CommitLds {
+  static constexpr uint32_t kPass = U * PER;
+  uint32_t cnt[U], off[U + 1], fill[U], n0[U];         // per LP: events, their first place, and its count before
+  uint32_t ts[kPass], src[kPass], seq[kPass];          // the events of the pass in LP order, then in key order
+  uint16_t lp[kPass];
+  uint32_t wave[U / kWave];
+};
+
+// The log's n events counted per LP, the counts' prefix sum, and with n <= kPass the events placed in
+// LP order; e[0 .. loaded) hold the thread's first ones already.  Returns the events of the
+// thread's LP.  cnt is clear before, and the caller synchronizes after.
+template <int U, uint32_t PER>
+__device__ __forceinline__ uint32_t group_log(CommitLds<U, PER>& s, const LaqView& q, const Event* lg, uint32_t n,
+                                              uint32_t lp0, Event* e, uint32_t loaded) {
+  const uint32_t t = threadIdx.x;
+  uint32_t l[PER], k[PER];
+#pragma unroll
+  for (uint32_t j = 0; j < PER; ++j) {
+    const uint32_t i = t + j * U;
+    l[j] = U;
+    k[j] = 0;
+    if (i < n) {
+      if (j >= loaded) e[j] = load_event(&lg[i]);
+      l[j] = e[j].dst - lp0;                           // < U: these LPs only
+      if (l[j] < (uint32_t)U) k[j] = atomicAdd(&s.cnt[l[j]], 1u);
+      else atomicOr(&q.ws->error, kErrBadState);
+    }
+  }
+  for (uint32_t i = t + CommitLds<U, PER>::kPass; i < n; i += U) {
+    const uint32_t x = lg[i].dst - lp0;
+    if (x < (uint32_t)U) atomicAdd(&s.cnt[x], 1u);
+    else atomicOr(&q.ws->error, kErrBadState);
+  }
+  __syncthreads();
+  const uint32_t mine = s.cnt[t];
+  if (mine > kLpMost) atomicOr(&q.ws->error, kErrStageOverflow);
+  uint32_t inc = mine;
+#pragma unroll
+  for (int off = 1; off < kWave; off <<= 1) {
+    const uint32_t y = (uint32_t)__shfl_up((int)inc, off, kWave);
+    if (lane_id() >= off) inc += y;
+  }
+  if (lane_id() == kWave - 1) s.wave[t / kWave] = inc;
+  __syncthreads();
+  for (uint32_t w = 0; w < t / kWave; ++w) inc += s.wave[w];
+  s.off[t + 1u] = inc;
+  if (t == 0) s.off[0] = 0u;
+  __syncthreads();
+  if (n <= CommitLds<U, PER>::kPass) {                 // from registers
+#pragma unroll
+    for (uint32_t j = 0; j < PER; ++j) {
+      if (l[j] >= (uint32_t)U) continue;
+      const uint32_t p = s.off[l[j]] + k[j];
+      s.ts[p] = e[j].ts;
+      s.src[p] = e[j].src;
+      s.seq[p] = e[j].seq;
+      s.lp[p] = (uint16_t)l[j];
+    }
+  }
+  return mine;
+}
+
+// The pass over the LPs from `first` on: *last past its last LP.  A log of more than kPass events is
+// taken in several, each over the LPs whose events fit; false when LP `first` alone does not (it was
+// refused: kPass > kLpMost), and the caller goes on with the next one.  Uniform; the caller
+// synchronizes after.
+template <int U, uint32_t PER>
+__device__ __forceinline__ bool begin_pass(CommitLds<U, PER>& s, uint32_t n, uint32_t first, uint32_t* last) {
+  const uint32_t t = threadIdx.x;
+  *last = U;
+  if (n <= CommitLds<U, PER>::kPass) return true;
+  *last = first + (uint32_t)__syncthreads_count(t >= first && s.off[t + 1u] - s.off[first] <= CommitLds<U, PER>::kPass);
+  s.fill[t] = 0u;
+  return *last != first;
+}
+
+// With n > kPass: the pass's events from the log into LP order.
+template <int U, uint32_t PER>
+__device__ __forceinline__ void fill_pass(CommitLds<U, PER>& s, const Event* lg, uint32_t n, uint32_t lp0, uint32_t first,
+                                          uint32_t last) {
+  if (n <= CommitLds<U, PER>::kPass) return;
+  __syncthreads();
+  for (uint32_t i = threadIdx.x; i < n; i += U) {
+    const Event x = load_event(&lg[i]);
+    const uint32_t xl = x.dst - lp0;
+    if (xl < first || xl >= last) continue;
+    const uint32_t p = s.off[xl] - s.off[first] + atomicAdd(&s.fill[xl], 1u);
+    s.ts[p] = x.ts;
+    s.src[p] = x.src;
+    s.seq[p] = x.seq;
+    s.lp[p] = (uint16_t)xl;
+  }
+}
+
+// A thread per event: its rank among its LP's events, and the events moved into key order.  The
+// caller synchronizes before and after.
+template <int U, uint32_t PER>
+__device__ __forceinline__ void order_pass(CommitLds<U, PER>& s, uint32_t base, uint32_t take) {
+  const uint32_t t = threadIdx.x;
+  uint32_t ets[PER], esrc[PER], eseq[PER], to[PER];
+#pragma unroll
+  for (uint32_t j = 0; j < PER; ++j) {
+    const uint32_t p = t + j * U;
+    if (p >= take) continue;
+    const uint32_t el = s.lp[p], o = s.off[el] - base, kk = s.cnt[el];
+    ets[j] = s.ts[p];
+    esrc[j] = s.src[p];
+    eseq[j] = s.seq[p];
+    uint32_t rank = 0;
+    for (uint32_t i = 0; i < kk; ++i) {
+      const uint32_t ot = s.ts[o + i];
+      bool before = ot < ets[j];
+      if (ot == ets[j] && o + i != p) {                // equal times: by source, then number, then arrival
+        const uint32_t os = s.src[o + i], oq = s.seq[o + i];
+        before = os != esrc[j] ? os < esrc[j] : (oq != eseq[j] ? oq < eseq[j] : o + i < p);
+      }
+      rank += before ? 1u : 0u;
+    }
+    to[j] = o + rank;
+  }
+  __syncthreads();                                     // every rank is taken
+#pragma unroll
+  for (uint32_t j = 0; j < PER; ++j) {
+    if (t + j * U >= take) continue;
+    s.ts[to[j]] = ets[j];
+    s.src[to[j]] = esrc[j];
+    s.seq[to[j]] = eseq[j];
+  }
+}
+
+// A thread per LP: the trace hash over its k events in key order, at place o.
+template <int U, uint32_t PER>
+__device__ __forceinline__ uint64_t hash_events(const CommitLds<U, PER>& s, const LaqView& q, const FusedModel& m, uint32_t lp,
+                                                uint32_t o, uint32_t k, uint64_t h) {
+  uint32_t prev = m.last_ts ? m.last_ts[lp] : 0u;
+  for (uint32_t i = 0; i < k; ++i) {
+    const uint32_t xt = s.ts[o + i];
+    h = trace_step(h, xt, s.src[o + i], s.seq[o + i]);
+    if (m.last_ts) {
+      if (xt < prev) atomicOr(&q.ws->error, kErrBadState);
+      prev = xt;
+    }
+  }
+  if (m.last_ts && k) m.last_ts[lp] = prev;
+  return h;
+}
+
 // Commit block `blk` of step c (window c).  The block's log of the window is grouped by LP in LDS
 // (a count per LP, its prefix sum, the records in LP order), and then worked on event by event, a
 // thread per event: its rank among its LP's events (compared one by one: three on average),
@@ -170,7 +319,7 @@ __device__ __forceinline__ Event successor(const FusedModel& m, uint32_t lp, uin
 // self-addressed ones) and one for a list take a rank in the block's LDS count of their window or
 // list, one thread per window and list reserves the block's run, and they are written into
 // the runs; a successor for another block goes to that block's log by its own atomic.  The log is
-// emptied at the end.  A log of more than kPassCap records is taken in passes over ranges of LPs.
+// emptied at the end.  A log of more than kPer events per thread is taken in passes over ranges of LPs.
 //
 // What bounds it: the atomics on the logs' counters, which are performed at the memory side at 26.6
 // G/s whatever lines they meet on: 1.7 M per step at 2^20 LPs x 32 events, 64 us of its 126.
@@ -181,13 +330,9 @@ __device__ __forceinline__ Event successor(const FusedModel& m, uint32_t lp, uin
 __device__ __forceinline__ void commit_block(const LaqView& q, const FusedModel& m, float end_time, float inv, uint32_t c,
                                              uint32_t blk) {
   __shared__ uint32_t sw[kCalMaxWindows];
-  __shared__ uint32_t s_cnt[kBlock], s_off[kBlock + 1], s_fill[kBlock], s_n0[kBlock];
-  __shared__ uint32_t s_ts[kPassCap], s_src[kPassCap], s_seq[kPassCap];
-  __shared__ uint8_t s_lp[kPassCap];
-  __shared__ uint32_t s_wave[kBlock / kWave];
+  __shared__ CommitLds<kBlock, kPer> s;
   __shared__ uint32_t s_lcnt[2], s_lbase[2];
   __shared__ uint32_t s_wcnt[kCalMaxWindows], s_wbase[kCalMaxWindows];
-  static_assert(kBlock <= 256, "an LP's index in its block fits a byte");
   const uint32_t t = threadIdx.x;
   const uint32_t lp0 = blk << q.cal_block_log2;
   const uint32_t lp = lp0 + t;
@@ -206,132 +351,26 @@ __device__ __forceinline__ void commit_block(const LaqView& q, const FusedModel&
   load_windows(q, c, sw);
   const uint32_t B = q.cal_windows;
   const uint32_t end_bits = f_to_bits(end_time);
-  s_cnt[t] = 0u;
-  s_n0[t] = cnt_pre;
+  s.cnt[t] = 0u;
+  s.n0[t] = cnt_pre;
   __syncthreads();
   const uint32_t n = n0 < q.cal_sub_cap ? n0 : q.cal_sub_cap;
-  uint32_t l[kPer], k[kPer];
-#pragma unroll
-  for (uint32_t j = 0; j < kPer; ++j) {
-    const uint32_t i = t + j * kBlock;
-    l[j] = kBlock;
-    k[j] = 0;
-    if (i < n) {
-      if (j >= 2u) e[j] = load_event(&lg[i]);
-      l[j] = e[j].dst - lp0;                           // < kBlock: this block's LPs only
-      if (l[j] < (uint32_t)kBlock) k[j] = atomicAdd(&s_cnt[l[j]], 1u);
-      else atomicOr(&q.ws->error, kErrBadState);
+  const uint32_t mine = group_log(s, q, lg, n, lp0, e, 2u);
+  for (uint32_t first = 0, last; first < (uint32_t)kBlock; first = last) {   // one pass unless the log is long
+    if (!begin_pass(s, n, first, &last)) {
+      ++last;
+      continue;
     }
-  }
-  for (uint32_t i = t + kPassCap; i < n; i += kBlock) {
-    const uint32_t x = lg[i].dst - lp0;
-    if (x < (uint32_t)kBlock) atomicAdd(&s_cnt[x], 1u);
-    else atomicOr(&q.ws->error, kErrBadState);
-  }
-  __syncthreads();
-  const uint32_t mine = s_cnt[t];                      // events of the thread's LP
-  if (mine > kLpMost) atomicOr(&q.ws->error, kErrStageOverflow);
-  uint32_t inc = mine;
-#pragma unroll
-  for (int off = 1; off < kWave; off <<= 1) {
-    const uint32_t y = (uint32_t)__shfl_up((int)inc, off, kWave);
-    if (lane_id() >= off) inc += y;
-  }
-  if (lane_id() == kWave - 1) s_wave[t / kWave] = inc;
-  __syncthreads();
-  for (uint32_t w = 0; w < t / kWave; ++w) inc += s_wave[w];
-  s_off[t + 1u] = inc;
-  if (t == 0) s_off[0] = 0u;
-  __syncthreads();
-  const bool whole = n <= kPassCap;
-  if (whole) {                                         // the records into LP order, from registers
-#pragma unroll
-    for (uint32_t j = 0; j < kPer; ++j) {
-      if (l[j] >= (uint32_t)kBlock) continue;
-      const uint32_t p = s_off[l[j]] + k[j];
-      s_ts[p] = e[j].ts;
-      s_src[p] = e[j].src;
-      s_seq[p] = e[j].seq;
-      s_lp[p] = (uint8_t)l[j];
-    }
-  }
-  for (uint32_t first = 0; first < (uint32_t)kBlock;) {   // one pass unless the log is longer than kPassCap
-    uint32_t last = kBlock;
-    const uint32_t base = s_off[first];
-    if (!whole) {                                      // the LPs from `first` on whose events fit
-      last = first + (uint32_t)__syncthreads_count(t >= first && s_off[t + 1u] - base <= kPassCap);
-      if (last == first) {                             // an LP of more than kPassCap > kLpMost events: refused above
-        ++first;
-        continue;
-      }
-      s_fill[t] = 0u;
-    }
-    const uint32_t take = s_off[last] - base;
+    const uint32_t base = s.off[first], take = s.off[last] - base;
     for (uint32_t i = t; i < B; i += kBlock) s_wcnt[i] = 0u;
     if (t < 2) s_lcnt[t] = 0u;
-    if (!whole) {
-      __syncthreads();
-      for (uint32_t i = t; i < n; i += kBlock) {
-        const Event x = load_event(&lg[i]);
-        const uint32_t xl = x.dst - lp0;
-        if (xl < first || xl >= last) continue;
-        const uint32_t p = s_off[xl] - base + atomicAdd(&s_fill[xl], 1u);
-        s_ts[p] = x.ts;
-        s_src[p] = x.src;
-        s_seq[p] = x.seq;
-        s_lp[p] = (uint8_t)xl;
-      }
-    }
+    fill_pass(s, lg, n, lp0, first, last);
     __syncthreads();
-    // a thread per event: its rank among its LP's events
-    {
-      uint32_t ets[kPer], esrc[kPer], eseq[kPer], to[kPer];
-#pragma unroll
-      for (uint32_t j = 0; j < kPer; ++j) {
-        const uint32_t p = t + j * kBlock;
-        if (p >= take) continue;
-        const uint32_t el = s_lp[p], o = s_off[el] - base, kk = s_cnt[el];
-        ets[j] = s_ts[p];
-        esrc[j] = s_src[p];
-        eseq[j] = s_seq[p];
-        uint32_t rank = 0;
-        for (uint32_t i = 0; i < kk; ++i) {
-          const uint32_t ot = s_ts[o + i];
-          bool before = ot < ets[j];
-          if (ot == ets[j] && o + i != p) {            // equal times: by source, then number, then arrival
-            const uint32_t os = s_src[o + i], oq = s_seq[o + i];
-            before = os != esrc[j] ? os < esrc[j] : (oq != eseq[j] ? oq < eseq[j] : o + i < p);
-          }
-          rank += before ? 1u : 0u;
-        }
-        to[j] = o + rank;
-      }
-      __syncthreads();                                 // every rank is taken; the records move into key order
-#pragma unroll
-      for (uint32_t j = 0; j < kPer; ++j) {
-        if (t + j * kBlock >= take) continue;
-        s_ts[to[j]] = ets[j];
-        s_src[to[j]] = esrc[j];
-        s_seq[to[j]] = eseq[j];
-      }
-    }
+    order_pass(s, base, take);
     __syncthreads();
-    // a thread per LP: the trace hash
     if (in_range && mine && t >= first && t < last) {
-      uint64_t h = h_pre;
-      uint32_t prev = m.last_ts ? m.last_ts[lp] : 0u;
-      const uint32_t o = s_off[t] - base;
-      for (uint32_t i = 0; i < mine; ++i) {
-        const uint32_t xt = s_ts[o + i];
-        h = trace_step(h, xt, s_src[o + i], s_seq[o + i]);
-        if (m.last_ts) {
-          if (xt < prev) atomicOr(&q.ws->error, kErrBadState);
-          prev = xt;
-        }
-      }
+      m.hash[lp] = hash_events(s, q, m, lp, s.off[t] - base, mine, h_pre);
       m.count[lp] = cnt_pre + mine;
-      m.hash[lp] = h;
-      if (m.last_ts) m.last_ts[lp] = prev;
     }
     __syncthreads();                                   // the events' words now hold their successors
     // a thread per event, one after the other (side by side they take 108 registers, four waves per
@@ -339,26 +378,26 @@ __device__ __forceinline__ void commit_block(const LaqView& q, const FusedModel&
     // block's run of that window or list
 #pragma unroll 1
     for (uint32_t p = t; p < take; p += kBlock) {
-      const uint32_t el = s_lp[p], elp = lp0 + el;
+      const uint32_t el = s.lp[p], elp = lp0 + el;
       uint32_t way = Route::kNone;
       if (elp < q.num_lps && elp - m.base < m.lps) {
-        const Event sc = successor(m, elp, s_n0[el] + (p - (s_off[el] - base)), s_ts[p]);
+        const Event sc = successor(m, elp, s.n0[el] + (p - (s.off[el] - base)), s.ts[p]);
         const uint32_t r = route_of(sw, B, sc.ts, end_bits, 1u, inv);
-        s_ts[p] = sc.ts;
-        s_src[p] = sc.dst;
+        s.ts[p] = sc.ts;
+        s.src[p] = sc.dst;
         if (r >= kCalMaxWindows) way = r | (atomicAdd(&s_lcnt[r == Route::kParked ? 1u : 0u], 1u) << 16);
         else if ((sc.dst >> q.cal_block_log2) == blk) way = r | (atomicAdd(&s_wcnt[r], 1u) << 16);
         else way = r | kRemote;
       }
-      s_seq[p] = way;
+      s.seq[p] = way;
     }
     // successors for other blocks' logs: every slot atomic of the thread in flight at once
     uint32_t pos[kPer];
 #pragma unroll
     for (uint32_t j = 0; j < kPer; ++j) {
       const uint32_t p = t + j * kBlock;
-      const uint32_t way = p < take ? s_seq[p] : (uint32_t)Route::kNone;
-      pos[j] = way & kRemote ? atomicAdd(log_count(q, c + (way & 0xFFFu), s_src[p] >> q.cal_block_log2), 1u) : 0u;
+      const uint32_t way = p < take ? s.seq[p] : (uint32_t)Route::kNone;
+      pos[j] = way & kRemote ? atomicAdd(log_count(q, c + (way & 0xFFFu), s.src[p] >> q.cal_block_log2), 1u) : 0u;
     }
     __syncthreads();
     // one run per window (this block's own log) and per list for the block
@@ -371,22 +410,22 @@ __device__ __forceinline__ void commit_block(const LaqView& q, const FusedModel&
       s_lbase[t] = x ? atomicAdd(list_count(q, c & 1u, t ? Route::kParked : Route::kOver), x) : 0u;
     }
     auto record = [&](uint32_t p) {
-      const uint32_t el = s_lp[p];
-      return make_uint4(s_ts[p], s_src[p], lp0 + el - m.base, m.init_per_lp + s_n0[el] + (p - (s_off[el] - base)));
+      const uint32_t el = s.lp[p];
+      return make_uint4(s.ts[p], s.src[p], lp0 + el - m.base, m.init_per_lp + s.n0[el] + (p - (s.off[el] - base)));
     };
 #pragma unroll
     for (uint32_t j = 0; j < kPer; ++j) {
       const uint32_t p = t + j * kBlock;
-      const uint32_t way = p < take ? s_seq[p] : (uint32_t)Route::kNone;
+      const uint32_t way = p < take ? s.seq[p] : (uint32_t)Route::kNone;
       if (!(way & kRemote)) continue;
       if (pos[j] < q.cal_sub_cap)
-        *reinterpret_cast<uint4*>(log_base(q, c + (way & 0xFFFu), s_src[p] >> q.cal_block_log2) + pos[j]) = record(p);
+        *reinterpret_cast<uint4*>(log_base(q, c + (way & 0xFFFu), s.src[p] >> q.cal_block_log2) + pos[j]) = record(p);
       else
         atomicOr(&q.ws->error, kErrQueueOverflow);
     }
     __syncthreads();
     for (uint32_t p = t; p < take; p += kBlock) {
-      const uint32_t way = s_seq[p], r = way & 0xFFFu, rank = way >> 16;
+      const uint32_t way = s.seq[p], r = way & 0xFFFu, rank = way >> 16;
       if ((way & kRemote) || r == Route::kNone) continue;
       if (r < kCalMaxWindows) {
         const uint32_t i = s_wbase[r] + rank;
@@ -396,8 +435,7 @@ __device__ __forceinline__ void commit_block(const LaqView& q, const FusedModel&
         list_store(q, c & 1u, r, s_lbase[r == Route::kParked ? 1u : 0u] + rank, record(p));
       }
     }
-    first = last;
-    if (first < (uint32_t)kBlock) __syncthreads();     // the next pass clears the counts
+    if (last < (uint32_t)kBlock) __syncthreads();      // the next pass clears the counts
   }
   if (t == 0) *log_count(q, c, blk) = 0u;              // the block's log of window c is consumed
 }

@@ -49,10 +49,7 @@ __device__ __forceinline__ uint32_t* unit_count(const LaqView& q, const Groups& 
 __device__ __forceinline__ void commit_unit(const LaqView& q, const Groups& g, const FusedModel& m, float end_time,
                                             float inv, uint32_t c, uint32_t unit) {
   __shared__ uint32_t sw[kCalMaxWindows];
-  __shared__ uint32_t s_cnt[kUnit], s_off[kUnit + 1], s_fill[kUnit], s_n0[kUnit];
-  __shared__ uint32_t s_ts[kUnitPass], s_src[kUnitPass], s_seq[kUnitPass];
-  __shared__ uint16_t s_lp[kUnitPass];
-  __shared__ uint32_t s_wave[kUnit / kWave];
+  __shared__ CommitLds<kUnit, kUnitPer> s;
   __shared__ uint32_t s_wcnt[kCalMaxWindows], s_wbase[kCalMaxWindows];
   __shared__ uint32_t s_gcnt[kMaxGroups], s_goff[kMaxGroups];
   __shared__ uint32_t s_pcnt, s_pbase;
@@ -71,150 +68,44 @@ __device__ __forceinline__ void commit_unit(const LaqView& q, const Groups& g, c
   load_windows(q, c, sw);
   const uint32_t B = q.cal_windows;
   const uint32_t end_bits = f_to_bits(end_time);
-  s_cnt[t] = 0u;
-  s_n0[t] = cnt_pre;
+  s.cnt[t] = 0u;
+  s.n0[t] = cnt_pre;
   __syncthreads();
   const uint32_t n = n0 < g.log_cap ? n0 : g.log_cap;
-  uint32_t l[kUnitPer], k[kUnitPer];
-#pragma unroll
-  for (uint32_t j = 0; j < kUnitPer; ++j) {
-    const uint32_t i = t + j * kUnit;
-    l[j] = kUnit;
-    k[j] = 0;
-    if (i < n) {
-      if (j >= 2u) e[j] = load_event(&lg[i]);
-      l[j] = e[j].dst - lp0;                           // < kUnit: this unit's LPs only
-      if (l[j] < (uint32_t)kUnit) k[j] = atomicAdd(&s_cnt[l[j]], 1u);
-      else atomicOr(&q.ws->error, kErrBadState);
-    }
-  }
-  for (uint32_t i = t + kUnitPass; i < n; i += kUnit) {
-    const uint32_t x = lg[i].dst - lp0;
-    if (x < (uint32_t)kUnit) atomicAdd(&s_cnt[x], 1u);
-    else atomicOr(&q.ws->error, kErrBadState);
-  }
-  __syncthreads();
-  const uint32_t mine = s_cnt[t];                      // events of the thread's LP
-  if (mine > kLpMost) atomicOr(&q.ws->error, kErrStageOverflow);
-  uint32_t inc = mine;
-#pragma unroll
-  for (int off = 1; off < kWave; off <<= 1) {
-    const uint32_t y = (uint32_t)__shfl_up((int)inc, off, kWave);
-    if (lane_id() >= off) inc += y;
-  }
-  if (lane_id() == kWave - 1) s_wave[t / kWave] = inc;
-  __syncthreads();
-  for (uint32_t w = 0; w < t / kWave; ++w) inc += s_wave[w];
-  s_off[t + 1u] = inc;
-  if (t == 0) s_off[0] = 0u;
-  __syncthreads();
-  const bool whole = n <= kUnitPass;
-  if (whole) {                                         // the records into LP order, from registers
-#pragma unroll
-    for (uint32_t j = 0; j < kUnitPer; ++j) {
-      if (l[j] >= (uint32_t)kUnit) continue;
-      const uint32_t p = s_off[l[j]] + k[j];
-      s_ts[p] = e[j].ts;
-      s_src[p] = e[j].src;
-      s_seq[p] = e[j].seq;
-      s_lp[p] = (uint16_t)l[j];
-    }
-  }
+  const uint32_t mine = group_log(s, q, lg, n, lp0, e, 2u);
   uint32_t pass = 0;
-  for (uint32_t first = 0; first < (uint32_t)kUnit && n;) {   // one pass unless the log is longer than kUnitPass
-    uint32_t last = kUnit;
-    const uint32_t base = s_off[first];
-    if (!whole) {                                      // the LPs from `first` on whose events fit
-      last = first + (uint32_t)__syncthreads_count(t >= first && s_off[t + 1u] - base <= kUnitPass);
-      if (last == first) {                             // an LP of more than kUnitPass > kLpMost events: refused above
-        ++first;
-        continue;
-      }
-      s_fill[t] = 0u;
+  for (uint32_t first = 0, last; first < (uint32_t)kUnit && n; first = last) {   // one pass unless the log is long
+    if (!begin_pass(s, n, first, &last)) {
+      ++last;
+      continue;
     }
     if (pass >= g.passes) {                            // only after an LP was refused: others fill their passes
       if (t == 0) atomicOr(&q.ws->error, kErrStageOverflow);
       break;
     }
-    const uint32_t take = s_off[last] - base;
+    const uint32_t base = s.off[first], take = s.off[last] - base;
     if (t < B) s_wcnt[t] = 0u;
     if (t < kMaxGroups) s_gcnt[t] = 0u;
     if (t == 0) s_pcnt = 0u;
     static_assert(kCalMaxWindows <= (uint32_t)kUnit && kMaxGroups <= (uint32_t)kUnit, "one thread clears each count");
-    if (!whole) {
-      __syncthreads();
-      for (uint32_t i = t; i < n; i += kUnit) {
-        const Event x = load_event(&lg[i]);
-        const uint32_t xl = x.dst - lp0;
-        if (xl < first || xl >= last) continue;
-        const uint32_t p = s_off[xl] - base + atomicAdd(&s_fill[xl], 1u);
-        s_ts[p] = x.ts;
-        s_src[p] = x.src;
-        s_seq[p] = x.seq;
-        s_lp[p] = (uint16_t)xl;
-      }
-    }
+    fill_pass(s, lg, n, lp0, first, last);
     __syncthreads();
-    // a thread per event: its rank among its LP's events
-    {
-      uint32_t ets[kUnitPer], esrc[kUnitPer], eseq[kUnitPer], to[kUnitPer];
-#pragma unroll
-      for (uint32_t j = 0; j < kUnitPer; ++j) {
-        const uint32_t p = t + j * kUnit;
-        if (p >= take) continue;
-        const uint32_t el = s_lp[p], o = s_off[el] - base, kk = s_cnt[el];
-        ets[j] = s_ts[p];
-        esrc[j] = s_src[p];
-        eseq[j] = s_seq[p];
-        uint32_t rank = 0;
-        for (uint32_t i = 0; i < kk; ++i) {
-          const uint32_t ot = s_ts[o + i];
-          bool before = ot < ets[j];
-          if (ot == ets[j] && o + i != p) {            // equal times: by source, then number, then arrival
-            const uint32_t os = s_src[o + i], oq = s_seq[o + i];
-            before = os != esrc[j] ? os < esrc[j] : (oq != eseq[j] ? oq < eseq[j] : o + i < p);
-          }
-          rank += before ? 1u : 0u;
-        }
-        to[j] = o + rank;
-      }
-      __syncthreads();                                 // every rank is taken; the records move into key order
-#pragma unroll
-      for (uint32_t j = 0; j < kUnitPer; ++j) {
-        if (t + j * kUnit >= take) continue;
-        s_ts[to[j]] = ets[j];
-        s_src[to[j]] = esrc[j];
-        s_seq[to[j]] = eseq[j];
-      }
-    }
+    order_pass(s, base, take);
     __syncthreads();
-    // a thread per LP: the trace hash
     if (in_range && mine && t >= first && t < last) {
-      uint64_t h = h_pre;
-      uint32_t prev = m.last_ts ? m.last_ts[lp] : 0u;
-      const uint32_t o = s_off[t] - base;
-      for (uint32_t i = 0; i < mine; ++i) {
-        const uint32_t xt = s_ts[o + i];
-        h = trace_step(h, xt, s_src[o + i], s_seq[o + i]);
-        if (m.last_ts) {
-          if (xt < prev) atomicOr(&q.ws->error, kErrBadState);
-          prev = xt;
-        }
-      }
+      m.hash[lp] = hash_events(s, q, m, lp, s.off[t] - base, mine, h_pre);
       m.count[lp] = cnt_pre + mine;
-      m.hash[lp] = h;
-      if (m.last_ts) m.last_ts[lp] = prev;
     }
     __syncthreads();                                   // the events' words now hold their successors
     // a thread per event: the successor's time and destination, and its way with its rank on it
 #pragma unroll 1
     for (uint32_t p = t; p < take; p += kUnit) {
-      const uint32_t el = s_lp[p], elp = lp0 + el;
+      const uint32_t el = s.lp[p], elp = lp0 + el;
       uint32_t way = Route::kNone;
       if (elp < q.num_lps && elp - m.base < m.lps) {
-        const Event sc = successor(m, elp, s_n0[el] + (p - (s_off[el] - base)), s_ts[p]);
-        s_ts[p] = sc.ts;
-        s_src[p] = sc.dst;
+        const Event sc = successor(m, elp, s.n0[el] + (p - (s.off[el] - base)), s.ts[p]);
+        s.ts[p] = sc.ts;
+        s.src[p] = sc.dst;
         if (!(sc.ts < end_bits)) {
           way = Route::kParked | (atomicAdd(&s_pcnt, 1u) << 16);
         } else {
@@ -228,7 +119,7 @@ __device__ __forceinline__ void commit_unit(const LaqView& q, const Groups& g, c
           }
         }
       }
-      s_seq[p] = way;
+      s.seq[p] = way;
     }
     __syncthreads();
     if (t < B) {                                       // the unit's runs in its own logs
@@ -268,10 +159,10 @@ __device__ __forceinline__ void commit_unit(const LaqView& q, const Groups& g, c
     if (t < kMaxGroups) g.parts[slot * kMaxGroups + t] = s_goff[t] | (s_gcnt[t] << 16);
     Event* out = g.out + slot * kUnitPass;
     for (uint32_t p = t; p < take; p += kUnit) {
-      const uint32_t way = s_seq[p], r = way & 0xFFFu, rank = way >> 16;
+      const uint32_t way = s.seq[p], r = way & 0xFFFu, rank = way >> 16;
       if (!(way & kToGroup) && r == Route::kNone) continue;
-      const uint32_t el = s_lp[p];
-      const uint4 ne = make_uint4(s_ts[p], s_src[p], lp0 + el - m.base, m.init_per_lp + s_n0[el] + (p - (s_off[el] - base)));
+      const uint32_t el = s.lp[p];
+      const uint4 ne = make_uint4(s.ts[p], s.src[p], lp0 + el - m.base, m.init_per_lp + s.n0[el] + (p - (s.off[el] - base)));
       if (way & kToGroup) {
         *reinterpret_cast<uint4*>(out + s_goff[r] + rank) = ne;
       } else if (r < kCalMaxWindows) {
@@ -283,8 +174,7 @@ __device__ __forceinline__ void commit_unit(const LaqView& q, const Groups& g, c
       }
     }
     ++pass;
-    first = last;
-    if (first < (uint32_t)kUnit) __syncthreads();      // the next pass clears the counts
+    if (last < (uint32_t)kUnit) __syncthreads();       // the next pass clears the counts
   }
   if (n == 0 && t < kMaxGroups) g.parts[(size_t)unit * g.passes * kMaxGroups + t] = 0u;   // an empty first part
   if (t == 0) {
