@@ -127,6 +127,8 @@ class GaqQueue final : public QueueBase {
   uint32_t tile_ = kMergeTile;  // records per merge block
 };
 
+struct HqHeap;   // one heap's device arrays (queue_hq.hip)
+
 class HqQueue final : public QueueBase {
  public:
   explicit HqQueue(const gpq_queue_config& c) : QueueBase(c) {}
@@ -143,19 +145,28 @@ class HqQueue final : public QueueBase {
 
  private:
   gpq_status step(bool select);
-  gpq_status merge_root(uint32_t h, hipStream_t s);
+  gpq_status merge_root(uint32_t h, bool select, hipStream_t s);
   gpq_status step_heap(uint32_t h, bool select, hipStream_t s);
+  template <typename Op>
+  gpq_status merges(uint32_t h, const Op& op, uint32_t ntasks, uint64_t max_total, hipStream_t s) const;
+  HqHeap heap(uint32_t h) const;
+  size_t dirty_words() const { return 2 * (size_t)slots_ + 4; }   // both lists and their three counts
+  const Event* node_at(uint32_t v, uint32_t slot) const;   // v over every heap
   gpq_status snapshot(std::vector<Event>* out, std::vector<uint32_t>* counts);
   HqView v_{};
   uint32_t r_ = 0, nodes_ = 0, levels_ = 0, slots_ = 1, depth_ = 0;
+  uint32_t chunks_ = 0, spares_ = 0;        // insert chunks of a step; node slots beyond the nodes
   uint32_t heaps_ = 1, lps_per_heap_ = 0;   // nodes_ is per heap
   uint64_t mcap_ = 0;                       // merged-buffer records per heap
   size_t scratch_n_ = 0, tasks_n_ = 0;      // per-heap sizes of scratch_ and tasks_
   std::vector<hipStream_t> hs_;             // one stream per heap (several heaps only)
   std::vector<hipEvent_t> ev_;              // joins of both phases, then the two forks
   Event* nodes_buf_ = nullptr;
+  uint32_t* slot_ = nullptr;    // by node: where its records are
+  uint32_t* spare_ = nullptr;
+  uint32_t* ticket_ = nullptr;
   uint32_t* counts_ = nullptr;
-  uint8_t* dirty_ = nullptr;
+  uint32_t* dirty_ = nullptr;   // the lists of a delete-update
   Event* sort_[2] = {nullptr, nullptr};
   uint32_t* order_ = nullptr;   // sample order of the insert sort
   Event* merged_ = nullptr;
@@ -163,17 +174,16 @@ class HqQueue final : public QueueBase {
   Event* carry_ = nullptr;
   Event* chunk_buf_ = nullptr;
   Event* tmp2_ = nullptr;
-  Event* tmp1_ = nullptr;
   uint32_t* first_ = nullptr;
   uint32_t* scratch_ = nullptr;
   MergeTask* tasks_ = nullptr;
+  MergeTask* second_ = nullptr; // the parents' merges of a delete-update level
+  uint32_t* second_v_ = nullptr;
   uint32_t* splits_ = nullptr;  // merge-path splits, split_stride_ words per task slot
   uint32_t split_stride_ = 0;
   uint32_t* seg_pre_ = nullptr; // per heap, segment offsets of the step's striped inserts
   uint64_t* sum_ = nullptr;
   uint32_t tile_ = kMergeTile;  // records per merge block
-  // the split buffer of task slot t (tasks_ + t)
-  uint32_t* splits_of(const MergeTask* t) const { return splits_ + (size_t)(t - tasks_) * split_stride_; }
 };
 
 }  // namespace gpq

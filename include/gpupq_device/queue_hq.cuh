@@ -4,7 +4,7 @@
 // post :1609-1719, partition :478-547, delete-update :631-784, insert-update :817-960,
 // copy_last :975-1094).
 //
-// HBM layout: nodes[v * r + i] (node v, position i), counts[v]; the step's inserts are
+// HBM layout: store[slot[v] * r + i] (node v, position i), counts[v]; the step's inserts are
 // appended to enq; queue_post leaves the next step's safe events in deq (peek slot = position).
 #pragma once
 
@@ -26,11 +26,10 @@ struct HqState {
   uint32_t pad[3];
   Event bound;             // the root's largest record while nodes exist below the root
   const Event* mptr;       // = merged buffer (pointer slot for the selection)
-  // insert-update chunks: target node, size, current data pointer, next data pointer
+  // insert-update chunks: target node, size, first record among the carried ones
   uint32_t chunk_target[kHqMaxChunks];
   uint32_t chunk_n[kHqMaxChunks];
-  const Event* chunk_ptr[kHqMaxChunks];
-  Event* chunk_alt[kHqMaxChunks];
+  uint32_t chunk_off[kHqMaxChunks];
 };
 
 // Several heaps (HQ_NUM_QUEUES): heap h owns the LPs [h * lps_per_heap, (h + 1) * lps_per_heap),
