@@ -114,7 +114,7 @@ gpq_status GaqQueue::init() {
   split_stride_ = merge_split_words(cap, tile_);
   GPQ_TRY(arena.alloc(&splits_, split_stride_));
   GPQ_TRY(arena.alloc(&first_, cfg.num_lps));
-  GPQ_TRY(arena.alloc(&scratch_, 2 * (size_t)ceil_div(cap, 1024) + 2));
+  GPQ_TRY(arena.alloc(&scratch_, ceil_div(cap, 1024)));
   v_.ws = ws;
   partial_slots = 1;
   GPQ_TRY(arena.alloc(&partial, 1));

@@ -544,7 +544,7 @@ gpq_status HqQueue::init() {
   GPQ_TRY(arena.alloc(&seg_pre_, (size_t)heaps_ * (kInsertStripes + 2)));
   GPQ_HIP(hipMemsetAsync(v_.seg_m, 0, sizeof(uint32_t) * heaps_ * kStripeCounterWords, stream));
   // working buffers, one set per heap so that the heaps' steps can run concurrently
-  scratch_n_ = 2 * (size_t)ceil_div(mcap_, 1024) + 2;
+  scratch_n_ = ceil_div(mcap_, 1024);
   tasks_n_ = spares_;   // the tasks of one launch
   GPQ_TRY(arena.alloc(&sort_[0], (size_t)heaps_ * enq_cap));
   GPQ_TRY(arena.alloc(&sort_[1], (size_t)heaps_ * enq_cap));

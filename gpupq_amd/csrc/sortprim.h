@@ -73,8 +73,8 @@ uint32_t merge_split_words(uint64_t max_total, uint32_t tile);
 // ts < *d_wend and key <= *d_bound (when *d_bound_valid) is scanned, the first record of
 // each LP in it is moved to `deq` (in order, count -> *d_deq_n) and the others to `rest`
 // (in order, count -> *d_rest_n); *d_prefix receives the prefix length.  `first` (one
-// u32 per LP, all 0xFFFFFFFF between calls) and `scratch` (>= 2 * ceil(cap / 1024) + 2
-// u32) are workspace; `acct` (optional) receives the prefix length.  Reference:
+// u32 per LP, all 0xFFFFFFFF between calls) and `scratch` (>= ceil(cap / 1024) u32)
+// are workspace; `acct` (optional) receives the prefix length.  Reference:
 // src/global_array_queue.cu:147-179 (serial scan) and src/heap_queue.cu:478-547 (atomicMin
 // per LP).
 struct SelectBufs {

@@ -10,7 +10,8 @@ namespace {
 
 constexpr int kThreads = 256;                       // selection blocks; merge blocks: kT of 128, 256 or
                                                     // 512 threads (tiles of 8 kT records)
-constexpr uint32_t kSelectTile = 1024;              // records per selection block (256 x 4)
+constexpr uint32_t kSelectTile = 1024;              // records per selection tile (256 threads x 4)
+constexpr uint32_t kSelectBlocks = 1024;            // blocks of a selection launch, at most
 constexpr uint32_t kSplitLanes = 8;                 // lanes per tile boundary in the merge partition
 
 __device__ __forceinline__ Event sentinel() { return Event{0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu}; }
@@ -560,161 +561,138 @@ __device__ __forceinline__ bool in_prefix(const Event& e, uint32_t wend, bool bo
   return e.ts < wend && (!bounded || !key_less(bound, e));
 }
 
-__global__ void select_prefix_kernel(const Event* const* d_s, const uint32_t* d_n, const uint32_t* d_wend, const Event* d_bound,
-                                     const uint32_t* d_bound_valid, uint32_t* d_prefix) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  const Event* s = *d_s;
-  const uint32_t n = *d_n, wend = *d_wend;
-  const bool bounded = d_bound_valid && *d_bound_valid;
-  const Event bound = bounded ? *d_bound : sentinel();
-  uint32_t lo = 0, hi = n;
+// The length of the prefix, by one wave: 64 probes a round.
+__device__ __forceinline__ uint32_t wave_prefix(const Event* s, uint32_t n, uint32_t wend, bool bounded, const Event& bound) {
+  uint32_t lo = 0, hi = n;                             // the prefix ends in [lo, hi]
   while (lo < hi) {
-    const uint32_t mid = (lo + hi) >> 1;
-    if (in_prefix(load_event(s + mid), wend, bounded, bound)) lo = mid + 1u; else hi = mid;
+    const uint32_t step = (hi - lo + kWave - 1u) / kWave, i = lo + (uint32_t)lane_id() * step;
+    const uint64_t out = __ballot(i < hi && !in_prefix(load_event(s + (i < hi ? i : lo)), wend, bounded, bound));
+    if (out == 0) {
+      lo = lo + (hi - lo - 1u) / step * step + 1u;     // past the last probe
+    } else {
+      const uint32_t f = (uint32_t)__ffsll((unsigned long long)out) - 1u;
+      hi = lo + f * step;
+      if (f) lo = lo + (f - 1u) * step + 1u;
+    }
   }
-  *d_prefix = lo;
+  return lo;
 }
 
-__global__ void select_mark_kernel(const Event* const* d_s, const uint32_t* d_prefix, uint32_t* first) {
+// Each block finds the prefix's length for itself (four rounds of loads; as a launch of its own, by
+// one thread's binary search, it took 6 us), and marks the first record of every LP in it.
+__global__ __launch_bounds__(kThreads) void select_mark_kernel(const Event* const* d_s, const uint32_t* d_n,
+                                                               const uint32_t* d_wend, const Event* d_bound,
+                                                               const uint32_t* d_bound_valid, uint32_t* d_prefix,
+                                                               uint32_t* first) {
+  __shared__ uint32_t s_p;
   const Event* s = *d_s;
-  const uint32_t p = *d_prefix;
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < p; i += gridDim.x * blockDim.x)
-    atomicMin(&first[s[i].dst], i);
+  if (threadIdx.x < (uint32_t)kWave) {
+    const bool bounded = d_bound_valid && *d_bound_valid;
+    const Event bound = bounded ? *d_bound : sentinel();
+    const uint32_t p = wave_prefix(s, *d_n, *d_wend, bounded, bound);
+    if (threadIdx.x == 0) {
+      s_p = p;
+      if (blockIdx.x == 0) *d_prefix = p;
+    }
+  }
+  __syncthreads();
+  const uint32_t p = s_p;
+  for (uint32_t i = blockIdx.x * kThreads + threadIdx.x; i < p; i += gridDim.x * kThreads) atomicMin(&first[s[i].dst], i);
 }
 
+// The marked records of every tile of the prefix.
 __global__ __launch_bounds__(kThreads) void select_count_kernel(const Event* const* d_s, const uint32_t* d_prefix,
                                                                 const uint32_t* first, uint32_t* counts) {
   __shared__ uint32_t s_w[kThreads / kWave];
   const Event* s = *d_s;
   const uint32_t p = *d_prefix;
-  const uint32_t base = blockIdx.x * kSelectTile;
-  uint32_t c = 0;
-  if (base < p) {
-    for (uint32_t i = base + threadIdx.x; i < base + kSelectTile && i < p; i += kThreads)
-      c += first[s[i].dst] == i ? 1u : 0u;
-  }
-  c = wave_sum_u32(c);
-  if (lane_id() == 0) s_w[threadIdx.x / kWave] = c;
-  __syncthreads();
-  if (threadIdx.x == 0) counts[blockIdx.x] = s_w[0] + s_w[1] + s_w[2] + s_w[3];
-}
-
-// Exclusive scan of counts[0:nb) into offsets[0:nb), nb = the blocks that hold the scanned
-// prefix (the count and scatter kernels do nothing past it); totals of marked / rest.  The
-// counts are read in sweeps of kScanRounds x 1024: element r * 1024 + t of a sweep goes to
-// thread t (coalesced, all loads of a sweep in flight together); each (round, wave) pair's
-// total goes to LDS and one wave scans those totals in order.
-constexpr int kScanRounds = 8;
-__global__ __launch_bounds__(1024) void select_scan_kernel(const uint32_t* counts, uint32_t* offsets, uint32_t nblk,
-                                                           const uint32_t* d_prefix, uint32_t* d_deq_n,
-                                                           uint32_t* d_rest_n) {
-  constexpr uint32_t kWaves = 1024 / kWave;
-  constexpr uint32_t kParts = kScanRounds * kWaves;          // (round, wave) totals per sweep
-  static_assert(kParts % kWave == 0, "whole parts per lane");
-  __shared__ uint32_t s_part[kParts];
-  __shared__ uint32_t s_total;
-  const uint32_t p = *d_prefix;
-  const uint32_t want = (uint32_t)(((uint64_t)p + kSelectTile - 1) / kSelectTile);
-  const uint32_t nb = want < nblk ? want : nblk;
-  const uint32_t lane = (uint32_t)lane_id(), wv = threadIdx.x / kWave;
-  uint32_t carry = 0;
-  for (uint32_t base = 0; base < nb; base += kScanRounds * 1024u) {
-    uint32_t v[kScanRounds];
+  for (uint32_t tile = blockIdx.x; (uint64_t)tile * kSelectTile < p; tile += gridDim.x) {
+    const uint32_t base = tile * kSelectTile;
+    uint32_t c = 0;
 #pragma unroll
-    for (int r = 0; r < kScanRounds; ++r) {
-      const uint32_t i = base + (uint32_t)r * 1024u + threadIdx.x;
-      v[r] = i < nb ? counts[i] : 0u;
+    for (uint32_t q = 0; q < kSelectTile / kThreads; ++q) {
+      const uint32_t i = base + q * kThreads + threadIdx.x, x = i < p ? i : base;
+      c += first[s[x].dst] == i ? 1u : 0u;             // i >= p is no record's place
     }
-#pragma unroll
-    for (int r = 0; r < kScanRounds; ++r) {   // v[r] becomes the exclusive prefix inside the wave
-      uint32_t x = v[r];
-      for (int off = 1; off < kWave; off <<= 1) {
-        const uint32_t y = (uint32_t)__shfl_up((int)x, off, kWave);
-        if ((int)lane >= off) x += y;
-      }
-      if (lane == kWave - 1) s_part[r * kWaves + wv] = x;
-      v[r] = x - v[r];
-    }
+    c = wave_sum_u32(c);
+    if (lane_id() == 0) s_w[threadIdx.x / kWave] = c;
     __syncthreads();
-    if (wv == 0) {   // exclusive scan of the parts in (round, wave) order, kParts / 64 per lane
-      constexpr uint32_t kPer = kParts / kWave;
-      uint32_t sum = 0;
-#pragma unroll
-      for (uint32_t u = 0; u < kPer; ++u) sum += s_part[lane * kPer + u];
-      uint32_t x = sum;
-      for (int off = 1; off < kWave; off <<= 1) {
-        const uint32_t y = (uint32_t)__shfl_up((int)x, off, kWave);
-        if ((int)lane >= off) x += y;
-      }
-      uint32_t run = x - sum;
-#pragma unroll
-      for (uint32_t u = 0; u < kPer; ++u) {
-        const uint32_t c = s_part[lane * kPer + u];
-        s_part[lane * kPer + u] = run;
-        run += c;
-      }
-      if (lane == kWave - 1) s_total = x;
-    }
+    if (threadIdx.x == 0) counts[tile] = s_w[0] + s_w[1] + s_w[2] + s_w[3];
     __syncthreads();
-#pragma unroll
-    for (int r = 0; r < kScanRounds; ++r) {
-      const uint32_t i = base + (uint32_t)r * 1024u + threadIdx.x;
-      if (i < nb) offsets[i] = carry + s_part[r * kWaves + wv] + v[r];
-    }
-    carry += s_total;
-    __syncthreads();   // s_part and s_total are rewritten by the next sweep
-  }
-  if (threadIdx.x == 0) {
-    *d_deq_n = carry;
-    *d_rest_n = p - carry;
   }
 }
 
+// The prefix's records to deq and rest, a tile at a time; a block adds up the counts of the tiles
+// before its own (as a launch of its own the scan of all counts took 5 us, which is more than the
+// reading of a few hundred words by every block), and the one with the last tile publishes the totals.
 __global__ __launch_bounds__(kThreads) void select_scatter_kernel(const Event* const* d_s, const uint32_t* d_prefix,
-                                                                  uint32_t* first, const uint32_t* offsets,
-                                                                  Event* deq, Event* rest) {
-  __shared__ uint32_t s_w[kThreads / kWave];
+                                                                  uint32_t* first, const uint32_t* counts,
+                                                                  Event* deq, Event* rest, uint32_t* d_deq_n,
+                                                                  uint32_t* d_rest_n) {
+  constexpr uint32_t kWaves = kThreads / kWave;
+  __shared__ uint32_t s_w[kWaves], s_c[kWaves];
   const Event* s = *d_s;
   const uint32_t p = *d_prefix;
-  const uint32_t base = blockIdx.x * kSelectTile;
-  if (base >= p) return;
   constexpr uint32_t kItems = kSelectTile / kThreads;   // 4 consecutive records per thread
-  const uint32_t i0 = base + threadIdx.x * kItems;
-  bool mark[kItems];
-  Event e[kItems];
-  uint32_t mine = 0;
+  const uint32_t wv = threadIdx.x / kWave;
+  uint32_t earlier = 0, counted = 0;                    // marked records of the tiles before `counted`
+  for (uint32_t tile = blockIdx.x; (uint64_t)tile * kSelectTile < p; tile += gridDim.x) {
+    uint32_t c = 0;
+    for (uint32_t i = counted + threadIdx.x; i < tile; i += kThreads) c += counts[i];
+    counted = tile;
+    const uint32_t i0 = tile * kSelectTile + threadIdx.x * kItems;
+    bool mark[kItems];
+    Event e[kItems];
+    uint32_t mine = 0;
 #pragma unroll
-  for (uint32_t q = 0; q < kItems; ++q) {
-    const uint32_t i = i0 + q;
-    mark[q] = false;
-    if (i < p) {
-      e[q] = load_event(s + i);
-      mark[q] = first[e[q].dst] == i;
+    for (uint32_t q = 0; q < kItems; ++q) {
+      const uint32_t i = i0 + q;
+      e[q] = load_event(s + (i < p ? i : p - 1u));
+    }
+#pragma unroll
+    for (uint32_t q = 0; q < kItems; ++q) {
+      mark[q] = first[e[q].dst] == i0 + q;              // i >= p is no record's place
       mine += mark[q] ? 1u : 0u;
     }
-  }
-  uint32_t x = mine;   // inclusive scan over the block, in thread order
-  for (int off = 1; off < kWave; off <<= 1) {
-    const uint32_t y = (uint32_t)__shfl_up((int)x, off, kWave);
-    if (lane_id() >= off) x += y;
-  }
-  if (lane_id() == kWave - 1) s_w[threadIdx.x / kWave] = x;
-  __syncthreads();
-  uint32_t wave_off = 0;
-  for (uint32_t w = 0; w < threadIdx.x / kWave; ++w) wave_off += s_w[w];
-  uint32_t before = offsets[blockIdx.x] + wave_off + x - mine;   // marked records before i0
+    uint32_t x = mine;   // inclusive scan over the block, in thread order
+    for (int off = 1; off < kWave; off <<= 1) {
+      const uint32_t y = (uint32_t)__shfl_up((int)x, off, kWave);
+      if (lane_id() >= off) x += y;
+    }
+    c = wave_sum_u32(c);
+    if (lane_id() == kWave - 1) s_w[wv] = x;
+    if (lane_id() == 0) s_c[wv] = c;
+    __syncthreads();
+    uint32_t in_tile = 0, wave_off = 0;
 #pragma unroll
-  for (uint32_t q = 0; q < kItems; ++q) {
-    const uint32_t i = i0 + q;
-    if (i < p) {
-      if (mark[q]) {
-        store_event(deq + before, e[q]);
-        first[e[q].dst] = 0xFFFFFFFFu;
-        ++before;
-      } else {
-        store_event(rest + (i - before), e[q]);
+    for (uint32_t w = 0; w < kWaves; ++w) {
+      earlier += s_c[w];
+      if (w < wv) wave_off += s_w[w];
+      in_tile += s_w[w];
+    }
+    uint32_t before = earlier + wave_off + x - mine;   // marked records before i0
+#pragma unroll
+    for (uint32_t q = 0; q < kItems; ++q) {
+      const uint32_t i = i0 + q;
+      if (i < p) {
+        if (mark[q]) {
+          store_event(deq + before, e[q]);
+          first[e[q].dst] = 0xFFFFFFFFu;
+          ++before;
+        } else {
+          store_event(rest + (i - before), e[q]);
+        }
       }
     }
+    if (threadIdx.x == 0 && (uint64_t)(tile + 1u) * kSelectTile >= p) {
+      *d_deq_n = earlier + in_tile;
+      *d_rest_n = p - (earlier + in_tile);
+    }
+    __syncthreads();                                   // s_w and s_c are rewritten
+  }
+  if (p == 0 && blockIdx.x == 0 && threadIdx.x == 0) {
+    *d_deq_n = 0;
+    *d_rest_n = 0;
   }
 }
 
@@ -816,16 +794,12 @@ gpq_status select_safe(const Event* const* s, const uint32_t* d_n, uint32_t cap,
                        Event* rest, hipStream_t stream, unsigned long long* acct) {
   const uint32_t nblk = grid_of(cap, kSelectTile);
   uint32_t* counts = b.scratch;
-  uint32_t* offsets = b.scratch + nblk;
-  hipLaunchKernelGGL(select_prefix_kernel, dim3(1), dim3(64), 0, stream, s, d_n, d_wend, d_bound, d_bound_valid,
-                     b.d_prefix);
-  hipLaunchKernelGGL(select_mark_kernel, dim3(grid_of(cap, kThreads) < 4096 ? grid_of(cap, kThreads) : 4096),
-                     dim3(kThreads), 0, stream, s, b.d_prefix, b.first);
-  hipLaunchKernelGGL(select_count_kernel, dim3(nblk), dim3(kThreads), 0, stream, s, b.d_prefix, b.first, counts);
-  hipLaunchKernelGGL(select_scan_kernel, dim3(1), dim3(1024), 0, stream, counts, offsets, nblk, b.d_prefix, b.d_deq_n,
-                     b.d_rest_n);
-  hipLaunchKernelGGL(select_scatter_kernel, dim3(nblk), dim3(kThreads), 0, stream, s, b.d_prefix, b.first, offsets, deq,
-                     rest);
+  const uint32_t blocks = std::min(nblk, kSelectBlocks);
+  hipLaunchKernelGGL(select_mark_kernel, dim3(std::min(grid_of(cap, kThreads), kSelectBlocks)), dim3(kThreads), 0, stream,
+                     s, d_n, d_wend, d_bound, d_bound_valid, b.d_prefix, b.first);
+  hipLaunchKernelGGL(select_count_kernel, dim3(blocks), dim3(kThreads), 0, stream, s, b.d_prefix, b.first, counts);
+  hipLaunchKernelGGL(select_scatter_kernel, dim3(blocks), dim3(kThreads), 0, stream, s, b.d_prefix, b.first, counts, deq,
+                     rest, b.d_deq_n, b.d_rest_n);
   GPQ_HIP(hipGetLastError());
   if (acct) {
     hipLaunchKernelGGL(acct_count_kernel, dim3(1), dim3(64), 0, stream, b.d_prefix, cap, acct);
