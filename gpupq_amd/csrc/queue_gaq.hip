@@ -27,31 +27,23 @@ __global__ void gaq_init_kernel(GaqState* st, Event* fel0, Event* fel1, uint32_t
     st->prefix = 0;
     st->deq_n = 0;
     st->rest_n = 0;
-    st->selected = 0;
-    st->n_next = 0;
     *ws = WindowState{kInfBits, 0u, 0u, 0u, 0ull, 0u, 0u};
   }
 }
 
-__global__ void gaq_mark_selected_kernel(GaqState* st) { st->selected = 1; }
-
-// Builds the merge task: (unselected prefix ++ rest of the array) with the sorted inserts.
-__global__ void gaq_plan_kernel(GaqState* st, MergeTask* task, const Event* sorted_ins, Event* rest, uint32_t cap,
-                                uint32_t enq_cap, WindowState* ws) {
+// Builds the merge task -- (unselected prefix ++ rest of the array) with the sorted inserts -- and what
+// is known before it runs: the buffers' swap, the new length, and the window, which starts at the
+// smallest of three first records.  (A launch after the merge for these, and one after the selection to
+// say that there was one, took 3 us each.)
+__global__ void gaq_plan_kernel(GaqState* st, MergeTask* task, const Event* sorted_ins, const Event* rest, uint32_t cap,
+                                uint32_t enq_cap, WindowState* ws, float lookahead, float horizon) {
   const uint32_t m = st->m < enq_cap ? st->m : enq_cap;
-  Event* live = st->fel[st->cur];
+  const uint32_t cur = st->cur, prefix = st->prefix;
   MergeTask t{};
-  if (st->selected) {
-    t.a1 = rest;
-    t.n_a1 = st->rest_n;
-    t.a2 = live + st->prefix;
-    t.n_a2 = st->n - st->prefix;
-  } else {
-    t.a1 = live;
-    t.n_a1 = st->n;
-    t.a2 = live;
-    t.n_a2 = 0;
-  }
+  t.a1 = rest;
+  t.n_a1 = st->rest_n;                            // 0 and 0 when nothing was selected
+  t.a2 = st->fel[cur] + prefix;
+  t.n_a2 = st->n - prefix;
   t.b = sorted_ins;
   t.n_b = m;
   uint64_t total = (uint64_t)t.n_a1 + t.n_a2 + t.n_b;
@@ -60,22 +52,18 @@ __global__ void gaq_plan_kernel(GaqState* st, MergeTask* task, const Event* sort
     t.n_b = 0;                                    // keep the array, drop the inserts
     total = (uint64_t)t.n_a1 + t.n_a2;
   }
-  t.out[0] = t.out[1] = t.out[2] = st->fel[st->cur ^ 1u];
+  t.out[0] = t.out[1] = t.out[2] = st->fel[cur ^ 1u];
   t.end[0] = t.end[1] = t.end[2] = (uint32_t)total;
   *task = t;
-  st->n_next = (uint32_t)total;
+  const uint32_t a = t.n_a1 ? t.a1[0].ts : (t.n_a2 ? t.a2[0].ts : kInfBits), b = t.n_b ? t.b[0].ts : kInfBits;
+  st->cur = cur ^ 1u;
+  st->front = st->fel[cur ^ 1u];
+  st->n = (uint32_t)total;
   st->m = 0;
+  st->prefix = 0;
+  st->rest_n = 0;
   st->deq_n = 0;
-  st->selected = 0;
-}
-
-// Swaps the live buffer and publishes gmin = first record, wend, done.
-__global__ void gaq_finish_kernel(GaqState* st, WindowState* ws, float lookahead, float horizon) {
-  st->cur ^= 1u;
-  st->n = st->n_next;
-  const Event* live = st->fel[st->cur];
-  st->front = live;
-  const uint32_t g = st->n ? live[0].ts : kInfBits;
+  const uint32_t g = a < b ? a : b;
   float wend = bits_to_f(g) + lookahead;
   if (horizon < wend) wend = horizon;
   ws->gmin = g;
@@ -127,11 +115,7 @@ gpq_status GaqQueue::init() {
 gpq_status GaqQueue::pre() {
   GaqState* st = v_.st;
   const SelectBufs b{first_, scratch_, &st->prefix, &st->deq_n, &st->rest_n};
-  GPQ_TRY(select_safe(&st->front, &st->n, cap_, &ws->wend, nullptr, nullptr, b, v_.deq, rest_, stream,
-                      acct(kStatSelected)));
-  hipLaunchKernelGGL(gaq_mark_selected_kernel, dim3(1), dim3(1), 0, stream, st);
-  GPQ_HIP(hipGetLastError());
-  return GPQ_OK;
+  return select_safe(&st->front, &st->n, cap_, &ws->wend, nullptr, nullptr, b, v_.deq, rest_, stream, acct(kStatSelected));
 }
 
 gpq_status GaqQueue::post() {
@@ -139,12 +123,10 @@ gpq_status GaqQueue::post() {
   GPQ_TRY(gather_inserts(v_.seg_m, v_.seg_cap, v_.enq_cap, v_.enq_cap, seg_pre_, &v_.st->m, ws, stream));
   GPQ_TRY(sort_records(v_.enq, sort_[0], sort_[1], order_, &v_.st->m, v_.enq_cap, stream, acct(kStatSorted), seg_pre_,
                        v_.seg_cap));
-  hipLaunchKernelGGL(gaq_plan_kernel, dim3(1), dim3(1), 0, stream, v_.st, task_, sorted, rest_, cap_, v_.enq_cap, ws);
+  hipLaunchKernelGGL(gaq_plan_kernel, dim3(1), dim3(1), 0, stream, v_.st, task_, sorted, rest_, cap_, v_.enq_cap, ws,
+                     cfg.lookahead, cfg.horizon);
   GPQ_HIP(hipGetLastError());
-  GPQ_TRY(merge_tasks(task_, 1, (uint64_t)cap_, stream, tile_, acct(kStatMerged), splits_, split_stride_));
-  hipLaunchKernelGGL(gaq_finish_kernel, dim3(1), dim3(1), 0, stream, v_.st, ws, cfg.lookahead, cfg.horizon);
-  GPQ_HIP(hipGetLastError());
-  return GPQ_OK;
+  return merge_tasks(task_, 1, (uint64_t)cap_, stream, tile_, acct(kStatMerged), splits_, split_stride_);
 }
 
 gpq_status GaqQueue::snapshot(std::vector<Event>* out) {
@@ -162,7 +144,7 @@ gpq_status GaqQueue::pending(uint64_t* n) {
   GaqState st;
   GPQ_HIP(hipMemcpyAsync(&st, v_.st, sizeof(st), hipMemcpyDeviceToHost, stream));
   GPQ_HIP(hipStreamSynchronize(stream));
-  *n = st.n - (st.selected ? st.deq_n : 0u);   // records handed out by queue_pre are gone
+  *n = st.n - st.deq_n;   // records handed out by queue_pre are gone
   return GPQ_OK;
 }
 

@@ -19,11 +19,10 @@ struct GaqState {
   uint32_t cur;
   uint32_t n;           // records in fel[cur]
   uint32_t m;           // inserts of this step (totalled over the stripes by queue_post)
-  uint32_t prefix;      // records scanned by the last selection
+  // of the selection, from queue_pre to queue_post; 0 outside
+  uint32_t prefix;      // records scanned
   uint32_t deq_n;       // records in the dequeue buffer
   uint32_t rest_n;      // unselected records of the scanned prefix
-  uint32_t selected;    // 1 between queue_pre and queue_post
-  uint32_t n_next;
 };
 
 struct GaqView {
