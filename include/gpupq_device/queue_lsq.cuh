@@ -46,51 +46,93 @@ struct LsqView {
     __device__ __forceinline__ Event key(uint32_t t) const { return load_event(&it[t]); }
 
     // Simple top-down splay of key k in the tree rooted at t; ties descend left, as the
-    // reference does (`i <= t->item`).  The header node is kept in registers.
+    // reference does (`i <= t->item`).  The header node is kept in registers, and so are the key and the links
+    // of the current node and of the child it descends to, loaded together: what bounds a splay is the
+    // chain of loads, one per level so, where a load for each key and each link made two to four.
     __device__ uint32_t splay(const Event& k, uint32_t t) {
       if (t == kNil) return t;
       uint32_t hl = kNil, hr = kNil;   // header's left / right
       uint32_t l = kNil, r = kNil;     // kNil here means "the header"
+      Event kt = key(t);
+      uint2 lt = ln[t];
       for (;;) {
         ++visits;
-        if (!key_less(key(t), k)) {                  // k <= t
-          uint32_t tl = L(t);
-          if (tl == kNil) break;
-          if (key_less(k, key(tl))) {                 // rotate right
-            setL(t, R(tl));
-            setR(tl, t);
-            t = tl;
-            tl = L(t);
-            if (tl == kNil) break;
+        if (!key_less(kt, k)) {                       // k <= t
+          uint32_t c = lt.x;
+          if (c == kNil) break;
+          Event kc = key(c);
+          uint2 lc = ln[c];
+          if (key_less(k, kc)) {                      // rotate right
+            ln[t] = make_uint2(lc.y, lt.y);
+            lc.y = t;
+            setR(c, t);
+            t = c;
+            lt = lc;
+            c = lt.x;
+            if (c == kNil) break;
+            kc = key(c);
+            lc = ln[c];
           }
           if (r == kNil) hl = t; else setL(r, t);     // link right
           r = t;
-          t = tl;
+          t = c;
+          kt = kc;
+          lt = lc;
         } else {
-          uint32_t tr = R(t);
-          if (tr == kNil) break;
-          if (key_less(key(tr), k)) {                 // rotate left
-            setR(t, L(tr));
-            setL(tr, t);
-            t = tr;
-            tr = R(t);
-            if (tr == kNil) break;
+          uint32_t c = lt.y;
+          if (c == kNil) break;
+          Event kc = key(c);
+          uint2 lc = ln[c];
+          if (key_less(kc, k)) {                      // rotate left
+            ln[t] = make_uint2(lt.x, lc.x);
+            lc.x = t;
+            setL(c, t);
+            t = c;
+            lt = lc;
+            c = lt.y;
+            if (c == kNil) break;
+            kc = key(c);
+            lc = ln[c];
           }
           if (l == kNil) hr = t; else setR(l, t);     // link left
           l = t;
-          t = tr;
+          t = c;
+          kt = kc;
+          lt = lc;
         }
       }
-      if (l == kNil) hr = L(t); else setR(l, L(t));   // assemble
-      if (r == kNil) hl = R(t); else setL(r, R(t));
-      setL(t, hr);
-      setR(t, hl);
+      if (l == kNil) hr = lt.x; else setR(l, lt.x);   // assemble
+      if (r == kNil) hl = lt.y; else setL(r, lt.y);
+      ln[t] = make_uint2(hr, hl);
       return t;
     }
 
-    __device__ uint32_t leftmost(uint32_t t) {
+    // The splay of the smallest key: always to the left, so that no key is read.
+    __device__ uint32_t splay_min(uint32_t t) {
       if (t == kNil) return t;
-      while (L(t) != kNil) { t = L(t); ++visits; }
+      uint2 lt = ln[t];
+      if (lt.x == kNil) return t;
+      uint32_t hl = kNil, r = kNil;
+      for (;;) {
+        ++visits;
+        uint32_t c = lt.x;
+        if (c == kNil) break;
+        uint2 lc = ln[c];
+        ln[t] = make_uint2(lc.y, lt.y);               // rotate right
+        lc.y = t;
+        setR(c, t);
+        t = c;
+        lt = lc;
+        c = lt.x;
+        if (c == kNil) break;
+        lc = ln[c];
+        if (r == kNil) hl = t; else setL(r, t);       // link right
+        r = t;
+        t = c;
+        lt = lc;
+      }
+      if (r == kNil) hl = lt.y; else setL(r, lt.y);   // assemble
+      ln[t] = make_uint2(kNil, hl);
       return t;
     }
   };
@@ -103,32 +145,25 @@ struct LsqView {
   __device__ __forceinline__ int peek(Event** out, int lp) const {
     if (!(head[lp] < ws->wend)) return -1;
     Tree t = tree((uint32_t)lp);
-    const uint32_t rt = root[lp];
-    const uint32_t m = t.leftmost(rt);
-    const uint32_t nr = t.splay(t.key(m), rt);
+    const uint32_t nr = t.splay_min(root[lp]);
     root[lp] = nr;
     *out = item + (size_t)lp * cap + nr;
     return (int)((uint32_t)lp * cap + nr);
   }
 
   // queue_set_done: deletes the root placed there by peek (delete_min, src/local_splay_queue.cu:233-273).
+  // The next minimum is splayed to the root here, where it has to be found for the head in any case;
+  // a peek that follows finds it there.
   __device__ __forceinline__ void set_done(int index) const {
     const uint32_t lp = (uint32_t)index / cap;
     const uint32_t node = (uint32_t)index % cap;
     Tree t = tree(lp);
-    uint32_t x;
-    if (t.L(node) == kNil) {
-      x = t.R(node);
-    } else {                                           // equal keys to its left
-      x = t.splay(t.key(node), t.L(node));
-      t.setR(x, t.R(node));
-    }
+    const uint32_t x = t.splay_min(t.R(node));         // the minimum has no left child
     t.setL(node, freelist[lp]);                        // free_ (src/local_splay_queue.cu:96-104)
     freelist[lp] = node;
     root[lp] = x;
     len[lp] -= 1u;
-    const uint32_t m = t.leftmost(x);
-    head[lp] = m == kNil ? kInfBits : t.key(m).ts;
+    head[lp] = x == kNil ? kInfBits : t.key(x).ts;
   }
 
   // queue_clear: the whole pool of the LP becomes free again (src/local_splay_queue.cu:469-494).
