@@ -717,7 +717,13 @@ gpq_status AstarModel::step() {
     GPQ_HIP(hipGetLastError());
     return GPQ_OK;
   }));
-  GPQ_TRY(q->post());
+  const bool checked = q->set_search(&st->best, &st->done, &st->steps);
+  const gpq_status posted = q->post();
+  if (checked) {
+    q->set_search(nullptr, nullptr, nullptr);
+    return posted;
+  }
+  GPQ_TRY(posted);
   hipLaunchKernelGGL(astar_check_kernel, dim3(1), dim3(1), 0, q->stream, st, q->ws);
   GPQ_HIP(hipGetLastError());
   return GPQ_OK;

@@ -136,8 +136,16 @@ class QueueBase {
   // Number of queue_peek() slots the model iterates over.
   virtual uint32_t peek_slots() const { return cfg.num_lps; }
 
-  // Folds partial[0 .. partial_slots) into the window state (one small kernel on stream).
+  // Folds partial[0 .. partial_slots) into the window state (one small kernel on stream), unless
+  // the post kernel has published the window (alloc_partial, publish_args).
   gpq_status publish_window();
+  // partial[0 .. partial_slots), and the words by which up to kFoldMost blocks fold their minima in the
+  // post kernel itself.
+  gpq_status alloc_partial();
+  WindowPublish publish_args() const;
+  // A search's end, decided where the window is published: between set_search and the post.  False when the
+  // queue publishes it by a launch of its own.
+  bool set_search(const uint32_t* best, uint32_t* done, unsigned long long* steps);
   gpq_status window(WindowState* out);   // synchronous copy of the device window state
   gpq_status error_flags(uint32_t* flags);
   gpq_status stats_get(gpq_queue_stats* out);
@@ -153,6 +161,10 @@ class QueueBase {
   hipEvent_t profile_mark = nullptr;  // when set, recorded just before the window publication
   uint32_t* partial = nullptr;        // device, one slot per reduction block
   uint32_t partial_slots = 0;
+  uint32_t* fold = nullptr;           // device, two words after the partials; nullptr: publish by a launch
+  const uint32_t* search_best = nullptr;
+  uint32_t* search_done = nullptr;
+  unsigned long long* search_steps = nullptr;
   uint32_t threads = 256;
   // Work counters (device, kStatSlots u64) when cfg.collect_stats; nullptr otherwise.
   // Slots: 0 inserted, 1 displaced, 2 merged LPs, 3 scanned LPs, 4 aux bytes, 5 records

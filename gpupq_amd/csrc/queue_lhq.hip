@@ -10,7 +10,7 @@ namespace {
 
 constexpr int kLhqBlock = 256;
 
-__global__ __launch_bounds__(kLhqBlock) void lhq_post_kernel(LhqView q, uint32_t* partial) {
+__global__ __launch_bounds__(kLhqBlock) void lhq_post_kernel(LhqView q, uint32_t* partial, WindowPublish w) {
   const uint32_t lp = blockIdx.x * blockDim.x + threadIdx.x;
   uint32_t root = kInfBits;
   uint32_t inserted = 0, moves = 0;
@@ -51,7 +51,7 @@ __global__ __launch_bounds__(kLhqBlock) void lhq_post_kernel(LhqView q, uint32_t
     stats_add(q.stats, 2, inserted ? 1u : 0u);
     stats_add(q.stats, 3, lp < q.num_lps ? 1u : 0u);
   }
-  block_min_to_partial(root, partial);
+  block_min_publish(root, partial, w);
 }
 
 __global__ void lhq_init_kernel(LhqView q) {
@@ -93,7 +93,7 @@ gpq_status LhqQueue::init() {
   v_.ws = ws;
   v_.stats = stats;
   partial_slots = ceil_div(L, kLhqBlock);
-  GPQ_TRY(arena.alloc(&partial, partial_slots));
+  GPQ_TRY(alloc_partial());
   hipLaunchKernelGGL(lhq_init_kernel, dim3(ceil_div(L, 256)), dim3(256), 0, stream, v_);
   GPQ_HIP(hipGetLastError());
   return GPQ_OK;
@@ -106,7 +106,8 @@ gpq_status LhqQueue::empty_all() {
 }
 
 gpq_status LhqQueue::post() {
-  hipLaunchKernelGGL(lhq_post_kernel, dim3(partial_slots), dim3(kLhqBlock), 0, stream, v_, partial);
+  hipLaunchKernelGGL(lhq_post_kernel, dim3(partial_slots), dim3(kLhqBlock), 0, stream, v_, partial,
+                     publish_args());
   GPQ_HIP(hipGetLastError());
   return publish_window();
 }

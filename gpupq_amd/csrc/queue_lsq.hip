@@ -10,7 +10,7 @@ namespace {
 
 constexpr int kLsqBlock = 256;
 
-__global__ __launch_bounds__(kLsqBlock) void lsq_post_kernel(LsqView q, uint32_t* partial) {
+__global__ __launch_bounds__(kLsqBlock) void lsq_post_kernel(LsqView q, uint32_t* partial, WindowPublish w) {
   const uint32_t lp = blockIdx.x * blockDim.x + threadIdx.x;
   uint32_t minimum = kInfBits;
   uint32_t inserted = 0, visits = 0;
@@ -66,7 +66,7 @@ __global__ __launch_bounds__(kLsqBlock) void lsq_post_kernel(LsqView q, uint32_t
     stats_add(q.stats, 2, inserted ? 1u : 0u);
     stats_add(q.stats, 3, lp < q.num_lps ? 1u : 0u);
   }
-  block_min_to_partial(minimum, partial);
+  block_min_publish(minimum, partial, w);
 }
 
 // Rebuilds LP pools: every slot free, threaded in index order.
@@ -111,7 +111,7 @@ gpq_status LsqQueue::init() {
   v_.ws = ws;
   v_.stats = stats;
   partial_slots = ceil_div(L, kLsqBlock);
-  GPQ_TRY(arena.alloc(&partial, partial_slots));
+  GPQ_TRY(alloc_partial());
   hipLaunchKernelGGL(lsq_reset_kernel, dim3(4096), dim3(256), 0, stream, v_, 0u, L);
   hipLaunchKernelGGL(lsq_ws_init_kernel, dim3(1), dim3(1), 0, stream, ws);
   GPQ_HIP(hipGetLastError());
@@ -125,7 +125,8 @@ gpq_status LsqQueue::empty_all() {
 }
 
 gpq_status LsqQueue::post() {
-  hipLaunchKernelGGL(lsq_post_kernel, dim3(partial_slots), dim3(kLsqBlock), 0, stream, v_, partial);
+  hipLaunchKernelGGL(lsq_post_kernel, dim3(partial_slots), dim3(kLsqBlock), 0, stream, v_, partial,
+                     publish_args());
   GPQ_HIP(hipGetLastError());
   return publish_window();
 }
