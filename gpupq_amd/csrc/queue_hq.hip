@@ -43,13 +43,14 @@ __device__ __forceinline__ uint32_t depth_of(uint32_t v) { return 31u - __clz(v 
 
 // One heap's arrays.  Node v's records are at store + slot[v] * r; spare[0 .. spares) are the slots
 // that no node has: one per task of the widest delete-update level, then one per insert chunk.
+constexpr uint32_t kTickets = 8, kTicketWords = 32;
 struct HqHeap {
   HqState* st;
   uint32_t* counts;      // by node
   uint32_t* slot;
   uint32_t* spare;
   Event* store;
-  uint32_t* ticket;      // blocks of a launch that have planned; 0 between launches
+  uint32_t* ticket;      // kTickets + 1 counts of blocks that have planned, a line each; 0 between launches
   uint32_t* dirty;       // per parity of a level, `slots` nodes whose children are to be looked at
   uint32_t* dirty_n;     // ... and their number; dirty_n[2]: the tasks of `second`
   MergeTask* second;     // a level's merges of parents with their children
@@ -82,7 +83,7 @@ __global__ void hq_init_kernel(Heap p, uint32_t spares, uint32_t* first, uint32_
     HqState s{};
     s.mptr = merged;
     *p.st = s;
-    *p.ticket = 0;
+    for (uint32_t x = 0; x <= kTickets; ++x) p.ticket[x * kTicketWords] = 0;
     *p.ws = WindowState{kInfBits, 0u, 0u, 0u, 0ull, 0u, 0u};
   }
 }
@@ -410,7 +411,7 @@ __global__ __launch_bounds__(kT) void hq_merge_kernel(Op op) {
     }
     __syncthreads();
     // the plan's loads have returned: they decided what is in LDS
-    if (Op::kTicket && threadIdx.x == 0) ticket = atomicAdd(op.p.ticket, 1u);
+    if (Op::kTicket && threadIdx.x == 0) ticket = atomicAdd(&op.p.ticket[(1u + blockIdx.x % kTickets) * kTicketWords], 1u);
     const uint32_t all = first[kWave];
     for (uint32_t x = (blockIdx.x + gridDim.x - before % gridDim.x) % gridDim.x; x < all; x += gridDim.x) {
       uint32_t j = 0;                                  // the task of tile x: first[j] <= x < first[j + 1]
@@ -427,7 +428,15 @@ __global__ __launch_bounds__(kT) void hq_merge_kernel(Op op) {
   } while (g < n);
   if (threadIdx.x >= (uint32_t)kWave) return;
   if (Op::kTicket) {
-    if ((uint32_t)__shfl((int)ticket, 0, kWave) != gridDim.x - 1u) return;
+    // Counted on kTickets words and by the last of each on another one: atomics on one word take 30 ns
+    // each, one after the other.
+    const uint32_t c = blockIdx.x % kTickets, mine = (gridDim.x - c + kTickets - 1u) / kTickets;
+    if ((uint32_t)__shfl((int)ticket, 0, kWave) != mine - 1u) return;
+    if (lane == 0) {
+      op.p.ticket[(1u + c) * kTicketWords] = 0;
+      ticket = atomicAdd(op.p.ticket, 1u);
+    }
+    if ((uint32_t)__shfl((int)ticket, 0, kWave) != min(gridDim.x, kTickets) - 1u) return;
     if (lane == 0) *op.p.ticket = 0;
     commit_lane(op, lane, n, t[lane], k);
   } else if (blockIdx.x == 0 && lane == 0) {
@@ -489,7 +498,7 @@ uint32_t levels_with_children(uint32_t nodes) {
 HqHeap HqQueue::heap(uint32_t h) const {
   uint32_t* dirty = dirty_ + (size_t)h * dirty_words();
   return HqHeap{v_.st + h, counts_ + (size_t)h * nodes_, slot_ + (size_t)h * nodes_, spare_ + (size_t)h * spares_,
-                nodes_buf_ + (size_t)h * (nodes_ + spares_) * r_, ticket_ + h, dirty, dirty + 2 * (size_t)slots_,
+                nodes_buf_ + (size_t)h * (nodes_ + spares_) * r_, ticket_ + (size_t)h * (kTickets + 1) * kTicketWords, dirty, dirty + 2 * (size_t)slots_,
                 second_ + (size_t)h * slots_, second_v_ + (size_t)h * slots_, ws, acct(kStatMerged), r_, nodes_, slots_};
 }
 
@@ -534,7 +543,7 @@ gpq_status HqQueue::init() {
   GPQ_TRY(arena.alloc(&nodes_buf_, (size_t)heaps_ * (nodes_ + spares_) * r_));
   GPQ_TRY(arena.alloc(&slot_, (size_t)heaps_ * nodes_));
   GPQ_TRY(arena.alloc(&spare_, (size_t)heaps_ * spares_));
-  GPQ_TRY(arena.alloc(&ticket_, (size_t)heaps_));
+  GPQ_TRY(arena.alloc(&ticket_, (size_t)heaps_ * (kTickets + 1) * kTicketWords));
   GPQ_TRY(arena.alloc(&counts_, (size_t)heaps_ * nodes_));
   GPQ_TRY(arena.alloc(&dirty_, (size_t)heaps_ * dirty_words()));
   v_.seg_cap = insert_stripe_cap(enq_cap);
