@@ -85,8 +85,8 @@ gpq_status QueueBase::sum_u32(const uint32_t* d_values, uint32_t count, uint64_t
   return GPQ_OK;
 }
 
-// Up to this many blocks fold their minima by atomics on one word, which take 30 ns each one after the
-// other: binary heaps, 16 events per LP to time 10, 16,000 LPs (63 blocks) 6.2 ms and 6.9 with a launch
+// Up to this many blocks fold their minima by atomics on one word; the blocks of a post arrive there
+// together, and more of them wait longer than a launch takes: binary heaps, 16 events per LP to time 10, 16,000 LPs (63 blocks) 6.2 ms and 6.9 with a launch
 // that folds them, 32,000 (125) 7.1 and 7.3, 64,000 (250) 9.8 and 8.6.
 constexpr uint32_t kFoldMost = 128;
 
