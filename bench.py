@@ -283,7 +283,7 @@ QUEUE_GROUPS = {
     "lsq": ["post"],
 }
 GROUP_KERNELS = {
-    "sort": ("tile_sort_kernel", "merge_pass_kernel"),
+    "sort": ("tile_sort_kernel", "sample_rank_kernel", "bucket_merge_kernel"),
     "merge": ("merge_tasks_kernel",),
     "select": ("select_",),
 }
@@ -596,6 +596,15 @@ def traffic_from_profiles(kernel, workload):
     return None
 
 
+def step_traffic(kernel, workload):
+    """traffic_from_profiles of a step's launches: the filing launch of a large calendar belongs to it."""
+    t = traffic_from_profiles(kernel, workload)
+    if t is None or kernel != "phold_calendar_units_kernel":
+        return t
+    filing = traffic_from_profiles("cal_file_kernel", workload)
+    return None if filing is None else t + filing
+
+
 def copy_calibration():
     """A plain device copy of known size, for scaling the FETCH_SIZE / WRITE_SIZE counters."""
     import torch
@@ -752,10 +761,12 @@ def main():
         if args.queue == "laq" and dom == "queue_post":
             kname = "laq_post_far_kernel" if FAR else "laq_post_kernel"
         if dom == "merge_commit_step":
-            kname = "phold_calendar_kernel" if CAL else "phold_fused_kernel"
+            # a large calendar's step is two launches: cal_file_kernel files, the other commits
+            kname = ("phold_fused_kernel" if not CAL else "phold_calendar_units_kernel"
+                     if wl["num_lps"] >= 196608 else "phold_calendar_kernel")
         out = {"bound": "hbm", "kernel": dom, "kernel_symbol": kname, "achieved": k["gbps"], "peak": HBM_PEAK_GBPS,
                "unit": "GB/s", "frac": k["gbps"] / HBM_PEAK_GBPS,
-               "traffic": traffic_from_profiles(kname, args.workload),
+               "traffic": step_traffic(kname, args.workload),
                "alg_bytes_per_launch": k["alg_bytes"], "mean_launch_us": k["us"], "launches": k["launches"],
                "alg_bytes_model": ("88 B per committed event + 4 B per LP and step" if dom != "queue_post" else
                                    "sorted insert 16*(2k+2d) + 4 B per scanned LP head and per block partial"),

@@ -11,7 +11,9 @@
 //     logs of their windows and LP blocks;
 //   * a few list blocks: the events beyond the calendar (over[(c + 1) & 1]) whose window the
 //     calendar now reaches move into the logs.
-// No sorted run is kept, merged or shifted, and no separate pass groups the events by LP.
+// No sorted run is kept, merged or shifted, and no separate pass groups the events by LP.  Calendars of
+// LaqQueue::kGroupedMinLps LPs or more have logs with one writer instead (laq_calendar_groups.cuh); what the two
+// share is here.
 //
 // Layout (B = cal_windows, a power of two; L = num_lps; K = kBlock LPs per block):
 //   wlog   [B][blocks][sub_cap]  Event   window x, LP block b: count wlog_n[((x mod B) * blocks + b) * 16]
@@ -33,8 +35,8 @@ namespace gpq {
 namespace cal {
 
 // LPs per commit block, and so per log.  Smaller blocks mean more logs and shorter runs of the
-// self-addressed successors, larger ones fewer blocks in flight: at 2^20 LPs 64 LPs 1.37e10,
-// 128 LPs 1.59-1.66e10, 256 LPs 1.74-1.83e10, 512 LPs 1.60e10, 1024 LPs 1.42e10 events/s.
+// self-addressed successors, larger ones fewer blocks in flight: with a thread per LP and at 2^20 LPs, 64
+// LPs 1.37e10, 128 LPs 1.59-1.66e10, 256 LPs 1.74-1.83e10, 512 LPs 1.60e10, 1024 LPs 1.42e10 events/s.
 constexpr int kBlock = 256;
 constexpr uint32_t kLpMost = 64;  // events of one LP in one window
 constexpr uint32_t kPer = 4;      // events of one thread in a pass over the log

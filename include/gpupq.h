@@ -88,10 +88,12 @@ typedef struct {
   uint32_t calendar_windows;  /* LAQ calendar mode (0 = off; a power of two in [8, 256]; needs far_per_lp):
                                 for the PHOLD merge-and-commit step (drain 2) only, whose windows end one
                                 lookahead apart: one unsorted append log for each of the next
-                                calendar_windows windows and each block of 256 LPs, holding
+                                calendar_windows windows and each block of 256 LPs (512 from
+                                196608 LPs on), holding
                                 capacity_per_lp (<= 64) records per LP of the block; a step reads only
                                 the logs of the window it commits.  Events beyond the calendar wait in
-                                two lists, and events at or past the horizon in a parked list, of
+                                two lists (one per group of blocks from 196608 LPs on: the same room),
+                                and events at or past the horizon in a parked list, of
                                 num_lps * far_per_lp records each.  Same committed trace. */
   uint32_t sort_tile;         /* GAQ / HQ: records per block of the merge kernels:
                                 1024, 2048 or 4096 (0 = 2048); gpq_queue_autotune_sort picks one */

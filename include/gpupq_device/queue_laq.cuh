@@ -71,7 +71,8 @@ struct LaqView {
   // wlog_n[(((cur + o) mod cal_windows) * cal_blocks + b) * 16]; events beyond the calendar in over[p]
   // (p = parity of the step that appended them), count over_n[p]; events at or past the end
   // time in parked, count *parked_n.  A step's commit blocks read the log of their own LPs for
-  // its window and group it by LP in LDS.
+  // its window and group it by LP in LDS.  Large calendars keep the logs per unit of 512 LPs, with plain
+  // counts and outboxes between the units, in a layout of their own; wlog is then their logs.
   Event* wlog;
   uint32_t* wlog_n;
   Event* over;
