@@ -100,8 +100,8 @@ __device__ __forceinline__ void merge_tile(const ASrc& A, uint32_t na, const Eve
   const uint32_t j0 = t0 - i0;
   const uint32_t ca = i1 - i0, cb = (t1 - t0) - ca;
   const uint32_t len = t1 - t0;
-  // the thread's loads are all in flight at once: one after the other, each waits for memory (the
-  // GAQ's merge of 1.6 million records took 48 us, 40 so, with the heads below in registers)
+  // the thread's loads are all in flight at once: one after the other, each waits for memory (100,003
+  // LPs in the HQ 175 ms, 166 so, with the heads below in registers)
   uint4 res[kPerThread];
 #pragma unroll
   for (int q = 0; q < kPerThread; ++q) {
