@@ -69,6 +69,27 @@ __device__ __forceinline__ void block_min_publish(uint32_t v, uint32_t* partial,
   publish_window_at(w, atomicExch(&w.fold[0], kInfBits));
 }
 
+// A thread's inserts into the staging of LPs, each one's slot on its way while the thread works on the
+// next event: the record is stored when the next slot has been asked for, and by flush().
+struct StagedInserts {
+  Event e;
+  uint32_t pos;
+  bool any = false;
+  __device__ __forceinline__ void put(Event* stage, uint32_t* ins, uint32_t stage_cap, WindowState* ws, const Event& x) {
+    const uint32_t p = atomicAdd(&ins[x.dst], 1u);
+    flush(stage, stage_cap, ws);
+    e = x;
+    pos = p;
+    any = true;
+  }
+  __device__ __forceinline__ void flush(Event* stage, uint32_t stage_cap, WindowState* ws) {
+    if (!any) return;
+    if (pos < stage_cap) store_event(&stage[(size_t)e.dst * stage_cap + pos], e);
+    else atomicOr(&ws->error, kErrStageOverflow);
+    any = false;
+  }
+};
+
 // One block: folds the per-block minima and publishes gmin, the window end
 // min(gmin + lookahead, horizon) and the done flag.
 __global__ void window_publish_kernel(const uint32_t* partial, uint32_t count, WindowState* ws, float lookahead,

@@ -70,16 +70,19 @@ __device__ __forceinline__ void phold_drain(const Q& q, const PholdDev& m, uint3
 }
 
 // Drain mode on the local array queue: the same commits in the same order as repeated
-// peek / set_done, with the LP's ring cursor, count and hash held in registers and the
-// next record loaded while the current one is processed; written back once.
+// peek / set_done, with the LP's ring cursor, count and hash held in registers, the next record loaded
+// and the last successor's slot taken while the current record is processed; written back once.  An event
+// is a chain of memory accesses whatever is overlapped, and that is what bounds it (200,003 LPs, 16 events
+// each: 14.1 ms with the slot waited for before the next event, 13.7 so; serving 116.9 and 116.0).
 __device__ __forceinline__ void phold_drain(const LaqView& q, const PholdDev& m, uint32_t lp) {
-  const uint32_t wend = q.ws->wend;
-  if (!(q.head[lp] < wend)) return;
+  const uint32_t wend = q.ws->wend, head = q.head[lp];
   const uint32_t mask = (1u << q.cap_log2) - 1u;
   const Event* ring = q.ring + ((size_t)lp << q.cap_log2);
   uint32_t rd = q.rd[lp], len = q.len[lp];
   uint32_t n = m.count[lp];
   uint64_t h = m.hash[lp];
+  if (!(head < wend)) return;
+  StagedInserts out;
   uint32_t last = m.last_ts ? m.last_ts[lp] : 0u;
   Event cur = load_event(&ring[rd]);
   while (len && cur.ts < wend) {
@@ -93,12 +96,13 @@ __device__ __forceinline__ void phold_drain(const LaqView& q, const PholdDev& m,
     const float ex = exp_from_u32(r.x);
     const uint32_t dst = r.y < m.p_self ? lp : (uint32_t)(((uint64_t)r.z * m.num_lps) >> 32);
     const float t_new = (bits_to_f(cur.ts) + m.lookahead) + ex;
-    q.insert(Event{f_to_bits(t_new), dst, lp, m.init_per_lp + n});
+    out.put(q.stage, q.ins, q.stage_cap, q.ws, Event{f_to_bits(t_new), dst, lp, m.init_per_lp + n});
     ++n;
     rd = (rd + 1) & mask;
     --len;
     cur = nxt;
   }
+  out.flush(q.stage, q.stage_cap, q.ws);
   q.rd[lp] = rd;
   q.len[lp] = len;
   q.head[lp] = len ? cur.ts : kInfBits;

@@ -44,12 +44,14 @@ __global__ __launch_bounds__(256) void pool_step_kernel(LaqView q, const PoolIns
   const uint32_t lp = blockIdx.x * blockDim.x + threadIdx.x;
   const uint32_t local = lp - in.base;
   if (lp >= capacity || local >= in.lps) return;         // the instance's last block may be partly unused
-  if (!(q.head[lp] < wend)) return;
+  const uint32_t head = q.head[lp];
   const uint32_t mask = (1u << q.cap_log2) - 1u;
   const Event* ring = q.ring + ((size_t)lp << q.cap_log2);
   uint32_t rd = q.rd[lp], len = q.len[lp];
   uint32_t n = count[lp];
   uint64_t h = hash[lp];
+  if (!(head < wend)) return;
+  StagedInserts out;
   Event cur = load_event(&ring[rd]);
   while (len && cur.ts < wend) {
     const Event nxt = len > 1 ? load_event(&ring[(rd + 1) & mask]) : Event{kInfBits, 0u, 0u, 0u};
@@ -58,12 +60,13 @@ __global__ __launch_bounds__(256) void pool_step_kernel(LaqView q, const PoolIns
     const float ex = exp_from_u32(r.x);
     const uint32_t dst_local = r.y < in.p_self ? local : (uint32_t)(((uint64_t)r.z * in.lps) >> 32);
     const float t_new = (bits_to_f(cur.ts) + in.lookahead) + ex;
-    q.insert(Event{f_to_bits(t_new), in.base + dst_local, local, in.init_per_lp + n});
+    out.put(q.stage, q.ins, q.stage_cap, q.ws, Event{f_to_bits(t_new), in.base + dst_local, local, in.init_per_lp + n});
     ++n;
     rd = (rd + 1) & mask;
     --len;
     cur = nxt;
   }
+  out.flush(q.stage, q.stage_cap, q.ws);
   q.rd[lp] = rd;
   q.len[lp] = len;
   q.head[lp] = len ? cur.ts : kInfBits;

@@ -21,9 +21,8 @@ struct HqState {
   uint32_t mcount;         // records in the merged buffer
   uint32_t prefix, deq_n, rest_n;
   uint32_t bound_valid;
-  uint32_t carry_n;        // records that travel down as insert chunks
   uint32_t select;         // 1: queue_post selects the next step's events
-  uint32_t pad[3];
+  uint32_t pad[4];
   Event bound;             // the root's largest record while nodes exist below the root
   const Event* mptr;       // = merged buffer (pointer slot for the selection)
   // insert-update chunks: target node, size, first record among the carried ones
