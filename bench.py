@@ -284,7 +284,7 @@ QUEUE_GROUPS = {
 }
 GROUP_KERNELS = {
     "sort": ("tile_sort_kernel", "sample_rank_kernel", "bucket_merge_kernel"),
-    "merge": ("merge_tasks_kernel",),
+    "merge": ("merge_tasks_kernel", "hq_merge_kernel"),
     "select": ("select_",),
 }
 
