@@ -84,9 +84,29 @@ __device__ __forceinline__ uint32_t samples_of(uint32_t r, uint32_t len) {
   return len > off ? (len - off - 1u) / kSample + 1u : 0u;
 }
 // Record index of sample s of a level's input: the samples of whole runs are numbered run by run.
-__device__ __forceinline__ uint32_t sample_record(uint32_t s, uint32_t w) {
+__device__ __forceinline__ uint32_t sample_record(uint32_t s, uint32_t w, uint32_t fan) {
   const uint32_t run = s / (w / kSample);
-  return run * w + (s % (w / kSample)) * kSample + sample_offset(run % kFan);
+  return run * w + (s % (w / kSample)) * kSample + sample_offset(run % fan);
+}
+
+// Runs merged at once, for n records.  Two levels of 32 (up to 2^20 records) or 64 (2^22) runs each, with up
+// to 64 samples a block, where 128 runs leave a block room for 24 (all shares have to fit), so that a level
+// takes several rounds of blocks, and leave the second level few runs: 200,003 records 85 us and 93 with 128,
+// 500,009 133 and 163, 1,000,003 202 and 300.
+__host__ __device__ __forceinline__ uint32_t fan_of(uint64_t n) {
+  return n <= (uint64_t)kRun * kFan ? kFan : (n <= kRun << 10 ? 32u : (n <= kRun << 12 ? 64u : kFan));
+}
+// Samples per block of bucket_merge_kernel: as many blocks as the chip runs at once, two per CU.
+__device__ __forceinline__ uint32_t bucket_samples(uint32_t n, uint32_t fan) {
+  const uint32_t even = (n / kSample + 511u) / 512u;
+  return fan == kFan || even < kBucketSamples ? kBucketSamples : (even < 64u ? even : 64u);
+}
+static_assert((64u + 64u) * kSample <= kBucketCap, "a block of the narrower levels fits");
+// Records per run of a level's input.
+__device__ __forceinline__ uint32_t level_width(uint32_t level, uint32_t fan) {
+  uint32_t w = kRun;
+  for (uint32_t i = 1; i < level; ++i) w *= fan;
+  return w;
 }
 
 // A record as two words whose pair order is the sort order.
@@ -129,11 +149,6 @@ struct LdsRecs {
     return oh != h ? oh < h : (equal ? ol <= l : ol < l);
   }
 };
-
-// Blocks of bucket_merge_kernel per group of kFan runs of w records.
-__host__ __device__ __forceinline__ uint64_t buckets_per_group(uint64_t w) {
-  return (w * kFan / kSample + kBucketSamples - 1) / kBucketSamples;
-}
 
 // Levels that n records take.
 __host__ __device__ __forceinline__ uint32_t sort_levels(uint64_t n) {
@@ -293,27 +308,28 @@ __device__ __forceinline__ bool level_buffers(uint32_t n, uint32_t level, Event*
 // a power of two, at most a wave's, which then takes two runs each), and order[group's first
 // sample + rank] = the sample's index.
 __global__ __launch_bounds__(256) void sample_rank_kernel(Event* buf0, Event* buf1, const uint32_t* d_n, uint32_t cap,
-                                                          uint32_t level, uint32_t w, uint32_t* order) {
+                                                          uint32_t level, uint32_t most, uint32_t* order) {
   const uint32_t n = d_n ? *d_n : cap;
+  const uint32_t fan = fan_of(n), w = level_width(level, fan);
   const Event* in;
   Event* out;
   if (!level_buffers(n, level, buf0, buf1, &in, &out)) return;
   const uint32_t ns = (n + kSample - 1u) / kSample;
-  const uint64_t group = (uint64_t)w * kFan;                       // records per group
-  uint32_t lanes = 1;                                              // lanes per sample
-  while (lanes < (uint32_t)kWave && (uint64_t)lanes * w < n) lanes *= 2;
+  const uint64_t group = (uint64_t)w * fan;                        // records per group
+  uint32_t lanes = 1;                                              // lanes per sample, `most` at most
+  while (lanes < most && lanes < fan && (uint64_t)lanes * w < n) lanes *= 2;
   const uint32_t t = blockIdx.x * 256u + threadIdx.x;
   const uint64_t s = (uint64_t)t / lanes;
   const uint32_t k = t % lanes;
   if (((uint64_t)t & ~63ull) / lanes >= ns) return;                // the whole wave is past the samples
   uint32_t rank = 0;
-  const uint32_t i = sample_record((uint32_t)s, w);
+  const uint32_t i = sample_record((uint32_t)s, w, fan);
   const uint32_t g0 = (uint32_t)(i / group * group);               // first record of its group
   const bool is = s < ns && i < n;                                 // the last run may be short of its last sample
   if (is) {
     const uint32_t own = (i - g0) / w;
     const Rec me = load_rec(in + i);
-    for (uint32_t r = k; r < kFan; r += lanes) {
+    for (uint32_t r = k; r < fan; r += lanes) {
       const uint64_t r0 = (uint64_t)g0 + (uint64_t)r * w;          // first record of run r
       if (r0 >= n) break;
       const uint32_t len = (uint32_t)(n - r0 < w ? n - r0 : w);
@@ -325,11 +341,11 @@ __global__ __launch_bounds__(256) void sample_rank_kernel(Event* buf0, Event* bu
   if (is && k == 0) order[g0 / kSample + rank] = (uint32_t)s;
 }
 
-// A block merges, for kBucketSamples samples of its group from rank b0 on (in sample order), the
+// A block merges, for bucket_samples of its group from rank b0 on (in sample order), the
 // records from the first of them up to the first of the next block (the group's first block:
 // from its first record; the last: to its end).
 __global__ __launch_bounds__(kBucketThreads) void bucket_merge_kernel(Event* buf0, Event* buf1, const uint32_t* d_n,
-                                                                      uint32_t cap, uint32_t level, uint32_t w,
+                                                                      uint32_t cap, uint32_t level,
                                                                       const uint32_t* order) {
   __shared__ LdsRecs<kBucketCap> s;
   __shared__ uint32_t s_from[kFan], s_off[kFan + 1];
@@ -337,8 +353,9 @@ __global__ __launch_bounds__(kBucketThreads) void bucket_merge_kernel(Event* buf
   const Event* in;
   Event* out;
   if (!level_buffers(n, level, buf0, buf1, &in, &out)) return;
-  const uint64_t group = (uint64_t)w * kFan;
-  const uint64_t per = buckets_per_group(w);
+  const uint32_t fan = fan_of(n), w = level_width(level, fan), samples = bucket_samples(n, fan);
+  const uint64_t group = (uint64_t)w * fan;
+  const uint64_t per = (group / kSample + samples - 1u) / samples;  // blocks per group
   const uint64_t start = blockIdx.x / per * group;                 // first record of the block's group
   if (start >= n) return;
   const uint32_t g0 = (uint32_t)start;
@@ -346,18 +363,18 @@ __global__ __launch_bounds__(kBucketThreads) void bucket_merge_kernel(Event* buf
   const uint32_t runs = (glen + w - 1u) / w;
   const uint32_t last = (runs - 1u) * w;                           // the group's last run may be short
   const uint32_t gs = last / kSample + samples_of(runs - 1u, glen - last);   // samples of the group
-  const uint32_t b0 = (uint32_t)(blockIdx.x % per) * kBucketSamples;
+  const uint32_t b0 = (uint32_t)(blockIdx.x % per) * samples;
   if (b0 && b0 >= gs) return;
   // kFindLanes lanes each: the block's first record in run r, and the record past its last
   {
-    const uint32_t job = threadIdx.x / kFindLanes, r = job >> 1, at = b0 + (job & 1u) * kBucketSamples;
+    const uint32_t job = threadIdx.x / kFindLanes, r = job >> 1, at = b0 + (job & 1u) * samples;
     const uint32_t r0 = g0 + r * w;
     const uint32_t len = r < runs ? (n - r0 < w ? n - r0 : w) : 0u;
     uint32_t c = at ? len : 0u, find = 0;
     Rec me{0, 0};
     uint32_t own = 0;
     if (at && at < gs) {
-      const uint32_t i = sample_record(order[g0 / kSample + at], w);   // the splitting record
+      const uint32_t i = sample_record(order[g0 / kSample + at], w, fan);   // the splitting record
       own = (i - g0) / w;
       if (r == own) {
         c = i - r0;
@@ -725,17 +742,17 @@ gpq_status sort_records(const Event* in, Event* buf0, Event* buf1, uint32_t* ord
                         hipStream_t stream, unsigned long long* acct, const uint32_t* seg_pre, uint32_t seg_cap) {
   hipLaunchKernelGGL(tile_sort_kernel, dim3(grid_of(cap, kRun)), dim3(kTileThreads), 0, stream, in, buf0, buf1,
                      d_n, cap, seg_pre, seg_cap);
-  uint64_t w = kRun;
-  for (uint32_t level = 1; level <= sort_levels(cap); ++level, w *= kFan) {
+  // Grids for any number of records up to cap, and so for either width of the levels: a group's blocks hold 768
+  // records or more on average, and its last one may hold fewer.
+  const uint64_t blocks = cap / 762u + 45u;
+  for (uint32_t level = 1; level <= sort_levels(cap); ++level) {
+    const uint64_t w = level == 1 ? kRun : (level == 2 ? (uint64_t)kRun * fan_of(cap) : (uint64_t)kRun * kFan * kFan);
     const uint64_t runs = std::min<uint64_t>((cap + w - 1) / w, kWave);
-    const uint64_t lanes = 1ull << log2u(runs);
+    const uint32_t lanes = 1u << log2u(runs);
     hipLaunchKernelGGL(sample_rank_kernel, dim3(grid_of(((uint64_t)cap + kSample - 1) / kSample * lanes, 256)), dim3(256),
-                       0, stream, buf0, buf1, d_n, cap, level, (uint32_t)w, order);
-    // whole groups take buckets_per_group blocks each, the last one as many as its records need
-    const uint64_t groups = cap / (w * kFan), rest = cap % (w * kFan);
-    const uint64_t blocks = groups * buckets_per_group(w) + grid_of(rest, kSample * kBucketSamples);
-    hipLaunchKernelGGL(bucket_merge_kernel, dim3((uint32_t)blocks), dim3(kBucketThreads), 0, stream,
-                       buf0, buf1, d_n, cap, level, (uint32_t)w, order);
+                       0, stream, buf0, buf1, d_n, cap, level, lanes, order);
+    hipLaunchKernelGGL(bucket_merge_kernel, dim3((uint32_t)blocks), dim3(kBucketThreads), 0, stream, buf0, buf1, d_n, cap,
+                       level, order);
   }
   GPQ_HIP(hipGetLastError());
   if (!acct) return GPQ_OK;

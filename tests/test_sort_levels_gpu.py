@@ -62,3 +62,12 @@ def test_sort_three_levels(gpq):
     src = np.zeros_like(a)
     src[a["dst"]] = a
     assert np.array_equal(back, src)
+
+
+@pytest.mark.parametrize("how", ["equal", "interleaved", "random"])
+@pytest.mark.parametrize("n", [163841, 393217, 524288, 700001, 1048575, 1048576, 1048577, 4194304, 4194305])
+def test_sort_of_two_narrow_levels(gpq, n, how):
+    # up to 2^20 records the two levels merge up to 32 runs each, up to 2^22 64, above it 128
+    a = _make(gpq, n, how)
+    want = a[np.lexsort((a["dst"], a["seq"], a["src"], a["ts"]))]
+    assert np.array_equal(_sort(gpq, a), want)
