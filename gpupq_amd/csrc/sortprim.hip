@@ -47,10 +47,10 @@ __device__ __forceinline__ uint32_t group_merge_split(const ASrc& A, uint32_t na
 // --- sort -------------------------------------------------------------------------
 //
 // A run of up to kRun records is sorted by one block (tile_sort_kernel); a level then merges up to
-// kFan sorted runs at once: every kSampleth record of a run is a sample (from an offset of the run's
+// fan_of() sorted runs at once: every kSampleth record of a run is a sample (from an offset of the run's
 // own: the same quantiles sampled in every run would leave gaps without samples, and blocks with
 // three times the others' records), sample_rank_kernel ranks
-// all samples of the runs against each other, and bucket_merge_kernel takes kBucketSamples
+// all samples of the runs against each other, and bucket_merge_kernel takes bucket_samples()
 // consecutive samples' worth of records per block -- its share of every run, found by searching
 // each run for two samples -- and merges the shares in LDS.  Between two samples of a run lie fewer
 // than kSample records, so a block's shares hold at most (kBucketSamples + kFan) * kSample =
