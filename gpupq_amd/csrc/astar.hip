@@ -280,7 +280,6 @@ __global__ __launch_bounds__(kTileBlock) void astar_tile_kernel(AstarDev a, Asta
     }
     if (tid < 3) s_n[tid] = 0;
     if (tid == 0) {
-      t.count[(size_t)par * t.tiles + tile] = 0;  // consumed; refilled two steps on
       s_park = n_park ? 0u : parked;              // only this workgroup parks in the tile
       s_pmin = n_park ? 0xFFFFFFFFu : park_f;
     }
@@ -395,7 +394,8 @@ __global__ __launch_bounds__(kTileBlock) void astar_tile_kernel(AstarDev a, Asta
       fmin_pushed = min(fmin_pushed, g_out + grid_heur(a.conn, hnx, hny, (int)a.tx, (int)a.ty));
     }
     __syncthreads();
-    if (tid == 0) {
+    if (tid == 0) {                               // barriers after every wave's loads of these words
+      t.count[(size_t)par * t.tiles + tile] = 0;  // consumed; refilled two steps on
       t.park_count[tile] = s_park;
       t.park_fmin[tile] = s_pmin;
     }
