@@ -1022,7 +1022,7 @@ gpq_status LaqQueue::init_calendar() {
   GPQ_TRY(arena.alloc(&v_.ins, L));
   GPQ_TRY(arena.alloc(&v_.head, L));
   GPQ_TRY(arena.alloc(&sum_, 1));
-  if (L >= kGroupedMinLps) {
+  if (plan_calendar_groups()) {
     GPQ_TRY(init_calendar_groups());
     GPQ_TRY(arena.alloc(&v_.over_n, 64));             // the list counters' places; only the parked one is used
     v_.wlog = groups_.wlog;
@@ -1054,12 +1054,22 @@ gpq_status LaqQueue::init_calendar() {
   return GPQ_OK;
 }
 
-// Units, groups and their buffers.  A group's list holds twice its share of far_per_lp, so that
-// uniform destinations never fill it before the whole queue's bound; a pass over a log takes all
-// but the last LP's events that fit.
-gpq_status LaqQueue::init_calendar_groups() {
-  const uint32_t L = cfg.num_lps, B = cfg.calendar_windows;
-  cal::Groups& g = groups_;
+// LDS of the filing launch: the counts of a group's logs.
+static size_t file_lds(const cal::Groups& g, uint32_t windows) {
+  return sizeof(uint32_t) * ((size_t)windows << (g.group_shift - cal::kUnitLog2));
+}
+// At most this much, beside the launch's own 25 KiB of the CU's 160.
+constexpr size_t kFileLdsMost = 96 * 1024;
+
+// Whether the logs have one writer each, and then their sizes.  A group's list holds twice its share
+// of far_per_lp, so that uniform destinations never fill it before the whole queue's bound; a pass
+// over a log takes all but the last LP's events that fit.  Calendars whose filing launch would need
+// more LDS than there is (more than 2^23 LPs with 256 windows, 2^24 with 128, 2^25 with 64) keep the
+// logs with atomics.
+bool LaqQueue::plan_calendar_groups() {
+  const uint32_t L = cfg.num_lps;
+  if (L < kGroupedMinLps) return false;
+  cal::Groups g{};
   g.units = (uint32_t)ceil_div(L, cal::kUnit);
   g.group_shift = cal::kUnitLog2;
   while (((L - 1u) >> g.group_shift) + 1u > cal::kMaxGroups) ++g.group_shift;
@@ -1067,8 +1077,15 @@ gpq_status LaqQueue::init_calendar_groups() {
   g.log_cap = cal::kUnit * cfg.capacity_per_lp;
   g.passes = g.log_cap / (cal::kUnitPass - cal::kLpMost) + 1u;
   const uint64_t over = 2ull * cfg.far_per_lp << g.group_shift;
-  GPQ_CHECK_ARG(over < (1ull << 32), "LAQ calendar: num_lps too large for the groups' lists");
   g.over_cap = (uint32_t)over;
+  if (over >= (1ull << 32) || file_lds(g, cfg.calendar_windows) > kFileLdsMost) return false;
+  groups_ = g;
+  return true;
+}
+
+gpq_status LaqQueue::init_calendar_groups() {
+  const uint32_t B = cfg.calendar_windows;
+  cal::Groups& g = groups_;
   const size_t slots = (size_t)g.units * g.passes;
   GPQ_TRY(arena.alloc(&g.wlog, (size_t)g.units * B * g.log_cap));
   GPQ_TRY(arena.alloc(&g.wlog_n, (size_t)g.units * B));
@@ -1081,8 +1098,7 @@ gpq_status LaqQueue::init_calendar_groups() {
   GPQ_HIP(hipMemsetAsync(g.npass, 0, sizeof(uint32_t) * g.units, stream));
   GPQ_HIP(hipMemsetAsync(g.parts, 0, sizeof(uint32_t) * slots * cal::kMaxGroups, stream));
   GPQ_HIP(hipMemsetAsync(g.over_n, 0, sizeof(uint32_t) * g.groups * 16u, stream));
-  const size_t lds = sizeof(uint32_t) * ((size_t)B << (g.group_shift - cal::kUnitLog2));
-  GPQ_CHECK_ARG(lds <= 96u * 1024u, "LAQ calendar: num_lps * calendar_windows too large for the filing step's counts");
+  const size_t lds = file_lds(g, B);
   if (lds > 16u * 1024u)
     GPQ_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(cal_file_kernel),
                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
@@ -1092,9 +1108,8 @@ gpq_status LaqQueue::init_calendar_groups() {
 gpq_status LaqQueue::calendar_file() {
   const cal::Groups& g = groups_;
   GPQ_CHECK_ARG(g.units, "LAQ: calendar_file needs a large calendar");
-  const size_t lds = sizeof(uint32_t) * ((size_t)cfg.calendar_windows << (g.group_shift - cal::kUnitLog2));
-  hipLaunchKernelGGL(cal_file_kernel, dim3(ceil_div(g.groups, cal::kXcds) * cal::kXcds), dim3(cal::kFileThreads), lds, stream, v_, g, cfg.horizon,
-                     1.0f / cfg.lookahead);
+  hipLaunchKernelGGL(cal_file_kernel, dim3(ceil_div(g.groups, cal::kXcds) * cal::kXcds), dim3(cal::kFileThreads),
+                     file_lds(g, cfg.calendar_windows), stream, v_, g, cfg.horizon, 1.0f / cfg.lookahead);
   GPQ_HIP(hipGetLastError());
   return GPQ_OK;
 }

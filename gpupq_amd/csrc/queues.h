@@ -67,6 +67,7 @@ class LaqQueue final : public QueueBase {
 
  private:
   gpq_status init_calendar();
+  bool plan_calendar_groups();
   gpq_status init_calendar_groups();
   cal::Groups groups_{};
   gpq_status calendar_gather(uint32_t lp, std::vector<Event>* out);
