@@ -1098,10 +1098,9 @@ gpq_status LaqQueue::init_calendar_groups() {
   GPQ_HIP(hipMemsetAsync(g.npass, 0, sizeof(uint32_t) * g.units, stream));
   GPQ_HIP(hipMemsetAsync(g.parts, 0, sizeof(uint32_t) * slots * cal::kMaxGroups, stream));
   GPQ_HIP(hipMemsetAsync(g.over_n, 0, sizeof(uint32_t) * g.groups * 16u, stream));
-  const size_t lds = file_lds(g, B);
-  if (lds > 16u * 1024u)
-    GPQ_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(cal_file_kernel),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  // the same bound for every queue: the attribute is the kernel's, and the last one to set it decides for all
+  GPQ_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(cal_file_kernel),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)kFileLdsMost));
   return GPQ_OK;
 }
 
