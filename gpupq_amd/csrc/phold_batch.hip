@@ -606,32 +606,27 @@ gpq_status PholdBatch::run_calendar_union(uint32_t batch, double* seconds) {
   uint64_t total = 0;
   uint32_t max_init = 0;
   float la = inst[0].lookahead, horizon = inst[0].end_time;
+  uint64_t in_blocks = 0, in_units = 0;       // LPs, in whole commit blocks and in whole units of a large calendar
   for (uint32_t i = 0; i < n; ++i) {
-    // whole units of a large calendar, so whole commit blocks of a small one
-    const uint32_t blocks = (uint32_t)ceil_div(inst[i].num_lps, cal::kUnit) * (cal::kUnit / kCalBlk);
-    PoolInst& t = tab[i];
-    t = PoolInst{};
-    t.base = (uint32_t)total;
-    t.lps = inst[i].num_lps;
-    t.init_per_lp = inst[i].init_per_lp;
-    t.seed = inst[i].seed;
-    t.end_time = inst[i].end_time;
-    t.lookahead = inst[i].lookahead;
-    t.p_self = inst[i].p_self_u32;
-    t.active = 1;
-    t.block_begin = (uint32_t)(total / kCalBlk);
-    t.block_end = t.block_begin + blocks;
-    total += (uint64_t)blocks * kCalBlk;
+    in_blocks += (uint64_t)ceil_div(inst[i].num_lps, kCalBlk) * kCalBlk;
+    in_units += (uint64_t)ceil_div(inst[i].num_lps, cal::kUnit) * cal::kUnit;
     max_init = std::max(max_init, inst[i].init_per_lp);
     la = std::min(la, inst[i].lookahead);
     horizon = std::max(horizon, inst[i].end_time);
   }
-  GPQ_CHECK_ARG(total < (1ull << 31), "phold batch: too many LPs for one queue");
+  GPQ_CHECK_ARG(in_blocks < (1ull << 31), "phold batch: too many LPs for one queue");
   GPQ_CHECK_ARG(far_per_lp >= max_init, "phold batch (calendar): far_per_lp must hold every initial event of an LP "
                 "(the parked list takes an LP's events past its end time)");
+  // Logs with one writer need whole units, and with many small instances the LPs that fill them up cost
+  // more than such logs save: they may be an eighth of the instances' blocks, from 2^19 LPs on a third.
+  // One writer against atomics, 16 events per LP to time 5: 150 instances of 2100 LPs (a ninth more) 2.03
+  // and 2.09 ms, 300 of 1100 (a fifth) 2.25 and 2.20, 400 of 600 (a third) 1.99 and 1.79, 1000 of 600 3.02
+  // and 3.15, 2000 of 700 5.03 and 5.38, 6000 of 250 (twice) 5.66 and 4.86.
+  const uint64_t pad = in_units - in_blocks;
+  bool units = in_blocks >= LaqQueue::kGroupedMinLps && pad <= in_blocks / (in_blocks >= (1u << 19) ? 3 : 8) &&
+               in_units < (1ull << 31);
   gpq_queue_config qc{};
   qc.kind = GPQ_LAQ;
-  qc.num_lps = (uint32_t)total;
   qc.capacity_per_lp = capacity_per_lp;
   qc.stage_per_lp = stage_per_lp;
   qc.far_per_lp = far_per_lp;
@@ -639,9 +634,38 @@ gpq_status PholdBatch::run_calendar_union(uint32_t batch, double* seconds) {
   qc.horizon = horizon;
   qc.block_threads = 256;
   qc.calendar_windows = calendar_windows;
-  std::unique_ptr<LaqQueue> q(new LaqQueue(qc));
-  GPQ_TRY(q->init_common());
-  GPQ_TRY(q->init());
+  std::unique_ptr<LaqQueue> q;
+  for (;; units = false) {                    // what whole units do not fit may in blocks
+    const uint32_t whole = units ? (uint32_t)cal::kUnit : kCalBlk;
+    total = 0;
+    for (uint32_t i = 0; i < n; ++i) {
+      const uint32_t blocks = (uint32_t)ceil_div(inst[i].num_lps, whole) * (whole / kCalBlk);
+      PoolInst& t = tab[i];
+      t = PoolInst{};
+      t.base = (uint32_t)total;
+      t.lps = inst[i].num_lps;
+      t.init_per_lp = inst[i].init_per_lp;
+      t.seed = inst[i].seed;
+      t.end_time = inst[i].end_time;
+      t.lookahead = inst[i].lookahead;
+      t.p_self = inst[i].p_self_u32;
+      t.active = 1;
+      t.block_begin = (uint32_t)(total / kCalBlk);
+      t.block_end = t.block_begin + blocks;
+      total += (uint64_t)blocks * kCalBlk;
+    }
+    qc.num_lps = (uint32_t)total;
+    q.reset(new LaqQueue(qc));
+    if (!units) q->use_atomic_logs();
+    GPQ_TRY(q->init_common());
+    const gpq_status s = q->init();
+    if (units && (s != GPQ_OK || !q->groups().units)) {
+      q.reset();
+      continue;
+    }
+    GPQ_TRY(s);
+    break;
+  }
   PinnedBlock pinned_count, pinned_hash;      // host staging of the counters and hashes
   DeviceArena arena;                          // destroyed first, so after the stream's last work
   arena.on(q->stream);

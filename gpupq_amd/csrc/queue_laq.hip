@@ -1068,7 +1068,7 @@ constexpr size_t kFileLdsMost = 96 * 1024;
 // logs with atomics.
 bool LaqQueue::plan_calendar_groups() {
   const uint32_t L = cfg.num_lps;
-  if (L < kGroupedMinLps) return false;
+  if (atomic_logs_ || L < kGroupedMinLps) return false;
   cal::Groups g{};
   g.units = (uint32_t)ceil_div(L, cal::kUnit);
   g.group_shift = cal::kUnitLog2;

@@ -57,6 +57,8 @@ class LaqQueue final : public QueueBase {
   // Large calendars (calendar_groups.h): logs with one writer, filed by a launch of their own
   // before each commit step.  units == 0 otherwise.
   const cal::Groups& groups() const { return groups_; }
+  // Before init: a calendar of any size keeps the logs with atomics (whose blocks are half a unit).
+  void use_atomic_logs() { atomic_logs_ = true; }
   gpq_status calendar_file();
   static constexpr uint32_t kGatherCap = 1u << 16;   // records one LP may hold for lp_contents
   // Two-tier mode, several windows: block b follows the near horizon of ws_array[win[b]].
@@ -70,6 +72,7 @@ class LaqQueue final : public QueueBase {
   bool plan_calendar_groups();
   gpq_status init_calendar_groups();
   cal::Groups groups_{};
+  bool atomic_logs_ = false;
   gpq_status calendar_gather(uint32_t lp, std::vector<Event>* out);
   LaqView v_{};
   uint64_t* sum_ = nullptr;
