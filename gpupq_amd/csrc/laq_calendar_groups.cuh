@@ -19,7 +19,12 @@
 //   out   [U][passes][kUnitPass]      outbox of each pass of a unit's last step
 //   parts [U][passes][kMaxGroups]     the part of group g in it: first event | number << 16
 //   npass [U]                         passes of the unit's last step
-//   over  [G][over_cap]               the group's events beyond the calendar: over_n[g * 16] of them
+//   over  [G][own_cap], [G * own_cap] the groups' events beyond the calendar.  Half of the room is the
+//                                     groups' own, far_per_lp records per LP; the other half is dealt
+//                                     out at the start (cal_start_groups_kernel): to each group what its
+//                                     initial events need beyond its own, and the rest evenly, so that
+//                                     initial events may lie anywhere, as in the one list of a small
+//                                     calendar.  Until then the shared half holds them unsorted.
 // The outboxes of the last step are part of the queue's contents.
 #pragma once
 
@@ -40,6 +45,19 @@ constexpr uint32_t kToGroup = 0x1000u;   // flag on a way: to a group's part of 
 __device__ __forceinline__ Event* unit_log(const LaqView& q, const Groups& g, uint32_t unit, uint32_t x) {
   return g.wlog + ((size_t)unit * q.cal_windows + (x & (q.cal_windows - 1u))) * g.log_cap;
 }
+// A group's events beyond the calendar: `cap` places at most, of which the first are its own.
+struct OverList {
+  Event* own;
+  Event* more;
+  uint32_t own_cap, cap;
+  __device__ __forceinline__ Event* at(uint32_t p) const { return p < own_cap ? own + p : more + (p - own_cap); }
+};
+__device__ __forceinline__ Event* shared_over(const Groups& g) { return g.over + (size_t)g.groups * g.own_cap; }
+__device__ __forceinline__ OverList over_list(const Groups& g, uint32_t grp) {
+  const uint32_t* w = g.over_n + grp * kOverWords;
+  return OverList{g.over + (size_t)grp * g.own_cap, shared_over(g) + w[kOverFrom], g.own_cap, g.own_cap + w[kOverMore]};
+}
+
 __device__ __forceinline__ uint32_t* unit_count(const LaqView& q, const Groups& g, uint32_t unit, uint32_t x) {
   return g.wlog_n + (size_t)unit * q.cal_windows + (x & (q.cal_windows - 1u));
 }
@@ -186,7 +204,7 @@ __device__ __forceinline__ void commit_unit(const LaqView& q, const Groups& g, c
 // Files an event of the group in the log of its window, seen from window x over all B windows, or
 // behind the group's events beyond the calendar.  s_n: the counts of the group's logs.
 __device__ __forceinline__ void file_event(const LaqView& q, const Groups& g, const uint32_t* sw, uint32_t x, float inv,
-                                           uint32_t unit0, uint32_t nu, uint32_t* s_n, uint32_t* s_over, Event* over,
+                                           uint32_t unit0, uint32_t nu, uint32_t* s_n, uint32_t* s_over, const OverList& over,
                                            const Event& e) {
   const uint32_t B = q.cal_windows;
   const uint32_t u = (e.dst >> kUnitLog2) - unit0;
@@ -201,7 +219,7 @@ __device__ __forceinline__ void file_event(const LaqView& q, const Groups& g, co
     else atomicOr(&q.ws->error, kErrQueueOverflow);
   } else {
     const uint32_t pos = atomicAdd(s_over, 1u);
-    if (pos < g.over_cap) store_event(over + pos, e);
+    if (pos < over.cap) store_event(over.at(pos), e);
     else atomicOr(&q.ws->error, kErrQueueOverflow);
   }
 }
@@ -227,9 +245,9 @@ __device__ __forceinline__ void file_group(const LaqView& q, const Groups& g, fl
   const uint32_t unit0 = grp * per;
   const uint32_t nu = g.units - unit0 < per ? g.units - unit0 : per;
   const uint32_t end_bits = f_to_bits(end_time);
-  Event* over = g.over + (size_t)grp * g.over_cap;
-  const uint32_t no0 = g.over_n[grp * 16u];
-  const uint32_t no = no0 < g.over_cap ? no0 : g.over_cap;
+  const OverList over = over_list(g, grp);
+  const uint32_t no0 = g.over_n[grp * kOverWords];
+  const uint32_t no = no0 < over.cap ? no0 : over.cap;
   // issued first: the parts of the first units' first passes (always valid) and their pass counts
   uint32_t np[2], part[2];
   auto load_parts = [&](uint32_t u0) {
@@ -249,7 +267,7 @@ __device__ __forceinline__ void file_group(const LaqView& q, const Groups& g, fl
   // in registers before any of it is written, and never to a place past what has been read)
   for (uint32_t c0 = 0; c0 < no; c0 += kFileThreads) {
     const bool has = c0 + t < no;
-    const Event e = has ? load_event(over + c0 + t) : Event{};
+    const Event e = has ? load_event(over.at(c0 + t)) : Event{};
     __syncthreads();
     const bool parked = has && !(e.ts < end_bits);
     const bool keep = has && !parked && !(e.ts < sw[B - 1u]);
@@ -260,7 +278,7 @@ __device__ __forceinline__ void file_group(const LaqView& q, const Groups& g, fl
     uint32_t at = 0;
     if (mk && lane_id() == 0) at = atomicAdd(&s_over, (uint32_t)__popcll(mk));
     at = (uint32_t)__shfl((int)at, 0, kWave);
-    if (keep) store_event(over + at + (uint32_t)__popcll(mk & ((1ull << lane_id()) - 1ull)), e);
+    if (keep) store_event(over.at(at + (uint32_t)__popcll(mk & ((1ull << lane_id()) - 1ull))), e);
     __syncthreads();
     if (s_pn) {                                        // uniform: read after a barrier
       if (t == 0) s_pb = atomicAdd(q.parked_n, s_pn);
@@ -327,7 +345,7 @@ __device__ __forceinline__ void file_group(const LaqView& q, const Groups& g, fl
   }
   __syncthreads();
   for (uint32_t i = t; i < nu * B; i += kFileThreads) g.wlog_n[(size_t)unit0 * B + i] = s_n[i];
-  if (t == 0) g.over_n[grp * 16u] = s_over;
+  if (t == 0) g.over_n[grp * kOverWords] = s_over;
 }
 
 }  // namespace cal

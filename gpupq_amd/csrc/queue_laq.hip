@@ -715,9 +715,9 @@ __global__ __launch_bounds__(kLaqBlock) void cal_post_init_kernel(LaqView q, cal
   const int lane = lane_id(), wave = (int)threadIdx.x / kWave;
   // the list of the LPs' group, or the one list of a small calendar
   const uint32_t grp = g.units ? (blockIdx.x * kLaqBlock) >> g.group_shift : 0u;
-  Event* list = g.units ? g.over + (size_t)grp * g.over_cap : q.over;
-  uint32_t* list_n = g.units ? g.over_n + grp * 16u : &q.over_n[0];
-  const uint32_t list_cap = g.units ? g.over_cap : q.over_cap;
+  const cal::OverList list = g.units ? cal::over_list(g, grp) : cal::OverList{q.over, q.over, q.over_cap, q.over_cap};
+  uint32_t* list_n = g.units ? g.over_n + grp * cal::kOverWords : &q.over_n[0];
+  const bool spill = g.units && !list_n[cal::kOverShared];   // past the list, before the calendar's start
   uint32_t k0 = 0, k = 0;
   if (lp < q.num_lps) {
     k0 = q.ins[lp];
@@ -746,7 +746,12 @@ __global__ __launch_bounds__(kLaqBlock) void cal_post_init_kernel(LaqView q, cal
   for (uint32_t i = 0; i < k; ++i) {
     const Event e = load_event(&q.stage[(size_t)lp * q.stage_cap + i]);
     m = e.ts < m ? e.ts : m;
-    if (start + i < list_cap) store_event(&list[start + i], e);
+    Event* to = start + i < list.cap ? list.at(start + i) : nullptr;
+    if (!to && spill) {
+      const uint32_t pos = atomicAdd(g.spill_n, 1u);
+      if (pos < g.groups * g.own_cap) to = cal::shared_over(g) + pos;
+    }
+    if (to) store_event(to, e);
     else atomicOr(&q.ws->error, kErrQueueOverflow);
   }
   if (k0) q.ins[lp] = 0;
@@ -777,7 +782,7 @@ __global__ void cal_init_publish_kernel(const uint32_t* partial, uint32_t count,
 
 // The ends of windows 0 .. B from the first one (published from the initial events), each one
 // lookahead after the previous in float arithmetic, capped at the end time.
-__global__ void cal_start_kernel(LaqView q, float lookahead, float end_time) {
+__device__ __forceinline__ void cal_start(const LaqView& q, float lookahead, float end_time) {
   CalState* st = q.cal_st;
   const uint32_t B = q.cal_windows;
   st->cur = 0;
@@ -791,6 +796,55 @@ __global__ void cal_start_kernel(LaqView q, float lookahead, float end_time) {
     st->w[i] = w;
   }
   q.ws->sel = 0;
+}
+
+__global__ void cal_start_kernel(LaqView q, float lookahead, float end_time) { cal_start(q, lookahead, end_time); }
+
+// The same for a large calendar, and the shared records dealt out to the groups, by one block.  Initial
+// events that did not fit their group's own records lie in the shared ones in any order; they go to the
+// groups' parts by way of the free end of the parked list, which in the end holds every event that
+// is pending now.  (Only initial events that concentrate on a few groups are moved at all.)
+__global__ __launch_bounds__(1024) void cal_start_groups_kernel(LaqView q, cal::Groups g, float lookahead, float end_time) {
+  __shared__ uint32_t s_wave[1024 / kWave];
+  __shared__ uint32_t s_next[cal::kMaxGroups];
+  const uint32_t t = threadIdx.x;
+  if (t == 0) cal_start(q, lookahead, end_time);
+  if (g.over_n[cal::kOverShared]) return;              // dealt out before: a second start
+  // Events that did not fit, here or in the end: refused, and only the groups' own records are kept.
+  const uint32_t room = g.groups * g.own_cap, spilled = *g.spill_n, parked = *q.parked_n;
+  const bool lost = spilled > room || parked > q.parked_cap || spilled > q.parked_cap - parked;
+  const uint32_t n = lost ? 0u : spilled;
+  uint32_t* w = g.over_n + (t < g.groups ? t : 0u) * cal::kOverWords;
+  const uint32_t count = w[cal::kOverN], over = n && count > g.own_cap ? count - g.own_cap : 0u;
+  const uint32_t more = t < g.groups ? over + (room - n) / g.groups : 0u;
+  uint32_t inc = more;
+#pragma unroll
+  for (int off = 1; off < kWave; off <<= 1) {
+    const uint32_t y = (uint32_t)__shfl_up((int)inc, off, kWave);
+    if (lane_id() >= off) inc += y;
+  }
+  if (lane_id() == kWave - 1) s_wave[t / kWave] = inc;
+  __syncthreads();                                     // and every thread has read the words it goes by
+  for (uint32_t x = 0; x < t / kWave; ++x) inc += s_wave[x];
+  if (t < g.groups) {
+    w[cal::kOverFrom] = s_next[t] = inc - more;
+    w[cal::kOverMore] = more;
+    w[cal::kOverShared] = 1u;
+    if (lost && count > g.own_cap) w[cal::kOverN] = g.own_cap;
+  }
+  if (t == 0) {
+    *g.spill_n = 0u;
+    if (lost) atomicOr(&q.ws->error, kErrQueueOverflow);
+  }
+  if (n == 0) return;
+  Event* shared = cal::shared_over(g);
+  Event* end = q.parked + (q.parked_cap - n);
+  for (uint32_t i = t; i < n; i += 1024u) store_event(end + i, load_event(shared + i));
+  __syncthreads();
+  for (uint32_t i = t; i < n; i += 1024u) {
+    const Event e = load_event(end + i);
+    store_event(shared + atomicAdd(&s_next[e.dst >> g.group_shift], 1u), e);
+  }
 }
 
 // Files every initial event (the list over[0]) in the log of its window (windows 0 .. B - 1)
@@ -882,11 +936,11 @@ __global__ void cal_units_count_kernel(LaqView q, cal::Groups g, unsigned long l
   unsigned long long n = 0;
   for (uint32_t i = t; i < q.num_lps; i += stride) n += min(q.ins[i], q.stage_cap);
   for (uint32_t i = t; i < g.units * q.cal_windows; i += stride) n += min(g.wlog_n[i], g.log_cap);
-  for (uint32_t i = t; i < g.groups; i += stride) n += min(g.over_n[i * 16u], g.over_cap);
+  for (uint32_t i = t; i < g.groups; i += stride) n += min(g.over_n[i * cal::kOverWords], cal::over_list(g, i).cap);
   for (uint32_t u = t; u < g.units; u += stride)
     for (uint32_t p = 0; p < g.npass[u]; ++p)
       for (uint32_t i = 0; i < cal::kMaxGroups; ++i) n += g.parts[((size_t)u * g.passes + p) * cal::kMaxGroups + i] >> 16;
-  if (t == 0) n += min(*q.parked_n, q.parked_cap);
+  if (t == 0) n += min(*q.parked_n, q.parked_cap) + min(*g.spill_n, g.groups * g.own_cap);
   for (int off = 32; off > 0; off >>= 1) n += __shfl_xor(n, off, kWave);
   if (lane_id() == 0) s[threadIdx.x / kWave] = n;
   __syncthreads();
@@ -906,8 +960,11 @@ __global__ void cal_units_gather_kernel(LaqView q, cal::Groups g, uint32_t lp, E
     const Event* lg = cal::unit_log(q, g, unit, x);
     for (uint32_t i = t; i < c; i += stride) gather_one(&lg[i], lp, out, cap, n);
   }
-  const uint32_t no = min(g.over_n[grp * 16u], g.over_cap);
-  for (uint32_t i = t; i < no; i += stride) gather_one(&g.over[(size_t)grp * g.over_cap + i], lp, out, cap, n);
+  const cal::OverList over = cal::over_list(g, grp);
+  const uint32_t no = min(g.over_n[grp * cal::kOverWords], over.cap);
+  for (uint32_t i = t; i < no; i += stride) gather_one(over.at(i), lp, out, cap, n);
+  const uint32_t ns = min(*g.spill_n, g.groups * g.own_cap);
+  for (uint32_t i = t; i < ns; i += stride) gather_one(cal::shared_over(g) + i, lp, out, cap, n);
   for (uint32_t u = t; u < g.units; u += stride)
     for (uint32_t p = 0; p < g.npass[u]; ++p) {
       const size_t slot = (size_t)u * g.passes + p;
@@ -1023,8 +1080,9 @@ gpq_status LaqQueue::init_calendar() {
   GPQ_TRY(arena.alloc(&v_.head, L));
   GPQ_TRY(arena.alloc(&sum_, 1));
   if (plan_calendar_groups()) {
+    GPQ_TRY(arena.alloc(&v_.over_n, 64));             // the list counters' places; the parked one and the spill's are used
+    groups_.spill_n = v_.over_n + 16u;
     GPQ_TRY(init_calendar_groups());
-    GPQ_TRY(arena.alloc(&v_.over_n, 64));             // the list counters' places; only the parked one is used
     v_.wlog = groups_.wlog;
     v_.parked_n = v_.over_n + 32u;
     GPQ_HIP(hipMemsetAsync(v_.over_n, 0, sizeof(uint32_t) * 64, stream));
@@ -1061,9 +1119,9 @@ static size_t file_lds(const cal::Groups& g, uint32_t windows) {
 // At most this much, beside the launch's own 25 KiB of the CU's 160.
 constexpr size_t kFileLdsMost = 96 * 1024;
 
-// Whether the logs have one writer each, and then their sizes.  A group's list holds twice its share
-// of far_per_lp, so that uniform destinations never fill it before the whole queue's bound; a pass
-// over a log takes all but the last LP's events that fit.  Calendars whose filing launch would need
+// Whether the logs have one writer each, and then their sizes.  The groups' lists hold twice
+// far_per_lp events per LP, half of them anywhere, so that uniform destinations never fill one before the
+// whole queue's bound; a pass over a log takes all but the last LP's events that fit.  Calendars whose filing launch would need
 // more LDS than there is (more than 2^23 LPs with 256 windows, 2^24 with 128, 2^25 with 64) keep the
 // logs with atomics.
 bool LaqQueue::plan_calendar_groups() {
@@ -1076,9 +1134,10 @@ bool LaqQueue::plan_calendar_groups() {
   g.groups = ((L - 1u) >> g.group_shift) + 1u;
   g.log_cap = cal::kUnit * cfg.capacity_per_lp;
   g.passes = g.log_cap / (cal::kUnitPass - cal::kLpMost) + 1u;
-  const uint64_t over = 2ull * cfg.far_per_lp << g.group_shift;
-  g.over_cap = (uint32_t)over;
-  if (over >= (1ull << 32) || file_lds(g, cfg.calendar_windows) > kFileLdsMost) return false;
+  // own records, and as many shared ones
+  const uint64_t own = (uint64_t)cfg.far_per_lp << g.group_shift;
+  g.own_cap = (uint32_t)own;
+  if (own * g.groups >= (1ull << 32) || file_lds(g, cfg.calendar_windows) > kFileLdsMost) return false;
   groups_ = g;
   return true;
 }
@@ -1092,12 +1151,12 @@ gpq_status LaqQueue::init_calendar_groups() {
   GPQ_TRY(arena.alloc(&g.out, slots * cal::kUnitPass));
   GPQ_TRY(arena.alloc(&g.parts, slots * cal::kMaxGroups));
   GPQ_TRY(arena.alloc(&g.npass, g.units));
-  GPQ_TRY(arena.alloc(&g.over, (size_t)g.groups * g.over_cap));
-  GPQ_TRY(arena.alloc(&g.over_n, (size_t)g.groups * 16u));
+  GPQ_TRY(arena.alloc(&g.over, 2 * (size_t)g.groups * g.own_cap));
+  GPQ_TRY(arena.alloc(&g.over_n, (size_t)g.groups * cal::kOverWords));
   GPQ_HIP(hipMemsetAsync(g.wlog_n, 0, sizeof(uint32_t) * g.units * B, stream));
   GPQ_HIP(hipMemsetAsync(g.npass, 0, sizeof(uint32_t) * g.units, stream));
   GPQ_HIP(hipMemsetAsync(g.parts, 0, sizeof(uint32_t) * slots * cal::kMaxGroups, stream));
-  GPQ_HIP(hipMemsetAsync(g.over_n, 0, sizeof(uint32_t) * g.groups * 16u, stream));
+  GPQ_HIP(hipMemsetAsync(g.over_n, 0, sizeof(uint32_t) * g.groups * cal::kOverWords, stream));
   // the same bound for every queue: the attribute is the kernel's, and the last one to set it decides for all
   GPQ_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(cal_file_kernel),
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)kFileLdsMost));
@@ -1115,11 +1174,12 @@ gpq_status LaqQueue::calendar_file() {
 
 gpq_status LaqQueue::calendar_start() {
   GPQ_CHECK_ARG(v_.wlog, "LAQ: calendar_start needs calendar mode");
-  hipLaunchKernelGGL(cal_start_kernel, dim3(1), dim3(1), 0, stream, v_, cfg.lookahead, cfg.horizon);
   if (groups_.units) {       // the groups' lists hold every initial event
+    hipLaunchKernelGGL(cal_start_groups_kernel, dim3(1), dim3(1024), 0, stream, v_, groups_, cfg.lookahead, cfg.horizon);
     GPQ_HIP(hipGetLastError());
     return calendar_file();
   }
+  hipLaunchKernelGGL(cal_start_kernel, dim3(1), dim3(1), 0, stream, v_, cfg.lookahead, cfg.horizon);
   hipLaunchKernelGGL(cal_fill_kernel, dim3(cal::kGroupBlocks), dim3(cal::kBlock), 0, stream, v_, cfg.horizon,
                      1.0f / cfg.lookahead);
   hipLaunchKernelGGL(cal_fill_done_kernel, dim3(1), dim3(1), 0, stream, v_);

@@ -92,9 +92,11 @@ typedef struct {
                                 196608 LPs on), holding
                                 capacity_per_lp (<= 64) records per LP of the block; a step reads only
                                 the logs of the window it commits.  Events beyond the calendar wait in
-                                two lists (one per group of blocks from 196608 LPs on: the same room),
-                                and events at or past the horizon in a parked list, of
-                                num_lps * far_per_lp records each.  Same committed trace. */
+                                two lists, and events at or past the horizon in a parked list, of
+                                num_lps * far_per_lp records each.  (From 196608 LPs on the two lists are
+                                one per group of LPs in the same room: far_per_lp records per LP of the
+                                group, and a part of the other half, which the start of the calendar
+                                deals out by where the initial events lie.)  Same committed trace. */
   uint32_t sort_tile;         /* GAQ / HQ: records per block of the merge kernels:
                                 1024, 2048 or 4096 (0 = 2048); gpq_queue_autotune_sort picks one */
 } gpq_queue_config;
