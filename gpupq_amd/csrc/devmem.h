@@ -15,8 +15,9 @@ namespace gpq {
 enum class MemKind { kDevice, kPinned };
 
 // A block of at least `bytes` (> 0) on the current device (kDevice) or in pinned host memory;
-// nullptr when there is none.  Its contents are undefined.  *size receives the block's own size.
-void* mem_get(MemKind kind, size_t bytes, size_t* size);
+// nullptr when there is none.  Its contents are undefined.  *size receives the block's own size: up
+// to twice `bytes` when it was kept, or with `exact` no more than `bytes` rounded up to 256.
+void* mem_get(MemKind kind, size_t bytes, size_t* size, bool exact = false);
 // Gives a block back.  No work that uses it may be pending: the callers synchronize first.
 void mem_put(MemKind kind, void* p, size_t size);
 // Frees every kept block.

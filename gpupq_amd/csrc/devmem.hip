@@ -72,19 +72,19 @@ void* fresh(MemKind kind, size_t size) {
 
 }  // namespace
 
-void* mem_get(MemKind kind, size_t bytes, size_t* size) {
+void* mem_get(MemKind kind, size_t bytes, size_t* size, bool exact) {
   int dev = -1;
   if (kind == MemKind::kDevice && hipGetDevice(&dev) != hipSuccess) {
     (void)hipGetLastError();
     return nullptr;
   }
-  const size_t want = rounded(bytes);
+  const size_t want = exact ? (bytes + 255) / 256 * 256 : rounded(bytes), most = exact ? want : 2 * want + 1;
   Kept& k = kept();
   {
     std::lock_guard<std::mutex> lock(k.mu);
     auto best = k.blocks.end();              // the smallest that fits without wasting half of it
     for (auto it = k.blocks.begin(); it != k.blocks.end(); ++it)
-      if (it->kind == kind && it->dev == dev && it->size >= want && it->size / 2 <= want &&
+      if (it->kind == kind && it->dev == dev && it->size >= want && it->size <= most &&
           (best == k.blocks.end() || it->size < best->size))
         best = it;
     if (best != k.blocks.end()) {

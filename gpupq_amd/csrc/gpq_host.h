@@ -47,21 +47,23 @@ class DeviceArena {
  public:
   ~DeviceArena() { release(); }
   void on(hipStream_t s) { streams_.push_back(s); }
+  // Blocks of no more than is asked for, for an owner whose memory has a stated bound.
+  void exact() { exact_ = true; }
   template <class T>
   gpq_status alloc(T** p, size_t count) {
     const size_t bytes = count * sizeof(T) > 0 ? count * sizeof(T) : 16;
     size_t size = 0;
-    void* raw = mem_get(MemKind::kDevice, bytes, &size);
+    void* raw = mem_get(MemKind::kDevice, bytes, &size, exact_);
     if (!raw) {
       set_error("hipMalloc of " + std::to_string(bytes) + " bytes failed");
       return GPQ_ERR_NOMEM;
     }
     blocks_.push_back({raw, size});
-    bytes_ += bytes;
+    bytes_ += size;
     *p = static_cast<T*>(raw);
     return GPQ_OK;
   }
-  size_t bytes() const { return bytes_; }
+  size_t bytes() const { return bytes_; }     // of the blocks held
   void release() {
     for (hipStream_t s : streams_) (void)hipStreamSynchronize(s);
     streams_.clear();
@@ -74,6 +76,7 @@ class DeviceArena {
   std::vector<std::pair<void*, size_t>> blocks_;
   std::vector<hipStream_t> streams_;
   size_t bytes_ = 0;
+  bool exact_ = false;
 };
 
 // Pinned host memory of one owner, which ends every copy to or from it first.

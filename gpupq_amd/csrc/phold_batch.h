@@ -17,9 +17,11 @@ namespace gpq {
 class PholdPool {
  public:
   // capacity_lps: LPs the pool can hold at once (rounded up to whole 256-LP blocks).
-  // far_per_lp > 0: two-tier LAQ, each instance with its own near horizon.
+  // far_per_lp > 0: two-tier LAQ, each instance with its own near horizon.  exact_memory: device_bytes()
+  // has a bound to keep, so no block is larger than asked for.
   static gpq_status create(uint32_t capacity_lps, uint32_t capacity_per_lp, uint32_t stage_per_lp,
-                           uint32_t max_instances, PholdPool** out, uint32_t far_per_lp = 0);
+                           uint32_t max_instances, PholdPool** out, uint32_t far_per_lp = 0,
+                           bool exact_memory = false);
   ~PholdPool();
 
   // Bytes of HBM one LP of the pool holds (ring, staging, queue words, model state).

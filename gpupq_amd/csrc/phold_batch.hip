@@ -249,7 +249,8 @@ uint64_t PholdPool::bytes_per_lp(uint32_t capacity_per_lp, uint32_t stage_per_lp
 uint64_t PholdPool::device_bytes() const { return (q_ ? q_->arena.bytes() : 0) + arena_.bytes(); }
 
 gpq_status PholdPool::create(uint32_t capacity_lps, uint32_t capacity_per_lp, uint32_t stage_per_lp,
-                             uint32_t max_instances, PholdPool** out, uint32_t far_per_lp) {
+                             uint32_t max_instances, PholdPool** out, uint32_t far_per_lp,
+                             bool exact_memory) {
   GPQ_CHECK_ARG(capacity_lps >= 1 && max_instances >= 1, "pool: empty");
   const uint32_t cap = (uint32_t)ceil_div(capacity_lps, kBlk) * kBlk;
   gpq_queue_config qc{};
@@ -263,6 +264,10 @@ gpq_status PholdPool::create(uint32_t capacity_lps, uint32_t capacity_per_lp, ui
   qc.far_per_lp = far_per_lp;
   auto p = std::make_unique<PholdPool>();
   p->q_ = new LaqQueue(qc);
+  if (exact_memory) {
+    p->q_->arena.exact();
+    p->arena_.exact();
+  }
   GPQ_TRY(p->q_->init_common());
   GPQ_TRY(p->q_->init());
   p->capacity_ = cap;

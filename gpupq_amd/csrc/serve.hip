@@ -103,6 +103,7 @@ gpq_status start_phold(const gpq_serve_config& c, const gpq_request& r, uint32_t
   const gpq_queue_config qc = phold_queue_config(r.size, c.phold_end_time);
   inst->q.reset(make_queue(qc));
   GPQ_CHECK_ARG(inst->q, "serve: queue kind not provided");
+  inst->q->arena.exact();            // within the budget, which was checked against the exact sizes
   GPQ_TRY(inst->q->init_common());
   GPQ_TRY(inst->q->init());
   PholdModel* m = nullptr;
@@ -279,7 +280,7 @@ gpq_status serve_run(const gpq_serve_config& cin, gpq_drive_mode mode, gpq_serve
       }
       PholdPool* raw = nullptr;
       GPQ_TRY(PholdPool::create((uint32_t)cap, kPholdCapacity, kPholdStage, std::min<uint32_t>(phold_n, 1024), &raw,
-                                kPholdFar));
+                                kPholdFar, true));
       pool.reset(raw);
       GPQ_TRY(pool->prepare(c.phold_batch));
       GPQ_HIP(hipStreamSynchronize(pool->queue()->stream));
