@@ -577,7 +577,10 @@ gpq_status HqQueue::init() {
     // stream twice per step; a hipGraph capture of the step records the branches
     hs_.assign(heaps_, nullptr);
     ev_.assign(2 * heaps_ + 2, nullptr);
-    for (auto& x : hs_) GPQ_HIP(hipStreamCreateWithFlags(&x, hipStreamNonBlocking));
+    for (auto& x : hs_) {
+      GPQ_HIP(hipStreamCreateWithFlags(&x, hipStreamNonBlocking));
+      arena.on(x);
+    }
     for (auto& e : ev_) GPQ_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
   }
   GPQ_TRY(arena.alloc(&sum_, 1));
@@ -594,7 +597,7 @@ gpq_status HqQueue::init() {
 }
 
 HqQueue::~HqQueue() {
-  if (stream) (void)hipStreamSynchronize(stream);   // the heap streams join it every step
+  arena.release();   // waits for the streams: a step that failed half way has not joined the heaps' to the queue's
   for (auto e : ev_) if (e) (void)hipEventDestroy(e);
   for (auto x : hs_) if (x) (void)hipStreamDestroy(x);
 }
