@@ -23,6 +23,7 @@ struct GaqState {
   uint32_t prefix;      // records scanned
   uint32_t deq_n;       // records in the dequeue buffer
   uint32_t rest_n;      // unselected records of the scanned prefix
+  uint32_t reserved[2];
 };
 
 struct GaqView {

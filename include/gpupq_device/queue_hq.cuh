@@ -15,20 +15,23 @@ namespace gpq {
 constexpr int kHqMaxLevels = 20;
 constexpr int kHqMaxChunks = 8;
 
+// The layout stays as model kernels are compiled against it, which find heap h's state by its size.
 struct HqState {
   uint32_t last;           // highest node holding records
   uint32_t m;              // inserts of this step (totalled over the stripes by queue_post)
   uint32_t mcount;         // records in the merged buffer
   uint32_t prefix, deq_n, rest_n;
   uint32_t bound_valid;
+  uint32_t reserved0;
   uint32_t select;         // 1: queue_post selects the next step's events
-  uint32_t pad[4];
+  uint32_t pad[3];
   Event bound;             // the root's largest record while nodes exist below the root
   const Event* mptr;       // = merged buffer (pointer slot for the selection)
   // insert-update chunks: target node, size, first record among the carried ones
   uint32_t chunk_target[kHqMaxChunks];
   uint32_t chunk_n[kHqMaxChunks];
   uint32_t chunk_off[kHqMaxChunks];
+  uint32_t reserved1[24];
 };
 
 // Several heaps (HQ_NUM_QUEUES): heap h owns the LPs [h * lps_per_heap, (h + 1) * lps_per_heap),
