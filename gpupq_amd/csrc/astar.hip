@@ -10,8 +10,7 @@
 // (src/a_star.cu:325-374,470-474), so it does not guarantee the optimum.
 //
 // Batched (gpq_astar_batch_*): one workgroup per query, pulled from a device counter as
-// get_new_agent does (src/a_star.cu:149-164), K = blockDim per-thread binary heaps of
-// 64-bit keys (f << 32 | cell) in HBM, successors routed through LDS staging.
+// get_new_agent does (src/a_star.cu:149-164), its open list a row of buckets by f; in astar_batch.hip.
 #include <algorithm>
 #include <chrono>
 #include <cmath>

@@ -20,10 +20,10 @@
 // What bounds it: the latency of an iteration (three barriers and four dependent accesses: bucket
 // entry, g and obstacle bits, relaxations, append), times the longest query's iterations, which its
 // path's steps bound from below.  Expanding an entry's best successor in the same iteration (2
-// to 16 of a chain) made iterations longer by more than it saved (15 to 29 ms).  The
+// to 16 of a chain) made iterations longer by more than it saved (15 to 29 ms where without it was 12).  The
 // list this replaced, a binary heap per thread, moved some 3 KB per expansion in sifts over
 // scattered lines and took 19 us per iteration against 7 us here: 512 queries of side 256 to
-// 2048 in 512-thread workgroups, 42.6 -> 12.0 ms.
+// 2048, 8-connected, in 512-thread workgroups 39.0 -> 14.6 ms, in 256-thread ones 30.4 -> 12.8.
 //
 // Entry = f << 22 | cell.  Limits that follow: side <= 2048 (cell < 2^22), f < 2^26.
 //
@@ -50,9 +50,10 @@ constexpr int kMaxWaves = 16;
 // Buckets of a query's open list: one per lane of the wave that plans an iteration.
 constexpr uint32_t kBuckets = 64;
 // f values per bucket, as a power of two: f - h(source) is even on both kinds of grid, so a bucket
-// is one f value.  Wider buckets expand more cells out of order: 512 queries of side 256 to 2048
-// took 12.0 ms at width 2, 13.2 at 4, 15.6 at 8 and 23 at 16.  Taking entries of the lowest 32,
-// 16 or 8 buckets only (fewer expansions, idler iterations) took 12.1, 16.6 and 18.7 ms.
+// is one f value.  Wider buckets expand more cells out of order: 512 queries of side 256 to 2048,
+// 8-connected, 512 threads each, took 14.7 ms at width 2, 16.0 at 4 and 17.4 at 8.  Taking entries of
+// the lowest 32, 16 or 8 buckets only (fewer expansions, idler iterations) took 13.4, 12.8 and 15.1 ms;
+// with 64 threads and 256 queries 20.5, 21.5 and 24.0 against 20.9 without a limit.
 constexpr uint32_t kShift = 1;
 constexpr uint32_t kNoBucket = 0xFFFFFFFFu;
 
@@ -420,7 +421,9 @@ __global__ __launch_bounds__(1024) void astar_batch_step_kernel(BatchDev d, uint
 
 __global__ void zero_u32_kernel(uint32_t* p) { *p = 0; }
 
-constexpr size_t kStageLimit = 64 * 1024;   // threads * (8 * stage_capacity + 4) bytes accepted
+// threads * (8 * stage_capacity + 4) accepted: the bound that stage_capacity has always had, though the open
+// list needs no staging now and takes any number of inserts per iteration.
+constexpr size_t kStageLimit = 64 * 1024;
 
 // Entries a bucket holds: half of the list's capacity over the row, within [256, 8192] (64 KiB); a fuller bucket spills into the far store.
 uint32_t bucket_cap_for(const gpq_batch_tuning& t) {
@@ -489,7 +492,7 @@ gpq_status AstarBatch::create(const gpq_query_spec* sp, uint32_t count, const gp
   GPQ_CHECK_ARG(tu.heap_capacity >= 16 && tu.heap_capacity <= (1u << 20), "batch: heap_capacity out of range");
   GPQ_CHECK_ARG(tu.stage_capacity >= 1 && tu.stage_capacity <= 64, "batch: stage_capacity must be in [1, 64]");
   GPQ_CHECK_ARG((size_t)tu.threads_per_query * (tu.stage_capacity * 8 + 4) <= kStageLimit,
-                "batch: staging (threads * (8 * stage + 4) bytes) must fit in 64 KiB");
+                "batch: threads_per_query * (8 * stage_capacity + 4) must be <= 65536");
   uint64_t max_cells = 0, words = 0;
   std::vector<BatchQuery> hq(count);
   std::vector<uint64_t> off(count);
@@ -656,19 +659,19 @@ gpq_status AstarBatch::run(gpq_drive_mode mode, double* seconds) {
 }
 
 // Times every workgroup size on the first `sample` queries (two persistent runs each, the second
-// timed) and returns the fastest; heap_capacity and max_resident are kept from `base`.  Candidates whose open lists overflow are skipped.
+// timed) and returns the fastest; heap_capacity and max_resident are kept from `base`.  Candidates
+// whose open lists overflow are skipped.
 gpq_status batch_autotune(const gpq_query_spec* sp, uint32_t count, uint32_t sample, const gpq_batch_tuning& base,
                           gpq_batch_tuning* out, double* best_seconds) {
   GPQ_CHECK_ARG(sp && count >= 1, "autotune: no queries");
   const uint32_t n = sample ? std::min(sample, count) : count;
-  static const uint32_t kThreads[] = {64, 128, 256, 512, 1024};
+  static const uint32_t kThreads[] = {64, 128, 256, 512};   // stage_capacity 8 excludes 1024
   double best = 1e300;
   gpq_batch_tuning pick{};
   for (uint32_t k : kThreads) {
     gpq_batch_tuning t = base;
     t.threads_per_query = k;
     t.stage_capacity = 8;
-    if ((size_t)k * (t.stage_capacity * 8 + 4) > kStageLimit) continue;
     AstarBatch* b = nullptr;
     if (AstarBatch::create(sp, n, t, &b) != GPQ_OK) continue;
     double sec = 0.0;

@@ -323,8 +323,11 @@ __device__ __forceinline__ uint64_t hash_events(const CommitLds<U, PER>& s, cons
 // the runs; a successor for another block goes to that block's log by its own atomic.  The log is
 // emptied at the end.  A log of more than kPer events per thread is taken in passes over ranges of LPs.
 //
-// What bounds it: the atomics on the logs' counters, which are performed at the memory side at 26.6
-// G/s whatever lines they meet on: 1.7 M per step at 2^20 LPs x 32 events, 64 us of its 126.
+// What bounds it: a block's chain of loads, LDS phases and the atomics' round trips, and the launch: 10.1
+// us a step at 1024 LPs x 16 events (four blocks), 21.4 at 65,536 x 32 (one block per CU), 30.2 at 131,072
+// x 32, where 7 us of it are the 190,000 atomics on other blocks' log counters (performed at the memory
+// side, at 26.6 G/s whatever lines they meet on).  At 2^20 LPs they were 64 us of 126, which is why large
+// calendars are kept otherwise.
 // With a thread per LP and its events in eight register slots (sorted by a network), a wave ran
 // all eight slots' draws for LPs that hold three events on average, and an LP with more was
 // committed by a wave of its own afterwards: 152 us per step (and 15.7 us at 1024 LPs, now 10.1).

@@ -31,9 +31,9 @@ struct OutMap {
 // Merge-path split: the number of A records among the first d outputs of the stable merge
 // (ties: A first) is the smallest i in [max(0, d - nb), min(d, na)] with B[d-1-i] < A[i].
 // Found for the block's two diagonals d0 and d1 at once, each by half of the block: every
-// round the 128 threads of a half probe 128 evenly spaced points of the remaining range and
+// round the kT / 2 threads of a half probe as many evenly spaced points of the remaining range and
 // keep the gap where the predicate turns true, so a range of n shrinks to nothing in
-// ceil(log_128 n) rounds of one load each, not log_2 n dependent loads.
+// ceil(log n / log(kT / 2)) rounds of one load each, not log_2 n dependent loads.
 template <int kT>
 __device__ __forceinline__ void block_merge_splits(const ASrc& A, uint32_t na, const Event* B, uint32_t nb, uint32_t d0, uint32_t d1,
                                    uint32_t* s_split) {

@@ -71,9 +71,10 @@ __device__ __forceinline__ void phold_drain(const Q& q, const PholdDev& m, uint3
 
 // Drain mode on the local array queue: the same commits in the same order as repeated
 // peek / set_done, with the LP's ring cursor, count and hash held in registers, the next record loaded
-// and the last successor's slot taken while the current record is processed; written back once.  An event
-// is a chain of memory accesses whatever is overlapped, and that is what bounds it (200,003 LPs, 16 events
-// each: 14.1 ms with the slot waited for before the next event, 13.7 so; serving 116.9 and 116.0).
+// and the last successor's slot taken while the current record is processed; written back once.  What
+// bounds it: the slots' atomics, one per event, which are performed at the memory side at 26.6 G/s: 291,000 a
+// step at 200,003 LPs x 16 events, 10.9 us of a launch of 18.4 (6 to 8 of which an empty one takes).  So
+// the overlap gains little: 14.1 ms with the slot waited for before the next event, 13.7 so; serving 116.9 and 116.0.
 __device__ __forceinline__ void phold_drain(const LaqView& q, const PholdDev& m, uint32_t lp) {
   const uint32_t wend = q.ws->wend, head = q.head[lp];
   const uint32_t mask = (1u << q.cap_log2) - 1u;

@@ -12,7 +12,8 @@
 // through a table of slots and a merge writes a free slot that then becomes the node's; the refill is
 // part of the merge that fills the root; and the insert chunks follow one another down the heap, a level
 // behind the one before.  100,003 LPs, 16 events each: 320 us a step with 39 merges and 30
-// planners, 219 us with the 18 merges here.
+// planners, 219 us with the 18 merges here; 200 with the selection in three launches and the tickets on
+// several words as well.
 //
 // queue_post:
 //  1. sort the step's inserts; M = merge(root, inserts)            (src/heap_queue.cu:1541-1553, 1448-1470)
@@ -243,7 +244,9 @@ struct ChildrenMerge : MergeOp {
   __device__ const uint32_t* list() const { return p.dirty + (level & 1u) * p.slots; }
   __device__ uint32_t tasks() const { return level ? p.dirty_n[level & 1u] : 1u; }
   // One exit, and loads that do not depend on one another: with a return from between the two
-  // comparisons the compiler lost the children's addresses on the way from the second one.
+  // comparisons the compiler (hipcc of ROCm 7.2.0, clang 22, -O3) lost the children's addresses on the way
+  // from the second one: in its assembly that path cleared their registers and went on with the counts.
+  // Keep it so, or read the assembly of what replaces it.
   __device__ MergeTask plan(uint32_t y, uint32_t n) const {
     const uint32_t top = p.nodes - 1u;
     const uint32_t v0 = level ? list()[min(y, p.slots - 1u)] : 0u, v = min(v0, top);   // any node for y >= n
@@ -387,7 +390,7 @@ __device__ __forceinline__ void commit_lane(const Op& op, uint32_t y, uint32_t n
 // The tiles of a launch's tasks, dealt out to its blocks.  Every block plans all tasks, a lane each
 // (a wave of them at a time), so that only tasks with records take tiles.  With a grid slot per tile
 // of every node of a level, 2352 blocks on the fifth level at 100,003 LPs, most found nothing to do: a
-// ParentMerge took 18 us on average and takes 10, a step 288 us and 219.
+// ParentMerge took 18 us on average and takes 10, a step went from 288 us to 219.
 template <typename Op, int kT>
 __global__ __launch_bounds__(kT) void hq_merge_kernel(Op op) {
   constexpr uint32_t kTile = kT * kPerThread;

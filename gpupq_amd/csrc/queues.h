@@ -37,7 +37,10 @@ class LaqQueue final : public QueueBase {
   // Calendars of this many LPs have logs with one writer (laq_calendar_groups.cuh): their step has
   // a launch more, which costs 8 us, but no atomic per successor.  Measured per window, one writer
   // against atomics: 65,536 LPs x 32 events 28.0 against 21.4 us, 131,072 x 32 31.8 against 30.2,
-  // 262,144 x 8 29.0 against 29.4, 262,144 x 32 40.1 against 46.8.
+  // 262,144 x 32 40.1 against 46.8.  Whole runs to time 5 with few events per LP: 200,003 LPs x 4 events
+  // (lookahead 0.05) 2.34 against 2.47 ms, x 2 2.28 against 2.27, x 1 2.24 against 2.11; 262,144 x 4 2.64
+  // against 3.02, x 2 2.56 against 2.72, x 1 2.50 and 2.50; 524,288 x 1 3.51 against 4.11.  So the line holds
+  // from two events per LP on, and with one from 262,144 LPs on.
   static constexpr uint32_t kGroupedMinLps = 196608;
   // Post blocks whose flag is 0 are skipped (their LPs hold nothing); nullptr = all live.
   void set_block_live(const uint8_t* flags) { v_.block_live = flags; }

@@ -59,8 +59,8 @@ gpq_status gather_inserts(uint32_t* seg_m, uint32_t seg_cap, uint32_t spill_cap,
 // Runs `ntasks` merge tasks (device array) in one launch; max_total bounds every task's
 // n_a1 + n_a2 + n_b.  `acct` (optional) receives the records merged (the tasks' totals).
 // `splits` (optional, ntasks * stride u32 with stride >= merge_split_words(max_total, tile)):
-// the merge-path splits of every tile boundary are computed by a partition launch first (one
-// wave per boundary), instead of by each merge block before it can load its input.
+// the merge-path splits of every tile boundary are computed by a partition launch first (eight
+// lanes per boundary), instead of by each merge block before it can load its input.
 // Merges whose max_total is below partition_min search their splits in the merge blocks even
 // with `splits` given.
 constexpr uint64_t kMergePartitionMin = 1ull << 20;
@@ -87,8 +87,5 @@ struct SelectBufs {
 gpq_status select_safe(const Event* const* d_s, const uint32_t* d_n, uint32_t cap, const uint32_t* d_wend,
                        const Event* d_bound, const uint32_t* d_bound_valid, const SelectBufs& b, Event* deq,
                        Event* rest, hipStream_t stream, unsigned long long* acct = nullptr);
-
-// Copies records: dst[i] = src[i] for i < *d_n (bounded by cap).
-gpq_status copy_records(const Event* src, Event* dst, const uint32_t* d_n, uint32_t cap, hipStream_t stream);
 
 }  // namespace gpq

@@ -566,12 +566,6 @@ __global__ __launch_bounds__(64) void gather_inserts_kernel(uint32_t* seg_m, uin
   }
 }
 
-__global__ void copy_records_kernel(const Event* src, Event* dst, const uint32_t* d_n, uint32_t cap) {
-  const uint32_t n = *d_n < cap ? *d_n : cap;
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
-    store_event(dst + i, load_event(src + i));
-}
-
 // --- selection --------------------------------------------------------------------
 
 __device__ __forceinline__ bool in_prefix(const Event& e, uint32_t wend, bool bounded, const Event& bound) {
@@ -830,13 +824,6 @@ gpq_status gather_inserts(uint32_t* seg_m, uint32_t seg_cap, uint32_t spill_cap,
   static_assert(kInsertStripes + 1 <= kWave, "one wave gathers the stripes");
   hipLaunchKernelGGL(gather_inserts_kernel, dim3(1), dim3(kWave), 0, stream, seg_m, seg_cap, spill_cap, max_total,
                      seg_pre, d_m, ws);
-  GPQ_HIP(hipGetLastError());
-  return GPQ_OK;
-}
-
-gpq_status copy_records(const Event* src, Event* dst, const uint32_t* d_n, uint32_t cap, hipStream_t stream) {
-  const uint32_t g = grid_of(cap, kThreads);
-  hipLaunchKernelGGL(copy_records_kernel, dim3(g < 8192 ? g : 8192), dim3(kThreads), 0, stream, src, dst, d_n, cap);
   GPQ_HIP(hipGetLastError());
   return GPQ_OK;
 }
