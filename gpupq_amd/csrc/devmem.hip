@@ -3,9 +3,12 @@
 
 #include <hip/hip_runtime.h>
 
-#include <list>
+#include <map>
 #include <mutex>
+#include <set>
+#include <tuple>
 #include <unordered_map>
+#include <vector>
 
 namespace gpq {
 namespace {
@@ -17,13 +20,34 @@ struct Block {
   MemKind kind;
 };
 
-// Kept blocks, oldest first.  A process keeps a few hundred at most, so a linear search is cheap
-// next to any launch.  Never destroyed: the HIP runtime may be gone when static objects end.
+// Kept blocks by kind: by age, and by device and size, kMostBlocks of a kind.  A process that had 1500 small
+// queues at once kept 13,000 blocks, and making the next queue took 1.4 ms, of which searching one list of
+// them took 1.0 and the runtime's own search among its allocations 0.2 (0.12 with none kept).  Never destroyed: the HIP runtime may be gone when static objects end.
+constexpr size_t kMostBlocks = 1024;
 struct Kept {
   std::mutex mu;
-  std::list<Block> blocks;
+  std::map<uint64_t, Block> by_age[2];                            // the oldest first
+  std::set<std::tuple<int, size_t, uint64_t>> by_size[2];         // device, size, age
+  uint64_t next_age = 0;
   std::unordered_map<void*, int> dev_of;     // device of every block handed out or kept
   size_t bytes[2] = {0, 0};
+
+  void add(const Block& b) {
+    const int i = (int)b.kind;
+    by_age[i].emplace(next_age, b);
+    by_size[i].emplace(b.dev, b.size, next_age);
+    ++next_age;
+    bytes[i] += b.size;
+  }
+  Block take(MemKind kind, uint64_t age) {
+    const int i = (int)kind;
+    const auto it = by_age[i].find(age);
+    const Block b = it->second;
+    by_age[i].erase(it);
+    by_size[i].erase(std::make_tuple(b.dev, b.size, age));
+    bytes[i] -= b.size;
+    return b;
+  }
 };
 
 Kept& kept() {
@@ -82,17 +106,12 @@ void* mem_get(MemKind kind, size_t bytes, size_t* size, bool exact) {
   Kept& k = kept();
   {
     std::lock_guard<std::mutex> lock(k.mu);
-    auto best = k.blocks.end();              // the smallest that fits without wasting half of it
-    for (auto it = k.blocks.begin(); it != k.blocks.end(); ++it)
-      if (it->kind == kind && it->dev == dev && it->size >= want && it->size <= most &&
-          (best == k.blocks.end() || it->size < best->size))
-        best = it;
-    if (best != k.blocks.end()) {
-      void* p = best->p;
-      *size = best->size;
-      k.bytes[(int)kind] -= best->size;
-      k.blocks.erase(best);
-      return p;
+    const auto& sizes = k.by_size[(int)kind];          // the smallest that fits without wasting half of it
+    const auto best = sizes.lower_bound(std::make_tuple(dev, want, (uint64_t)0));
+    if (best != sizes.end() && std::get<0>(*best) == dev && std::get<1>(*best) <= most) {
+      const Block b = k.take(kind, std::get<2>(*best));
+      *size = b.size;
+      return b.p;
     }
   }
   void* p = fresh(kind, want);
@@ -116,21 +135,16 @@ void mem_put(MemKind kind, void* p, size_t size) {
   if (!p) return;
   Kept& k = kept();
   const size_t most = bound(kind);
-  std::list<Block> out;
+  std::vector<Block> out;
   {
     std::lock_guard<std::mutex> lock(k.mu);
     const Block b{p, size, k.dev_of[p], kind};
     if (size > most) {
       out.push_back(b);
     } else {
-      k.blocks.push_back(b);
-      k.bytes[(int)kind] += size;
-      for (auto it = k.blocks.begin(); k.bytes[(int)kind] > most && it != k.blocks.end();) {
-        if (it->kind != kind) { ++it; continue; }
-        k.bytes[(int)kind] -= it->size;
-        out.push_back(*it);
-        it = k.blocks.erase(it);
-      }
+      k.add(b);
+      while (k.bytes[(int)kind] > most || k.by_age[(int)kind].size() > kMostBlocks)
+        out.push_back(k.take(kind, k.by_age[(int)kind].begin()->first));
     }
     for (const Block& x : out) k.dev_of.erase(x.p);
   }
@@ -139,11 +153,15 @@ void mem_put(MemKind kind, void* p, size_t size) {
 
 void mem_release_kept() {
   Kept& k = kept();
-  std::list<Block> out;
+  std::vector<Block> out;
   {
     std::lock_guard<std::mutex> lock(k.mu);
-    out.swap(k.blocks);
-    k.bytes[0] = k.bytes[1] = 0;
+    for (int i = 0; i < 2; ++i) {
+      for (const auto& x : k.by_age[i]) out.push_back(x.second);
+      k.by_age[i].clear();
+      k.by_size[i].clear();
+      k.bytes[i] = 0;
+    }
     for (const Block& x : out) k.dev_of.erase(x.p);
   }
   for (const Block& x : out) free_block(x);
