@@ -940,7 +940,7 @@ __global__ void cal_units_count_kernel(LaqView q, cal::Groups g, unsigned long l
   for (uint32_t u = t; u < g.units; u += stride)
     for (uint32_t p = 0; p < g.npass[u]; ++p)
       for (uint32_t i = 0; i < cal::kMaxGroups; ++i) n += g.parts[((size_t)u * g.passes + p) * cal::kMaxGroups + i] >> 16;
-  if (t == 0) n += min(*q.parked_n, q.parked_cap) + min(*g.spill_n, g.groups * g.own_cap);
+  if (t == 0) n += (unsigned long long)min(*q.parked_n, q.parked_cap) + min(*g.spill_n, g.groups * g.own_cap);
   for (int off = 32; off > 0; off >>= 1) n += __shfl_xor(n, off, kWave);
   if (lane_id() == 0) s[threadIdx.x / kWave] = n;
   __syncthreads();
